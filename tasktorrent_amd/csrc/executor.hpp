@@ -142,6 +142,8 @@ inline int vset_index(int needed) {
 // POTRF and TRSM items are called out of line from the executors: a kernel holding them
 // inline is register-allocated for their largest live set and spills in the GEMM loop,
 // which runs far more often. The call saves the callee's registers once per item.
+// Their arguments arrive in vector registers; they are moved to scalar ones, so that sizes, addresses and the
+// branches on them are scalar.
 // One instance per executor instantiation (VM): a callee shared by kernels compiled for
 // different occupancies would be register-allocated for the lowest of them.
 // POTRF and TRSM carry the critical path: their waves run at raised issue priority, so
@@ -150,7 +152,8 @@ template <typename TS, int VM>
 __device__ __attribute__((noinline)) void potrf_call(TS* A, long lda, int n, double* dinv, int* info, int col_off,
                                                      char* lds) {
     __builtin_amdgcn_s_setprio(3);
-    item_potrf<TS>(A, lda, n, dinv, info, col_off, lds);
+    item_potrf<TS>(wave_uniform(A), wave_uniform((int)lda), wave_uniform(n), wave_uniform(dinv), wave_uniform(info),
+                   wave_uniform(col_off), lds_uniform(lds));
     __builtin_amdgcn_s_setprio(0);
 }
 template <typename TS, int VM>
@@ -158,7 +161,9 @@ __device__ __attribute__((noinline)) void potrf_rows_call(TS* A, long lda, int n
                                                           int rb, int32_t* prog, int32_t* err, int64_t spin_limit,
                                                           char* lds) {
     __builtin_amdgcn_s_setprio(3);
-    item_potrf_rows<TS>(A, lda, n, dinv, info, col_off, rb, prog, err, spin_limit, lds);
+    item_potrf_rows<TS>(wave_uniform(A), wave_uniform((int)lda), wave_uniform(n), wave_uniform(dinv),
+                        wave_uniform(info), wave_uniform(col_off), wave_uniform(rb), wave_uniform(prog),
+                        wave_uniform(err), spin_limit, lds_uniform(lds));
     __builtin_amdgcn_s_setprio(0);
 }
 // Accumulate-mode GEMM items are called out of line too, so the default GEMM loop keeps its registers.
@@ -172,7 +177,9 @@ template <typename TS, typename TC, int VM>
 __device__ __attribute__((noinline)) void trsm_call(const TS* L, long ldl, const double* dinv, TS* X, long ldx, int m,
                                                     int n, int r0, char* lds, void* planes) {
     __builtin_amdgcn_s_setprio(3);
-    item_trsm<TS, TC>(L, ldl, dinv, X, ldx, m, n, r0, lds, planes);
+    item_trsm<TS, TC>(wave_uniform(L), wave_uniform((int)ldl), wave_uniform(dinv), wave_uniform(X),
+                      wave_uniform((int)ldx), wave_uniform(m), wave_uniform(n), wave_uniform(r0), lds_uniform(lds),
+                      wave_uniform(planes));
     __builtin_amdgcn_s_setprio(0);
 }
 

@@ -38,6 +38,16 @@ template <typename T> __device__ __forceinline__ T* wave_uniform(T* p) {
     return (T*)(((unsigned long long)hi << 32) | lo);
 }
 
+// The workgroup's dynamic LDS as a pointer in a scalar register. In a function called out of line its base is read
+// from a table in memory, and the compiler reads it again at every use it cannot hoist (a memory round trip in front
+// of LDS accesses on the critical path); the offset is opaque here, so it is read once.
+__device__ __forceinline__ char* lds_uniform(char* p) {
+    typedef __attribute__((address_space(3))) char lds_char;
+    unsigned off = (unsigned)(unsigned long long)(lds_char*)p;
+    asm volatile("" : "+v"(off));
+    return (char*)(lds_char*)(unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane(off);
+}
+
 // ---------------------------------------------------------------------------
 // MFMA 16x16 primitives. Operand layouts (lane l of the wave):
 //   f64/f32 16x16x4 : A[m = l%16][k = l/16], B[k = l/16][n = l%16]
@@ -754,11 +764,11 @@ __device__ __forceinline__ void decode_gemm_item(int it, int tr, bool syrk, int&
 // ---------------------------------------------------------------------------
 // 64x64 diagonal block in LDS (column-major, ld DP), blocked by 16: factor
 // (lower Cholesky) and inverse. FP64 throughout. Padding rows/cols beyond `w`
-// hold identity. Diagonal 16x16 blocks are handled element-wise (thread t owns
-// element (t%16, t/16), one barrier per column); everything else is 16x16x16
-// products on FP64 MFMA, one block per wave.
+// hold identity. 16-column panels are factored by one wave in registers;
+// everything else is 16x16x16 products on FP64 MFMA, one block per wave.
 // ---------------------------------------------------------------------------
 constexpr int DP = DB + 1;
+constexpr int POTRF_LDS = (2 * DB * DP + 2) * 8;  // D, X and a flag
 
 // acc += P Q (q_trans = false) or P Q^T (q_trans = true); P, Q 16x16 blocks in LDS, ld DP.
 __device__ __forceinline__ d4_t mma16(d4_t acc, const double* P, const double* Q, bool q_trans) {
@@ -801,102 +811,198 @@ __device__ __forceinline__ double rcp_nr(double x) {
     return __builtin_fma(r, e, r);
 }
 
-// X_KK = L_KK^{-1} for the 16x16 lower-triangular diagonal block at Lk (X block at Xk,
-// upper part left untouched). Row-by-row substitution with the partial sums in registers:
-// one barrier per row. All threads participate.
-__device__ __forceinline__ void tri_inv16(const double* Lk, double* Xk) {
-    const int ti = threadIdx.x & 15, tc = threadIdx.x >> 4;
-    const double rd = rcp_nr(Lk[ti + ti * DP]);  // 1 / L(ti, ti), ahead of the row-by-row chain
-    double acc = 0.0;
-    for (int q = 0; q < 16; q++) {
-        if (ti == q && tc <= q) Xk[q + tc * DP] = ((q == tc ? 1.0 : 0.0) - acc) * rd;
-        __syncthreads();
-        if (ti > q && tc <= q) acc += Lk[ti + q * DP] * Xk[q + tc * DP];
+// The value of lane SRC of each row of 16 lanes, in all 16 of them (one DPP move). Every lane has to be active.
+template <int SRC>
+__device__ __forceinline__ double row_value(double x) {
+    const long v = __builtin_bit_cast(long, x);
+    const long r = __builtin_amdgcn_update_dpp(v, v, 0x150 + SRC, 0xf, 0xf, true);  // row_newbcast
+    return __builtin_bit_cast(double, r);
+}
+// f(K) for K = 0 .. N - 1 as a compile-time constant (DPP controls are immediates).
+template <int K, int N, typename F>
+__device__ __forceinline__ void for_const(const F& f) {
+    if constexpr (K < N) {
+        f(std::integral_constant<int, K>{});
+        for_const<K + 1, N>(f);
     }
-    __syncthreads();
 }
 
-// Off-diagonal blocks of X = L^{-1} from L (D) and the diagonal inverses already in X:
-// X_IJ = -X_II sum_{Q=J}^{I-1} L_IQ X_QJ, in order of I - J (one wave per block).
+// Keeps the computation of x in front of this point.
+__device__ __forceinline__ void hold(double& x) { asm volatile("" : "+v"(x)); }
+
+// One wave factors a 16-column panel, a row per lane in a[]; p[] is the 16x16 diagonal block, row i in every lane with
+// lane % 16 == i, so that pivot rows reach all lanes by moves within 16 lanes: a column costs no LDS round trip and no
+// barrier. Lanes 0..15 hold the block's own rows in a[], every other lane a row b that becomes b L^{-T} (rows below
+// the block; rows of the identity, which become L^{-T} itself). Unscaled elimination by the pivots' reciprocals, then
+// the columns are scaled. Returns, in lane k < 16, whether pivot k is not positive.
+__device__ __forceinline__ bool panel16(double (&p)[16], double (&a)[16]) {
+    const int lane = threadIdx.x & 63, i = lane & 15;
+    double dk = 1.0;  // lanes with i = k: pivot k
+    double r = rcp_nr(row_value<0>(p[0]));
+    for_const<0, 16>([&](auto kc) {
+        constexpr int k = decltype(kc)::value;
+        if (i == k) dk = p[k];
+        const double lp = p[k] * r, la = a[k] * r;
+        for_const<k + 1, 16>([&](auto jc) {
+            constexpr int j = decltype(jc)::value;
+            const double s = row_value<j>(p[k]);
+            p[j] = __builtin_fma(-lp, s, p[j]);
+            a[j] = __builtin_fma(-la, s, a[j]);
+            // the next pivot's reciprocal, the chain of this loop, as soon as the pivot is final
+            if constexpr (j == k + 1) r = rcp_nr(row_value<j>(p[j]));
+        });
+        // every update happens in its own column: put off to a later one, its operands would spill
+#pragma unroll
+        for (int j = k + 1; j < 16; j++) hold(a[j]);
+        __builtin_amdgcn_sched_barrier(0);
+    });
+    const double s = sqrt(dk), rs = rcp_nr(s);
+    for_const<0, 16>([&](auto kc) {
+        constexpr int k = decltype(kc)::value;
+        const double c = row_value<k>(rs);  // outside the selection: every lane takes part in the move
+        a[k] = lane == k ? s : a[k] * c;
+    });
+    return !(dk > 0.0);
+}
+
+// X_KK = L_KK^{-1} for the 16x16 lower-triangular diagonal block at Lk (X block at Xk, all of it written), by one
+// wave: lane r solves row r of the identity, e_r L^{-T}, which is column r of the inverse.
+__device__ __forceinline__ void tri_inv16(const double* Lk, double* Xk) {
+    const int lane = threadIdx.x & 63, i = lane & 15;
+    double l[16], b[16];  // l: row i of the block
+#pragma unroll
+    for (int k = 0; k < 16; k++) {
+        l[k] = Lk[i + k * DP];
+        b[k] = i == k ? 1.0 : 0.0;
+    }
+    const double rd = rcp_nr(Lk[i + i * DP]);
+    for_const<0, 16>([&](auto kc) {
+        constexpr int k = decltype(kc)::value;
+        b[k] *= row_value<k>(rd);
+        for_const<k + 1, 16>([&](auto jc) {
+            constexpr int j = decltype(jc)::value;
+            b[j] = __builtin_fma(-b[k], row_value<j>(l[k]), b[j]);
+        });
+    });
+    if (lane < 16) {
+#pragma unroll
+        for (int k = 0; k < 16; k++) Xk[k + i * DP] = b[k];
+    }
+}
+
+// T_IJ = sum_{Q=J}^{I-1} L_IQ X_QJ (one wave): the off-diagonal block X_IJ of the inverse is -X_II T_IJ.
+__device__ __forceinline__ d4_t tri_inv_sum(const double* D, const double* X, int I, int J) {
+    d4_t T = {0, 0, 0, 0};
+    for (int Q = J; Q < I; Q++) T = mma16(T, D + 16 * I + 16 * Q * DP, X + 16 * Q + 16 * J * DP, false);
+    return T;
+}
+__device__ __forceinline__ void tri_inv_block(const double* D, double* X, int I, int J) {
+    const d4_t T = tri_inv_sum(D, X, I, J);
+    put16(X + 16 * I + 16 * J * DP, mma16_reg(X + 16 * I + 16 * I * DP, T), -1.0, false);
+}
+// Off-diagonal blocks of X = L^{-1} from L (D) and the diagonal inverses already in X, in order of I - J (one wave
+// per block).
 __device__ __forceinline__ void tri_inv_offdiag(const double* D, double* X) {
-    const int wv = threadIdx.x >> 6;
+    const int wv = wave_uniform((int)threadIdx.x >> 6);
     for (int d = 1; d < 4; d++) {
-        const int J = wv, I = wv + d;
-        if (I < 4) {
-            d4_t T = {0, 0, 0, 0};
-            for (int Q = J; Q < I; Q++) T = mma16(T, D + 16 * I + 16 * Q * DP, X + 16 * Q + 16 * J * DP, false);
-            put16(X + 16 * I + 16 * J * DP, mma16_reg(X + 16 * I + 16 * I * DP, T), -1.0, false);
-        }
+        if (wv + d < 4) tri_inv_block(D, X, wv + d, wv);
         __syncthreads();
     }
 }
 
 // Factor D in place (lower; the upper part is left undefined) and write X = L^{-1}
-// (lower, upper part zero). Returns the first failing local column + 1 (0 if
+// (lower, upper part zero); the LDS word after X is used too (POTRF_LDS bytes from D). Returns the first failing local column + 1 (0 if
 // positive definite) to every thread.
+// Four 16-column panels, each by wave 0 alone in registers (panel16): the chain of 64 pivots is what bounds this
+// block, and a pivot step through LDS with a barrier takes ~0.25 us where one in registers takes ~0.1 us. The panel's
+// spare lanes carry the identity, so the block's inverse comes out of the same pass; the other waves meanwhile do the
+// updates that the next panel does not wait for and the off-diagonal blocks of the inverse.
 __device__ __forceinline__ int lds_potrf_inv64(double* D, double* X, int w) {
-    const int tid = threadIdx.x, wv = tid >> 6;
-    const int ti = tid & 15, tj = tid >> 4;
-    __shared__ int s_bad;
-    if (tid == 0) s_bad = 0;
-    for (int e = tid; e < DB * DP; e += NTHREADS) X[e] = 0.0;
+    const int tid = threadIdx.x, lane = tid & 63, wv = wave_uniform(tid >> 6);
+    int* s_bad = reinterpret_cast<int*>(X + DB * DP);
+    if (tid == 0) *s_bad = 0;
+    // D_IJ -= L_IK L_JK^T
+    auto update = [&](int I, int J, int K) {
+        const d4_t acc = mma16(d4_t{0, 0, 0, 0}, D + 16 * I + 16 * K * DP, D + 16 * J + 16 * K * DP, true);
+        put16(D + 16 * I + 16 * J * DP, acc, -1.0, true);
+    };
+    d4_t T = {0, 0, 0, 0};
     __syncthreads();
+#pragma unroll 1
     for (int K = 0; K < 4; K++) {
         const int k0 = 16 * K;
-        double* Dk = D + k0 + k0 * DP;
-        // diagonal block: unscaled right-looking elimination, then column scaling
-        for (int k = 0; k < 16; k++) {
-            const double dkk = Dk[k + k * DP];
-            if (tid == 0 && !(dkk > 0.0) && s_bad == 0 && k0 + k < w) s_bad = k0 + k + 1;
-            if (ti > k && tj > k && ti >= tj) Dk[ti + tj * DP] -= Dk[ti + k * DP] * Dk[tj + k * DP] * rcp_nr(dkk);
+        // panel K: wave 0 holds rows k0 .. 63 and, in the lanes these leave, the identity; of panel 0 they leave none,
+        // and wave 1 repeats the diagonal block with the identity below it
+        if (wv == 0 || (wv == 1 && K == 0)) {
+            const int nreal = wv == 0 ? DB - k0 : 16, e = lane - nreal;
+            const int row = min(k0 + lane, DB - 1);
+            double p[16], a[16];
+#pragma unroll
+            for (int c = 0; c < 16; c++) {
+                p[c] = D[(k0 + (lane & 15)) + (k0 + c) * DP];
+                a[c] = D[row + (k0 + c) * DP];
+                if (lane >= nreal) a[c] = c == e ? 1.0 : 0.0;
+            }
+            if (K == 0) __syncthreads();  // both waves have read the block before wave 0 writes its factor
+            const bool bad = panel16(p, a);
+            if (wv == 0 && lane < nreal) {
+#pragma unroll
+                for (int c = 0; c < 16; c++) D[(k0 + lane) + (k0 + c) * DP] = a[c];
+            } else if (e >= 0 && e < 16) {  // row e of L_KK^{-T}
+#pragma unroll
+                for (int c = 0; c < 16; c++) X[(k0 + c) + (k0 + e) * DP] = a[c];
+            }
+            if (wv == 0) {
+                const unsigned long long m = __ballot(lane < 16 && k0 + lane < w && bad);
+                if (m && lane == 0 && *s_bad == 0) *s_bad = k0 + __ffsll((long long)m);
+            }
+        } else if (K == 0) {  // waves 2, 3: the blocks above the diagonal of X
+            for (int q = wv - 2; q < 6; q += 2) {
+                const int J = q < 3 ? 3 : q < 5 ? 2 : 1, I = q < 3 ? q : q < 5 ? q - 3 : 0;
+#pragma unroll
+                for (int r = 0; r < 4; r++) X[16 * I + (lane & 15) + (16 * J + (lane >> 4) + 4 * r) * DP] = 0.0;
+            }
             __syncthreads();
-        }
-        const double sj = sqrt(Dk[tj + tj * DP]);
-        const double v = Dk[ti + tj * DP];
-        __syncthreads();
-        if (ti > tj) Dk[ti + tj * DP] = v * rcp_nr(sj);
-        else if (ti == tj) Dk[ti + tj * DP] = sj;
-        __syncthreads();
-        tri_inv16(Dk, X + k0 + k0 * DP);
-        if (K == 3) break;
-        // panel: L_IK = D_IK X_KK^T (one wave per block below)
-        {
-            const int I = K + 1 + wv;
-            if (I < 4) {
-                double* Dik = D + 16 * I + k0 * DP;
-                const d4_t acc = mma16(d4_t{0, 0, 0, 0}, Dik, X + k0 + k0 * DP, true);
-                put16(Dik, acc, 1.0, false);
-            }
+        } else if (K == 1) {
+            if (wv == 1) update(3, 2, 0);
+            if (wv == 2) update(3, 3, 0);
+        } else if (K == 3) {
+            T = tri_inv_sum(D, X, 3, wv - 1);
         }
         __syncthreads();
-        // trailing update: D_IJ -= L_IK L_JK^T for K < J <= I < 4
-        {
-            const int nblk = (3 - K) * (4 - K) / 2;
-            for (int q = wv; q < nblk; q += 4) {
-                int J = K + 1, rem = q;
-                while (rem >= 4 - J) { rem -= 4 - J; J++; }
-                const int I = J + rem;
-                const d4_t acc = mma16(d4_t{0, 0, 0, 0}, D + 16 * I + k0 * DP, D + 16 * J + k0 * DP, true);
-                put16(D + 16 * I + 16 * J * DP, acc, -1.0, true);
-            }
+        // what panel K + 1 waits for first
+        if (K == 0) {
+            if (wv < 3) update(1 + wv, 1, 0);
+            else update(2, 2, 0);
+        } else if (K == 1) {
+            if (wv == 0) update(2, 2, 1);
+            if (wv == 1) update(3, 2, 1);
+            if (wv == 2) update(3, 3, 1);
+            if (wv == 3) tri_inv_block(D, X, 1, 0);
+        } else if (K == 2) {
+            if (wv == 0) update(3, 3, 2);
+            if (wv == 1) tri_inv_block(D, X, 2, 1);
+            if (wv == 2) tri_inv_block(D, X, 2, 0);
+        } else if (wv > 0) {
+            put16(X + 48 + 16 * (wv - 1) * DP, mma16_reg(X + 48 + 48 * DP, T), -1.0, false);
         }
         __syncthreads();
     }
-    tri_inv_offdiag(D, X);
-    return s_bad;
+    return *s_bad;
 }
 
 // In-place style inverse of a lower-triangular 64x64 L held in D (w valid, identity
 // padding set here): X = L^{-1}, lower, upper part zero.
 __device__ __forceinline__ void lds_trtri64(double* D, double* X, int w) {
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, wv = wave_uniform(tid >> 6);
     for (int e = tid; e < DB * DB; e += NTHREADS) {
         const int i = e % DB, j = e / DB;
         if (i >= w || j >= w) D[i + j * DP] = (i == j) ? 1.0 : 0.0;
     }
     for (int e = tid; e < DB * DP; e += NTHREADS) X[e] = 0.0;
     __syncthreads();
-    for (int K = 0; K < 4; K++) tri_inv16(D + 16 * K + 16 * K * DP, X + 16 * K + 16 * K * DP);
+    tri_inv16(D + 16 * wv + 16 * wv * DP, X + 16 * wv + 16 * wv * DP);
+    __syncthreads();
     tri_inv_offdiag(D, X);
 }
 
@@ -1286,9 +1392,8 @@ constexpr int LDS_GEMM_BF16_1 = GemmNTbf16<float, GEMM_BM, GEMM_BM, false, true>
 template <typename TS, int PREC> constexpr int gemm_item_lds() {
     return PREC == P_BF16X3 ? LDS_GEMM_BF16 : PREC == P_BF16 ? LDS_GEMM_BF16_1 : sizeof(TS) == 8 ? LDS_GEMM_F64 : LDS_GEMM_F32;
 }
-constexpr int LDS_POTRF = PotrfGemm<double>::G::LDS_BYTES > 2 * DB * DP * 8 ? PotrfGemm<double>::G::LDS_BYTES
-                                                                             : 2 * DB * DP * 8;
-constexpr int LDS_POTRF_ROWS = GemmNT<double, double, double, DB, DB, DB, false, true>::STAGE * 8;
+constexpr int LDS_POTRF = cmax(PotrfGemm<double>::G::LDS_BYTES, POTRF_LDS);
+constexpr int LDS_POTRF_ROWS = cmax(GemmNT<double, double, double, DB, DB, DB, false, true>::STAGE * 8, POTRF_LDS);
 constexpr int LDS_TRSM = cmax(GemmNT<double, double, double, TRSM_BM, DB, 32, true, true>::LDS_BYTES,
                               GemmNT<double, double, double, TRSM_BM, DB, DB, false, true>::STAGE * 8);
 constexpr int LDS_TRSM_F32 = cmax(GemmNT<float, float, float, TRSM_BM_F32, DB, trsm_bk<float>(), true, true>::LDS_BYTES,
