@@ -254,23 +254,22 @@ __global__ __launch_bounds__(NTHREADS, vset_occupancy(VM)) void k_persistent(Dev
             // ran items of the task has released.
             if (__hip_atomic_fetch_add(g.xcd_run + (long)task * NXCD + my_xcd, -1, __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_AGENT) == 1)
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+                release_agent();
             if (!ran) __hip_atomic_store(g.abort_flag, 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             const uint64_t t1 = g.trace ? wall_clock64() : 0;
-            // Counters are relaxed: the release fence above publishes this item's outputs. The thread
-            // that takes a counter to zero acquires what the other decrements released and releases it again
-            // before its own next counter update or queue entries (one acq_rel fence per task, and per
-            // successor it makes ready).
+            // Counters are relaxed: the release above has written this item's outputs back before the decrement.
+            // The thread that takes a counter to zero acquires what the other decrements released; it has nothing
+            // of its own left to write back, so its next counter update and queue entries need no release.
             const int left =
                 __hip_atomic_fetch_add(g.items_left + task, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - 1;
             if (left == 0) {  // last item of the task: release its successors
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "agent");
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
                 for (int q = g.out_ptr[task]; q < g.out_ptr[task + 1]; q++) {
                     const int s = g.out_idx[q];
                     const int d =
                         __hip_atomic_fetch_add(g.deps + s, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - 1;
                     if (d == 0) {
-                        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "agent");
+                        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
                         push_task(g, s);
                     }
                 }

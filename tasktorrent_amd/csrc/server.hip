@@ -121,10 +121,10 @@ __global__ __launch_bounds__(NTHREADS) void k_server(DevServer s) {
         srv_exec(s, t, task, item, lds);
         __syncthreads();
         if (tid == 0) {
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+            release_agent();
             if (t.kind != S_CHECK) {
                 const int left =
-                    __hip_atomic_fetch_add(s.items_left + task, -1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) - 1;
+                    __hip_atomic_fetch_add(s.items_left + task, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - 1;
                 if (left == 0) srv_complete(s, task);
             }
         }

@@ -104,7 +104,9 @@ struct DevServer {
     int64_t idle_limit;
 };
 
+// (one thread; what the task reads is released before the first entry is written)
 __device__ __forceinline__ void srv_push(const DevServer& s, int task) {
+    release_agent();
     const SrvTask t = s.tasks[task];
     const SrvRing& R = s.rings[t.bucket];
     const unsigned long long cap = 1ull << s.ring_log2;
@@ -114,18 +116,25 @@ __device__ __forceinline__ void srv_push(const DevServer& s, int task) {
         const unsigned long long idx = pos + r;
         const unsigned long long lap = ((idx >> s.ring_log2) + 1) & 0xFFFFFFull;
         const unsigned long long e = (lap << 40) | ((unsigned long long)task << 16) | (unsigned long long)r;
-        __hip_atomic_store(R.slots + (idx & (cap - 1)), e, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(R.slots + (idx & (cap - 1)), e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     __hip_atomic_fetch_add(R.count, (long long)t.n_items, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // A task finished: decrement successors, push those that become ready.
 __device__ __forceinline__ void srv_complete(const DevServer& s, int task) {
+    // acquires what the task's items released before they counted it down, and with each successor that becomes
+    // ready what its other predecessors released
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    release_agent();
     const SrvTask t = s.tasks[task];
     for (int q = 0; q < t.edge_cnt; q++) {
         const int succ = s.edges[t.edge_off + q];
-        const int d = __hip_atomic_fetch_add(s.deps + succ, -1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) - 1;
-        if (d == 0) srv_push(s, succ);
+        const int d = __hip_atomic_fetch_add(s.deps + succ, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - 1;
+        if (d == 0) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            srv_push(s, succ);
+        }
     }
 }
 
@@ -154,10 +163,10 @@ __device__ __forceinline__ void srv_admit(const DevServer& s, int slot) {
         const long words = (long)(cl[c].bytes >> 2);
         for (long w = threadIdx.x; w < words; w += NTHREADS) dst[w] = src[w];
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");  // each wave publishes its own copies
+    release_agent();  // each wave publishes its own copies
     __syncthreads();
     if (threadIdx.x == 0) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        // (the copies have been read from the host's memory: release_agent waited for all of them)
         __hip_atomic_store(&m->state, 2, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
         __hip_atomic_fetch_add(s.active, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         srv_push(s, s_seed);
@@ -276,6 +285,7 @@ __device__ __forceinline__ void srv_exec(const DevServer& s, const SrvTask& t, i
                 const long tot = (long)q.n * q.nrhs;
                 for (long e = threadIdx.x; e < tot; e += NTHREADS) q.x_host[e] = q.X[e];
                 __atomic_thread_fence(__ATOMIC_RELEASE);  // system scope: each wave's part of X reaches the host
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (behind the write-back, see release_agent)
                 __syncthreads();
                 if (threadIdx.x == 0) {
                     SrvDone& d = s.done[q.done_slot];
@@ -292,7 +302,7 @@ __device__ __forceinline__ void srv_exec(const DevServer& s, const SrvTask& t, i
                     q.flags_b[e] = 0;
                 }
                 for (int e = threadIdx.x; e < 3 * 32; e += NTHREADS) q.norms[e] = 0;
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+                release_agent();
                 __syncthreads();
                 if (threadIdx.x == 0) {
                     const int ids[4] = {q.t_fwd, q.t_bwd, q.t_res, q.t_chk};
@@ -300,7 +310,6 @@ __device__ __forceinline__ void srv_exec(const DevServer& s, const SrvTask& t, i
                     s.deps[q.t_bwd] = 1;
                     s.deps[q.t_res] = 1;
                     s.deps[q.t_chk] = 1;
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
                     srv_push(s, q.t_fwd);
                 }
             }

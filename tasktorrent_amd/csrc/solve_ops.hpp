@@ -343,7 +343,10 @@ __device__ __forceinline__ void item_sweep(const DevMat& M, const SweepTab& tab,
             }
         }
     __syncthreads();
-    if (threadIdx.x == 0) __hip_atomic_fetch_add(flags, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x == 0) {
+        release_agent();
+        __hip_atomic_fetch_add(flags, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
 }
 
 // LDS of item_sweep<.., PF> (and of item_resid<NR, false> for TC = double).

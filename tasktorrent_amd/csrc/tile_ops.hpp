@@ -38,6 +38,15 @@ template <typename T> __device__ __forceinline__ T* wave_uniform(T* p) {
     return (T*)(((unsigned long long)hi << 32) | lo);
 }
 
+// Agent-scope release that has completed when it returns: buffer_wbl2 starts the write-back of this XCD's L2 and
+// counts in vmcnt, but the compiler drops the wait that belongs behind it wherever it sees no other memory operation
+// of this wave outstanding (after an explicit vmcnt(0), or after a barrier), and the store or atomic that announces
+// the data would then pass the write-back. Every announcement therefore goes through this and is relaxed itself.
+__device__ __forceinline__ void release_agent() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
 // The workgroup's dynamic LDS as a pointer in a scalar register. In a function called out of line its base is read
 // from a table in memory, and the compiler reads it again at every use it cannot hoist (a memory round trip in front
 // of LDS accesses on the critical path); the offset is opaque here, so it is read once.
@@ -738,7 +747,10 @@ __device__ __forceinline__ void item_gemm_acc(const TS* __restrict__ A, long lda
                     }
                 }
         __syncthreads();
-        if (threadIdx.x == 0) __hip_atomic_store(lock, 0, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+        if (threadIdx.x == 0) {
+            release_agent();
+            __hip_atomic_store(lock, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
     };
     if constexpr (PREC == P_BF16 || PREC == P_BF16X3) {
         body((GemmNTbf16<TS, GEMM_BM, GEMM_BM, PREC == P_BF16X3, true>*)nullptr);

@@ -484,7 +484,10 @@ __device__ __forceinline__ void item_lsweep(const DevMat& M, const LSweepTab& lt
         }
         __builtin_amdgcn_s_waitcnt(0x0F70);
         __syncthreads();  // waves 4-7 only: waves 0-3 have ended
-        if (threadIdx.x == NTHREADS) __hip_atomic_fetch_add(ocnt + t, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+        if (threadIdx.x == NTHREADS) {
+            release_agent();
+            __hip_atomic_fetch_add(ocnt + t, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
         return;
     }
 
@@ -616,7 +619,10 @@ __device__ __forceinline__ void item_lsweep(const DevMat& M, const LSweepTab& lt
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the stores are in the L2 before the barrier
     __syncthreads();                     // (also: every wave is done reading As)
-    if (threadIdx.x == 0) __hip_atomic_fetch_add(rcnt + t, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x == 0) {
+        release_agent();
+        __hip_atomic_fetch_add(rcnt + t, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     // all of r'_t published: waves 4-7 take step C
     ls_wait(rcnt + t, nbt, err, spin_limit, false);
 }
