@@ -45,16 +45,6 @@ struct StreamPlan {
     int vset = N_VSETS - 1;  // executor instantiation covering the plan's item variants
 };
 
-// POTRF tasks (graphs and stream plans) run as one item per 64-row block of the tile (item_potrf_rows,
-// default); TTAD_POTRF_ROWS=0 runs each as one single-workgroup item (for comparisons).
-static bool potrf_rows_enabled() {
-    static const bool on = [] {
-        const char* v = getenv("TTAD_POTRF_ROWS");
-        return !(v && v[0] == '0');
-    }();
-    return on;
-}
-
 static std::shared_ptr<StreamPlan> build_stream_plan(ttad_matrix* M, int prec, int& rc) {
     auto plan = std::make_shared<StreamPlan>();
     std::vector<DevTask> tasks;
@@ -78,8 +68,8 @@ static std::shared_ptr<StreamPlan> build_stream_plan(ttad_matrix* M, int prec, i
         t.i = i;
         t.j = j;
         t.k = k;
-        t.n_items = kind == K_POTRF && potrf_rows_enabled() ? potrf_row_items(M->bsz[j])
-                                                            : std::max(1, items_of(kind, M->bsz[i], M->bsz[j], (int)M->elem));
+        t.n_items = kind == K_POTRF ? potrf_items(M->bsz[j])
+                                    : std::max(1, items_of(kind, M->bsz[i], M->bsz[j], (int)M->elem));
         t.bucket = 0;
         t.crit = 0;
         return t;
@@ -140,7 +130,7 @@ int ttad_init(int device, ttad_context** out) {
     if (e == hipSuccess) e = kernels_init();
     if (e == hipSuccess) e = factor_check_init();
     if (e == hipSuccess) e = solve_init();
-    if (e == hipSuccess) e = c->scratch_info.alloc(sizeof(int));
+    if (e == hipSuccess) e = c->scratch_info.alloc(2 * sizeof(int));
     // this device's copy of the no-allocation scratch (the device is current here)
     if (e == hipSuccess) e = hipGetSymbolAddress((void**)&c->noalloc_dinv, HIP_SYMBOL(scratch));
     if (e != hipSuccess) {
@@ -223,12 +213,25 @@ static int potrf_common(ttad_context* ctx, int prec, int n, void* A, int lda, in
     int rc = ensure_dinv(ctx, n);
     if (rc) return rc;
     hipStream_t s = pick(ctx, stream);
-    TTAD_HIP(hipMemsetAsync(ctx->scratch_info.p, 0, sizeof(int), s));
-    launch_raw_potrf(prec, A, lda, n, ctx->scratch_dinv.as<double>(), ctx->scratch_info.as<int>(), s);
+    const size_t fl = (size_t)potrf_flags(n) * sizeof(int32_t);
+    if (ctx->scratch_pflags.bytes < fl) {
+        TTAD_HIP(ctx->scratch_pflags.alloc(fl));
+        TTAD_HIP(hipMemsetAsync(ctx->scratch_pflags.p, 0, fl, s));
+    }
+    int* info_err = ctx->scratch_info.as<int>();  // the factorization's info, and the items' error word
+    TTAD_HIP(hipMemsetAsync(info_err, 0, 2 * sizeof(int), s));
+    launch_raw_potrf(prec, A, lda, n, ctx->scratch_dinv.as<double>(), info_err, ctx->scratch_pflags.as<int32_t>(),
+                     info_err + 1, s);
     TTAD_HIP(hipGetLastError());
-    int h = 0;
-    TTAD_HIP(hipMemcpyAsync(&h, ctx->scratch_info.p, sizeof(int), hipMemcpyDeviceToHost, s));
+    int he[2] = {0, 0};
+    TTAD_HIP(hipMemcpyAsync(he, info_err, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
     TTAD_HIP(hipStreamSynchronize(s));
+    if (he[1]) {
+        (void)hipMemsetAsync(ctx->scratch_pflags.p, 0, ctx->scratch_pflags.bytes, s);
+        (void)hipStreamSynchronize(s);
+        return set_error(TTAD_ERR_TIMEOUT, "potrf: an item waited past the device watchdog");
+    }
+    const int h = he[0];
     if (info) *info = h;
     return h ? set_error(TTAD_ERR_NOT_SPD, "potrf: non-positive pivot at column %d", h) : TTAD_OK;
 }
@@ -366,7 +369,9 @@ int ttad_matrix_create(ttad_context* ctx, int num_blocks, const int* block_sizes
     TTAD_HIP(M->tab_tiles.alloc((size_t)nt * nt * sizeof(void*)));
     TTAD_HIP(M->tab_dinv.alloc(nt * sizeof(double*)));
     TTAD_HIP(M->info.alloc(sizeof(int)));
-    TTAD_HIP(M->pflags.alloc((size_t)nt * POTRF_FLAGS * sizeof(int32_t)));
+    const int pf_stride = potrf_flags(*std::max_element(M->bsz.begin(), M->bsz.end()));
+    M->pflags_bytes = (size_t)nt * pf_stride * sizeof(int32_t);
+    TTAD_HIP(M->pflags.alloc(M->pflags_bytes));
     TTAD_HIP(M->locks.alloc((size_t)nt * nt * 16 * sizeof(int32_t)));
     TTAD_HIP(M->desc.alloc(sizeof(DevMat)));
     TTAD_HIP(hipMemcpy(M->tab_bsz.p, M->bsz.data(), nt * 4, hipMemcpyHostToDevice));
@@ -374,7 +379,7 @@ int ttad_matrix_create(ttad_context* ctx, int num_blocks, const int* block_sizes
     TTAD_HIP(hipMemcpy(M->tab_tiles.p, tp.data(), tp.size() * sizeof(void*), hipMemcpyHostToDevice));
     TTAD_HIP(hipMemcpy(M->tab_dinv.p, dp.data(), dp.size() * sizeof(double*), hipMemcpyHostToDevice));
     TTAD_HIP(hipMemset(M->info.p, 0, sizeof(int)));
-    TTAD_HIP(hipMemset(M->pflags.p, 0, (size_t)nt * POTRF_FLAGS * sizeof(int32_t)));
+    TTAD_HIP(hipMemset(M->pflags.p, 0, M->pflags_bytes));
     TTAD_HIP(hipMemset(M->locks.p, 0, (size_t)nt * nt * 16 * sizeof(int32_t)));
     TTAD_HIP(hipMemset(M->tiles.p, 0, off * M->elem));
     DevMat d{};
@@ -386,6 +391,7 @@ int ttad_matrix_create(ttad_context* ctx, int num_blocks, const int* block_sizes
     d.dinv = M->tab_dinv.as<double*>();
     d.info = M->info.as<int32_t>();
     d.pflags = M->pflags.as<int32_t>();
+    d.pf_stride = pf_stride;
     d.locks = M->locks.as<int32_t>();
     M->host_desc = d;
     TTAD_HIP(hipMemcpy(M->desc.p, &d, sizeof(DevMat), hipMemcpyHostToDevice));
@@ -497,7 +503,7 @@ int ttad_potrf_tiled(ttad_context* ctx, ttad_matrix* M, int schedule, int prio_k
     if (info) *info = 0;
     hipStream_t s = pick(ctx, stream);
     TTAD_HIP(hipMemsetAsync(M->info.p, 0, sizeof(int), s));
-    TTAD_HIP(hipMemsetAsync(M->pflags.p, 0, (size_t)M->nt * POTRF_FLAGS * sizeof(int32_t), s));
+    TTAD_HIP(hipMemsetAsync(M->pflags.p, 0, M->pflags_bytes, s));
     int rc = TTAD_OK;
     ctx->ev_valid = false;
     ctx->kernel_s = -1.0;
@@ -523,7 +529,7 @@ int ttad_potrf_tiled(ttad_context* ctx, ttad_matrix* M, int schedule, int prio_k
         TTAD_HIP(hipStreamSynchronize(s));
         if (err) {
             (void)hipMemset(plan->d_err.p, 0, sizeof(int32_t));
-            if (err == 1) return set_error(TTAD_ERR_TIMEOUT, "potrf_tiled: a row-block POTRF item waited too long");
+            if (err == 1) return set_error(TTAD_ERR_TIMEOUT, "potrf_tiled: a POTRF item waited too long");
             return set_error(TTAD_ERR_DEVICE, "potrf_tiled: item variant missing from the executor (%d)", err);
         }
     } else if (schedule == TTAD_SCHED_PERSISTENT) {
@@ -739,8 +745,8 @@ static int graph_prepare(ttad_graph* g) {
                                  x.k);
             if ((x.kind == K_GEMM || x.kind == K_SYRK) && ((x.prec == P_F64) != (M->storage == P_F64)))
                 return set_error(TTAD_ERR_INVALID, "graph: task %d precision does not match tile storage", t);
-            x.n_items = x.kind == K_POTRF && potrf_rows_enabled() ? potrf_row_items(M->bsz[x.j])
-                                                                  : std::max(1, items_of(x.kind, M->bsz[x.i], M->bsz[x.j], (int)M->elem));
+            x.n_items = x.kind == K_POTRF ? potrf_items(M->bsz[x.j])
+                                          : std::max(1, items_of(x.kind, M->bsz[x.i], M->bsz[x.j], (int)M->elem));
         }
         int needed = 0;
         for (auto& x : g->tasks)
@@ -890,8 +896,8 @@ int ttad_graph_launch(ttad_graph* g, int n_workers, int trace, void* stream) {
     for (auto* M : g->mats)
         if (M) {
             TTAD_HIP(hipMemsetAsync(M->info.p, 0, sizeof(int), g->stream));
-            // row-block POTRF flags: cleared by every completed task, and here after a stopped run
-            TTAD_HIP(hipMemsetAsync(M->pflags.p, 0, (size_t)M->nt * POTRF_FLAGS * sizeof(int32_t), g->stream));
+            // POTRF flags: cleared by every completed task, and here after a stopped run
+            TTAD_HIP(hipMemsetAsync(M->pflags.p, 0, M->pflags_bytes, g->stream));
             TTAD_HIP(hipMemsetAsync(M->locks.p, 0, (size_t)M->nt * M->nt * 16 * sizeof(int32_t), g->stream));
         }
     TTAD_HIP(hipEventRecord(g->ev_start, g->stream));

@@ -123,8 +123,8 @@ __host__ __device__ inline int item_variant(int kind, int prec, int storage) {
 // LDS of an executor instantiation: the largest item of its variants.
 constexpr int vset_lds(int vm) {
     int b = 0;
-    if (vm & V_F64S) b = cmax(b, cmax(cmax(LDS_GEMM_F64, cmax(LDS_POTRF, LDS_POTRF_ROWS)), LDS_TRSM));
-    if (vm & V_F32S) b = cmax(b, cmax(cmax(LDS_POTRF, LDS_POTRF_ROWS), LDS_TRSM_F32));
+    if (vm & V_F64S) b = cmax(b, cmax(cmax(LDS_GEMM_F64, LDS_POTRF), LDS_TRSM));
+    if (vm & V_F32S) b = cmax(b, cmax(LDS_POTRF, LDS_TRSM_F32));
     if (vm & V_G32) b = cmax(b, LDS_GEMM_F32);
     if (vm & V_GBF16) b = cmax(b, LDS_GEMM_BF16_1);
     if (vm & V_GBF16X3) b = cmax(b, LDS_GEMM_BF16);
@@ -150,20 +150,12 @@ inline int vset_index(int needed) {
 // that a GEMM item sharing the CU (two workgroups per CU) does not halve their MFMA share.
 template <typename TS, int VM>
 __device__ __attribute__((noinline)) void potrf_call(TS* A, long lda, int n, double* dinv, int* info, int col_off,
+                                                     int it, int32_t* flags, int32_t* err, int64_t spin_limit,
                                                      char* lds) {
     __builtin_amdgcn_s_setprio(3);
     item_potrf<TS>(wave_uniform(A), wave_uniform((int)lda), wave_uniform(n), wave_uniform(dinv), wave_uniform(info),
-                   wave_uniform(col_off), lds_uniform(lds));
-    __builtin_amdgcn_s_setprio(0);
-}
-template <typename TS, int VM>
-__device__ __attribute__((noinline)) void potrf_rows_call(TS* A, long lda, int n, double* dinv, int* info, int col_off,
-                                                          int rb, int32_t* prog, int32_t* err, int64_t spin_limit,
-                                                          char* lds) {
-    __builtin_amdgcn_s_setprio(3);
-    item_potrf_rows<TS>(wave_uniform(A), wave_uniform((int)lda), wave_uniform(n), wave_uniform(dinv),
-                        wave_uniform(info), wave_uniform(col_off), wave_uniform(rb), wave_uniform(prog),
-                        wave_uniform(err), spin_limit, lds_uniform(lds));
+                   wave_uniform(col_off), wave_uniform(it), wave_uniform(flags), wave_uniform(err), spin_limit,
+                   lds_uniform(lds));
     __builtin_amdgcn_s_setprio(0);
 }
 // Accumulate-mode GEMM items are called out of line too, so the default GEMM loop keeps its registers.
@@ -184,8 +176,8 @@ __device__ __attribute__((noinline)) void trsm_call(const TS* L, long ldl, const
 }
 
 // Execute work item `it` of task t. All 256 threads participate. Returns false
-// (doing nothing) for an item variant outside VM. A POTRF task of more than one item
-// runs as row-block items that wait on each other (item_potrf_rows): the caller must
+// (doing nothing) for an item variant outside VM. The items of a POTRF task wait on
+// each other (item_potrf): the caller must
 // have every lower-numbered item of the task running or done; their waits give up
 // after spin_limit ticks or once *err is nonzero (and set *err = 1 when they time out).
 template <int VM>
@@ -207,30 +199,17 @@ __device__ __forceinline__ bool exec_item(const DevTask& t, int it, const DevMat
     switch (t.kind) {
         case K_POTRF: {
             const int j = t.j, n = M.bsz[j];
-            if (t.n_items > 1) {
-                int32_t* prog = M.pflags + (long)j * POTRF_FLAGS;
-                if constexpr ((VM & V_F64S) != 0)
-                    if (f64s) {
-                        potrf_rows_call<double, VM>((double*)tile(j, j), n, n, M.dinv[j], M.info, M.boff[j], it, prog,
-                                                    err, spin_limit, lds);
-                        return true;
-                    }
-                if constexpr ((VM & V_F32S) != 0)
-                    if (!f64s) {
-                        potrf_rows_call<float, VM>((float*)tile(j, j), n, n, M.dinv[j], M.info, M.boff[j], it, prog,
-                                                   err, spin_limit, lds);
-                        return true;
-                    }
-                return false;
-            }
+            int32_t* flags = M.pflags + (long)j * M.pf_stride;
             if constexpr ((VM & V_F64S) != 0)
                 if (f64s) {
-                    potrf_call<double, VM>((double*)tile(j, j), n, n, M.dinv[j], M.info, M.boff[j], lds);
+                    potrf_call<double, VM>((double*)tile(j, j), n, n, M.dinv[j], M.info, M.boff[j], it, flags, err,
+                                           spin_limit, lds);
                     return true;
                 }
             if constexpr ((VM & V_F32S) != 0)
                 if (!f64s) {
-                    potrf_call<float, VM>((float*)tile(j, j), n, n, M.dinv[j], M.info, M.boff[j], lds);
+                    potrf_call<float, VM>((float*)tile(j, j), n, n, M.dinv[j], M.info, M.boff[j], it, flags, err,
+                                          spin_limit, lds);
                     return true;
                 }
             return false;

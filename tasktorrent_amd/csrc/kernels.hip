@@ -22,8 +22,8 @@ __global__ __launch_bounds__(NTHREADS, vset_occupancy(VM)) void k_items(const De
         else hi = mid - 1;
     }
     const DevTask t = tasks[lo];
-    // row-block POTRF items wait only on lower-numbered blocks of the same launch, which
-    // are dispatched first
+    // POTRF items wait only on lower-numbered blocks of the same launch, which are
+    // dispatched first
     if (!exec_item<VM>(t, g - prefix[lo], mats, lds, err, (int64_t)500000000) && threadIdx.x == 0) atomicCAS(err, 0, 3);
 }
 
@@ -353,10 +353,12 @@ __global__ __launch_bounds__(NTHREADS, 2 * (gemm_item_lds<TS, PREC>() + 1024) <=
     item_gemm<TS, PREC>(A, lda, B, ldb, C, ldc, m, n, K, rb * GEMM_BM, cb * GEMM_BM, syrk != 0, alpha, beta, lds);
 }
 
+// The items wait only on lower-numbered blocks of the launch, which are dispatched first.
 template <typename TS>
-__global__ __launch_bounds__(NTHREADS) void k_raw_potrf(TS* A, long lda, int n, double* dinv, int* info) {
+__global__ __launch_bounds__(NTHREADS, 2) void k_raw_potrf(TS* A, long lda, int n, double* dinv, int* info,
+                                                           int32_t* flags, int32_t* err) {
     extern __shared__ __align__(16) char lds[];
-    item_potrf<TS>(A, lda, n, dinv, info, 0, lds);
+    item_potrf<TS>(A, lda, n, dinv, info, 0, blockIdx.x, flags, err, (int64_t)500000000, lds);
 }
 
 template <typename TS, typename TC>
@@ -580,13 +582,13 @@ void launch_raw_gemm(int prec, const void* A, long lda, const void* B, long ldb,
                            (const float*)A, lda, (const float*)B, ldb, (float*)C, ldc, m, n, K, syrk, alpha, beta);
 }
 
-void launch_raw_potrf(int prec, void* A, long lda, int n, double* dinv, int* info, hipStream_t s) {
+void launch_raw_potrf(int prec, void* A, long lda, int n, double* dinv, int* info, int32_t* flags, int32_t* err,
+                      hipStream_t s) {
+    const dim3 grid(potrf_items(n)), block(NTHREADS);
     if (prec == P_F64)
-        hipLaunchKernelGGL((k_raw_potrf<double>), dim3(1), dim3(NTHREADS), LDS_POTRF, s, (double*)A, lda, n, dinv,
-                           info);
+        hipLaunchKernelGGL((k_raw_potrf<double>), grid, block, LDS_POTRF, s, (double*)A, lda, n, dinv, info, flags, err);
     else
-        hipLaunchKernelGGL((k_raw_potrf<float>), dim3(1), dim3(NTHREADS), LDS_POTRF, s, (float*)A, lda, n, dinv,
-                           info);
+        hipLaunchKernelGGL((k_raw_potrf<float>), grid, block, LDS_POTRF, s, (float*)A, lda, n, dinv, info, flags, err);
 }
 
 void launch_trtri_diag(int prec, const void* L, long ldl, int n, double* dinv, hipStream_t s) {

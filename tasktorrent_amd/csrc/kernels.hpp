@@ -19,7 +19,9 @@ void launch_read_clock(uint64_t* out, hipStream_t s);
 void launch_persistent(int vset, const DevGraph& g, int n_workers, hipStream_t s);
 void launch_raw_gemm(int prec, const void* A, long lda, const void* B, long ldb, void* C, long ldc, int m, int n,
                      int K, int syrk, double alpha, double beta, hipStream_t s);
-void launch_raw_potrf(int prec, void* A, long lda, int n, double* dinv, int* info, hipStream_t s);
+// flags: potrf_flags(n) zeroed ints (left zero); err: set to 1 if an item waited too long.
+void launch_raw_potrf(int prec, void* A, long lda, int n, double* dinv, int* info, int32_t* flags, int32_t* err,
+                      hipStream_t s);
 void launch_trtri_diag(int prec, const void* L, long ldl, int n, double* dinv, hipStream_t s);
 void launch_raw_trsm(int prec, const void* L, long ldl, const double* dinv, void* X, long ldx, int m, int n,
                      hipStream_t s);

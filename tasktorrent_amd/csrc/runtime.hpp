@@ -65,7 +65,8 @@ struct ttad_context {
     int workers_per_cu = 1;            // of the FP64 executor
     int vset_workers_per_cu[8] = {1, 1, 1, 1, 1, 1, 1, 1};  // per executor instantiation
     ttad::DevBuf scratch_dinv;  // inverse diagonal blocks for the raw tile entry points
-    ttad::DevBuf scratch_info;  // one int
+    ttad::DevBuf scratch_info;  // two ints: a raw POTRF's info and its items' error word
+    ttad::DevBuf scratch_pflags;  // flags of the raw POTRF's items (zero between calls)
     double* noalloc_dinv = nullptr;  // this device's address of the static scratch of ttad_dtrsm_noalloc
     // host-sequenced schedules, keyed by (matrix id, prec)
     std::map<std::pair<long long, int>, std::shared_ptr<ttad::StreamPlan>> stream_plans;
@@ -94,6 +95,7 @@ struct ttad_matrix {
     // bf16 hi/lo planes of the off-diagonal tiles (FP32 storage; allocated by the first bf16x3 factorization)
     ttad::DevBuf planes, tab_planes;
     size_t elem = 8;
+    size_t pflags_bytes = 0;
     long long bytes = 0;
     ttad::DevMat host_desc{};
     // 64-row block table of the solve phase (built on first use)

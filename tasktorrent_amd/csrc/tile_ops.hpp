@@ -780,7 +780,6 @@ __device__ __forceinline__ void decode_gemm_item(int it, int tr, bool syrk, int&
 // everything else is 16x16x16 products on FP64 MFMA, one block per wave.
 // ---------------------------------------------------------------------------
 constexpr int DP = DB + 1;
-constexpr int POTRF_LDS = (2 * DB * DP + 2) * 8;  // D, X and a flag
 
 // acc += P Q (q_trans = false) or P Q^T (q_trans = true); P, Q 16x16 blocks in LDS, ld DP.
 __device__ __forceinline__ d4_t mma16(d4_t acc, const double* P, const double* Q, bool q_trans) {
@@ -923,13 +922,15 @@ __device__ __forceinline__ void tri_inv_offdiag(const double* D, double* X) {
 }
 
 // Factor D in place (lower; the upper part is left undefined) and write X = L^{-1}
-// (lower, upper part zero); the LDS word after X is used too (POTRF_LDS bytes from D). Returns the first failing local column + 1 (0 if
+// (lower, upper part zero); the LDS word after X is used too. Returns the first failing local column + 1 (0 if
 // positive definite) to every thread.
 // Four 16-column panels, each by wave 0 alone in registers (panel16): the chain of 64 pivots is what bounds this
 // block, and a pivot step through LDS with a barrier takes ~0.25 us where one in registers takes ~0.1 us. The panel's
 // spare lanes carry the identity, so the block's inverse comes out of the same pass; the other waves meanwhile do the
-// updates that the next panel does not wait for and the off-diagonal blocks of the inverse.
-__device__ __forceinline__ int lds_potrf_inv64(double* D, double* X, int w) {
+// updates that the next panel does not wait for and the off-diagonal blocks of the inverse. `beside` is run by wave 3
+// while panel 0 is factored.
+template <typename F>
+__device__ __forceinline__ int lds_potrf_inv64(double* D, double* X, int w, const F& beside) {
     const int tid = threadIdx.x, lane = tid & 63, wv = wave_uniform(tid >> 6);
     int* s_bad = reinterpret_cast<int*>(X + DB * DP);
     if (tid == 0) *s_bad = 0;
@@ -975,6 +976,7 @@ __device__ __forceinline__ int lds_potrf_inv64(double* D, double* X, int w) {
                 for (int r = 0; r < 4; r++) X[16 * I + (lane & 15) + (16 * J + (lane >> 4) + 4 * r) * DP] = 0.0;
             }
             __syncthreads();
+            if (wv == 3) beside();
         } else if (K == 1) {
             if (wv == 1) update(3, 2, 0);
             if (wv == 2) update(3, 3, 0);
@@ -1018,112 +1020,6 @@ __device__ __forceinline__ void lds_trtri64(double* D, double* X, int w) {
     tri_inv_offdiag(D, X);
 }
 
-// ---------------------------------------------------------------------------
-// POTRF work item: the whole n x n diagonal tile in one workgroup, left-looking
-// over 64-column panels. Per panel: one tall GEMM updates the panel rows p0..n
-// (256 rows per call), the 64x64 diagonal block is factored and inverted in LDS
-// (lds_potrf_inv64), and the rows below are multiplied by the inverse's transpose.
-// Leaves the inverses of the 64x64 diagonal blocks of L in dinv. Arithmetic is
-// FP64 whatever the tile storage (the mixed variants keep the diagonal
-// factorization in FP64).
-// ---------------------------------------------------------------------------
-constexpr int POTRF_BM = 128;  // rows per panel GEMM call
-template <typename TS>
-struct PotrfGemm {
-    using G = GemmNT<TS, TS, double, POTRF_BM, DB, 16>;        // panel update
-    using G2 = GemmNT<TS, double, double, POTRF_BM, DB, 16>;   // times the inverse
-};
-
-template <typename TS>
-__device__ __forceinline__ void item_potrf(TS* __restrict__ A, long lda, int n, double* __restrict__ dinv, int* info, int col_off,
-                           char* lds) {
-    using G = typename PotrfGemm<TS>::G;
-    using G2 = typename PotrfGemm<TS>::G2;
-    double* D = reinterpret_cast<double*>(lds);  // shares the GEMM staging area (used between GEMM calls)
-    double* X = D + DB * DP;
-    const int tid = threadIdx.x;
-    const int nblk = (n + DB - 1) / DB;
-    for (int pb = 0; pb < nblk; pb++) {
-        const int p0 = pb * DB, pw = min(DB, n - p0), rows = n - p0;
-        typename G::acc_t acc[G::WM][G::WN];
-        // panel update: A(p0:n, p) -= L(p0:n, 0:p0) L(p, 0:p0)^T
-        if (p0 > 0) {
-            for (int r0 = 0; r0 < rows; r0 += POTRF_BM) {
-                const int mv = min(POTRF_BM, rows - r0);
-                TTAD_GLOBAL TS* T = gmem(A) + (p0 + r0) + (long)p0 * lda;
-                G::zero(acc);
-                G::run(acc, A + p0 + r0, lda, mv, A + p0, lda, pw, p0, lds);
-#pragma unroll
-                for (int a = 0; a < G::WM; a++)
-#pragma unroll
-                    for (int b = 0; b < G::WN; b++)
-#pragma unroll
-                        for (int r = 0; r < 4; r++) {
-                            const int rr = G::row_of(a, r), cc = G::col_of(b, r);
-                            if (rr < mv && cc < pw && (r0 + rr >= cc)) {
-                                TTAD_GLOBAL TS* q = T + rr + (long)cc * lda;
-                                *q = (TS)((double)(*q) - acc[a][b][r]);
-                            }
-                        }
-            }
-            __syncthreads();
-        }
-        // diagonal block into LDS (identity padding), every load in flight before the
-        // first LDS store; then factor + inverse
-        {
-            constexpr int PER = DB * DB / NTHREADS;
-            const int i = tid % DB, j0 = tid / DB;
-            TTAD_GLOBAL const TS* Ac = gmem(A) + (p0 + i) + (long)p0 * lda;
-            TS v[PER];
-#pragma unroll
-            for (int q = 0; q < PER; q++) {
-                const int j = j0 + q * (NTHREADS / DB);
-                v[q] = (i < pw && j < pw && i >= j) ? Ac[(long)j * lda] : TS(0);
-            }
-#pragma unroll
-            for (int q = 0; q < PER; q++) {
-                const int j = j0 + q * (NTHREADS / DB);
-                D[i + j * DP] = (i < pw && j < pw) ? (double)v[q] : (i == j) ? 1.0 : 0.0;
-            }
-        }
-        __syncthreads();
-        const int bad = lds_potrf_inv64(D, X, pw);
-        if (bad && tid == 0) atomicCAS(info, 0, col_off + p0 + bad);
-        double* Xinv = dinv + (long)pb * DB * DB;
-        {
-            constexpr int PER = DB * DB / NTHREADS;
-            const int i = tid % DB, j0 = tid / DB;
-            TTAD_GLOBAL TS* Ac = gmem(A) + (p0 + i) + (long)p0 * lda;
-#pragma unroll
-            for (int q = 0; q < PER; q++) {
-                const int j = j0 + q * (NTHREADS / DB);
-                const double dv = D[i + j * DP], xv = X[i + j * DP];
-                if (i < pw && j < pw && i >= j) Ac[(long)j * lda] = (TS)dv;
-                gmem(Xinv)[i + j * DB] = xv;
-            }
-        }
-        __syncthreads();
-        // rows below: L(q, p) = A(q, p) Xinv^T
-        for (int r0 = DB; r0 < rows; r0 += POTRF_BM) {
-            const int mv = min(POTRF_BM, rows - r0);
-            TS* T = A + (p0 + r0) + (long)p0 * lda;
-            TTAD_GLOBAL TS* Tg = gmem(T);
-            G2::zero(acc);
-            G2::run(acc, T, lda, mv, Xinv, DB, pw, pw, lds);
-#pragma unroll
-            for (int a = 0; a < G::WM; a++)
-#pragma unroll
-                for (int b = 0; b < G::WN; b++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        const int rr = G::row_of(a, r), cc = G::col_of(b, r);
-                        if (rr < mv && cc < pw) Tg[rr + (long)cc * lda] = (TS)acc[a][b][r];
-                    }
-        }
-        __syncthreads();
-    }
-}
-
 // Waits until *count >= want and returns the value seen. The polls are relaxed (an acquire
 // load invalidates the L2 on every iteration, which with hundreds of waiting workgroups
 // evicts everyone's data); one agent-scope acquire follows. Gives up after `limit` ticks
@@ -1150,155 +1046,236 @@ __device__ __forceinline__ int wait_count(const int32_t* count, int want, int32_
 
 
 // ---------------------------------------------------------------------------
-// POTRF split into row-block items (used by the persistent executor): item rb of the
-// task owns rows [64 rb, 64 rb + 64) of the n x n tile and computes L(rb, 0..rb) by a
-// right-looking pass over the 64-column panels j < rb:
-//   L(rb,j)   = A(rb,j) Xinv(j)^T          once panel j is published
-//   A(rb,rb) -= L(rb,j) L(rb,j)^T          kept in registers
-//   A(rb,q)  -= L(rb,j) L(q,j)^T, j<q<rb  once L(q,j) is published
-// and then factors and inverts its diagonal block (lds_potrf_inv64) and publishes
-// Xinv(rb). prog[rb] counts the panels whose part of row block rb is final (rb + 1:
-// the whole row block, diagonal block and its inverse included). An item waits only on
-// lower-numbered items of its task, which are claimed before it, so every wait ends.
-// From one diagonal block to the next the chain is one 64^3 product, one 64^3 update
-// and the 64x64 factorization, where the single-workgroup item_potrf runs every panel
-// GEMM of the tile in sequence. Same arithmetic (FP64, operands rounded to the tile's
-// storage type as stored) and outputs (L in the tile, dinv) as item_potrf.
+// POTRF of an n x n diagonal tile as items of 64x64 blocks, nb = ceil(n / 64) block rows. Row r has r items (row 0
+// one): block items (r, q), q < r - 1, and last its tail item, which owns blocks (r, r-1) and (r, r). An item keeps its
+// blocks in registers and is left-looking:
+//   A(r,q) -= L(r,j) L(q,j)^T, j = 0 .. q-1, each product once both blocks are published
+//   L(r,q)  = A(r,q) X(q)^T once X(q) = L(q,q)^{-1} is published
+// and the tail item also A(r,r) -= L(r,j) L(r,j)^T, j = 0 .. r-1, then factors and inverts the diagonal block in LDS
+// and publishes X(r). Flag r (r + 1) / 2 + q says that L(r,q) (q < r) or X(r) (q = r) is final. Items are numbered row
+// by row, so an item waits on lower-numbered items of its task only; these are claimed before it, and every wait ends.
+// Why blocks and tails: the chain from X(r-1) to X(r) is one hand-over between workgroups, a triangular 64^3 product,
+// the lower half of a 64^3 update and the diagonal block (8.8 us); everything else of row r has nb - r such steps
+// to finish in. With one item per block row the last row's 35 products in series bounded a 512 tile (231 us).
+// Outputs: L in the tile, the inverses in dinv. FP64 throughout; L is rounded to the tile's type as it is stored.
 // ---------------------------------------------------------------------------
-constexpr int POTRF_FLAGS = 128;  // ints of progress flags per diagonal tile
-constexpr int POTRF_FIN = POTRF_FLAGS - 1;  // completion count (clears the flags for the next run)
-__host__ __device__ inline int potrf_row_items(int n) { return (n + DB - 1) / DB; }
+constexpr int BP = DB + 2;  // LDS pitch of a 64x64 operand block: Blk[k * BP + m] = element (m, k)
+constexpr int LDS_POTRF = 2 * DB * BP * 8;
+static_assert(DB * BP * 8 + DB * DP * 8 <= LDS_POTRF && (DB * DP + 1) * 8 <= DB * BP * 8, "D, X and its flag word fit");
+__host__ __device__ inline int potrf_blocks(int n) { return (n + DB - 1) / DB; }
+__host__ __device__ inline int potrf_items(int n) { return 1 + potrf_blocks(n) * (potrf_blocks(n) - 1) / 2; }
+// ints of flags per tile: one per block, and the count of finished items (the last one clears them for the next run)
+__host__ __device__ inline int potrf_flags(int n) { return potrf_blocks(n) * (potrf_blocks(n) + 1) / 2 + 1; }
 
-// Dst[k * P + m] = (double) T[m + k * ld] for m < rows, k < cols (else 0); 64 x 64, every
-// global load in flight before the first LDS store.
-template <typename TS, int P>
-__device__ __forceinline__ void stage64(double* Dst, const TTAD_GLOBAL TS* T, long ld, int rows, int cols) {
-    constexpr int PER = DB * DB / NTHREADS;
-    const int m = threadIdx.x % DB, k0 = threadIdx.x / DB;
-    TS v[PER];
+// acc[cb] += At (rows 16w .. 16w+15) Bt^T (columns 16cb .. 16cb+15) of 64x64 operands in LDS; TRI: Bt is lower
+// triangular (k <= column), its zero blocks are skipped. A lane's results: row 16w + l%16, columns 16cb + l/16 + 4r.
+template <bool TRI>
+__device__ __forceinline__ void mma64(d4_t (&acc)[4], const double* At, const double* Bt, int w) {
+    const int lane = threadIdx.x & 63;
+    const double* a0 = At + 16 * w + (lane & 15) + (lane >> 4) * BP;
+    const double* b0 = Bt + (lane & 15) + (lane >> 4) * BP;
 #pragma unroll
-    for (int q = 0; q < PER; q++) {
-        const int k = k0 + q * (NTHREADS / DB);
-        v[q] = (m < rows && k < cols) ? T[m + (long)k * ld] : TS(0);
+    for (int kb = 0; kb < 4; kb++)
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            const int k = 16 * kb + 4 * s;
+            const double a = a0[k * BP];
+#pragma unroll
+            for (int cb = TRI ? kb : 0; cb < 4; cb++)
+                acc[cb] = Mfma<double>::mma(b0[k * BP + 16 * cb], a, acc[cb]);
+        }
+}
+// The lower 16x16 blocks (I, J) of a 64x64 block, shared out over four waves: three each to waves 0 and 1, two to
+// waves 2 and 3. Nibble b of the code is I * 4 + J.
+struct LowerBlocks {
+    unsigned code;
+    int cnt;
+    __device__ __forceinline__ explicit LowerBlocks(int w)
+        : code(w == 0 ? 0x0dcu : w == 1 ? 0x5feu : w == 2 ? 0x98u : 0x4au), cnt(w < 2 ? 3 : 2) {}
+    __device__ __forceinline__ int I(int b) const { return (code >> (4 * b + 2)) & 3; }
+    __device__ __forceinline__ int J(int b) const { return (code >> (4 * b)) & 3; }
+};
+// acc[b] += At At^T in this wave's lower blocks (a lane's results as in mma64).
+__device__ __forceinline__ void mma64_lower(d4_t (&acc)[3], const double* At, const LowerBlocks& lb) {
+    const int lane = threadIdx.x & 63;
+    const double* a0 = At + (lane & 15) + (lane >> 4) * BP;
+#pragma unroll
+    for (int b = 0; b < 3; b++) {
+        if (b < lb.cnt) {
+            const double *pi = a0 + 16 * lb.I(b), *pj = a0 + 16 * lb.J(b);
+#pragma unroll
+            for (int ks = 0; ks < 16; ks++)
+                acc[b] = Mfma<double>::mma(pj[4 * ks * BP], pi[4 * ks * BP], acc[b]);
+        }
     }
-#pragma unroll
-    for (int q = 0; q < PER; q++) Dst[(k0 + q * (NTHREADS / DB)) * P + m] = (double)v[q];
 }
 
+// Two 64x64 blocks into LDS operand layout, every global load in flight before the first LDS store. Block P: element
+// (m, k) at P[m + k * ldp], rows beyond `prows` zero; block Q whole.
+template <typename TP, typename TQ>
+__device__ __forceinline__ void stage_pair(double* At, const TTAD_GLOBAL TP* P, long ldp, int prows, double* Bt,
+                                           const TTAD_GLOBAL TQ* Q, long ldq) {
+    constexpr int PER = DB * DB / NTHREADS, KS = NTHREADS / DB;
+    const int m = threadIdx.x % DB, k0 = threadIdx.x / DB;
+    TP v[PER];
+    TQ u[PER];
+#pragma unroll
+    for (int e = 0; e < PER; e++) {
+        v[e] = P[min(m, prows - 1) + (long)(k0 + e * KS) * ldp];
+        u[e] = Q[m + (long)(k0 + e * KS) * ldq];
+    }
+#pragma unroll
+    for (int e = 0; e < PER; e++) {
+        At[(k0 + e * KS) * BP + m] = m < prows ? (double)v[e] : 0.0;
+        Bt[(k0 + e * KS) * BP + m] = (double)u[e];
+    }
+}
+__device__ __forceinline__ void stage_inv(double* Bt, const TTAD_GLOBAL double* X) {
+    constexpr int PER = DB * DB / NTHREADS, KS = NTHREADS / DB;
+    const int m = threadIdx.x % DB, k0 = threadIdx.x / DB;
+    double u[PER];
+#pragma unroll
+    for (int e = 0; e < PER; e++) u[e] = X[m + (k0 + e * KS) * DB];
+#pragma unroll
+    for (int e = 0; e < PER; e++) Bt[(k0 + e * KS) * BP + m] = u[e];
+}
+// Every store of this wave has reached the L2 (vmcnt(0) expcnt(7) lgkmcnt(15); gfx9 counts stores in vmcnt).
+__device__ __forceinline__ void stores_done() { __builtin_amdgcn_s_waitcnt(0x0F70); }
+
 template <typename TS>
-__device__ __forceinline__ void item_potrf_rows(TS* __restrict__ A, long lda, int n, double* __restrict__ dinv,
-                                                int* info, int col_off, int rb, int32_t* prog, int32_t* err,
-                                                int64_t spin_limit, char* lds) {
-    using G3 = GemmNT<double, double, double, DB, DB, DB, false, true>;  // 64x64x64, both operands in LDS
-    using acc_t = typename G3::acc_t;
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, wr = w / G3::WC, wc = w % G3::WC;
-    const int nrb = potrf_row_items(n);
-    const int p0 = rb * DB, pw = min(DB, n - p0);
-    double* At = reinterpret_cast<double*>(lds);  // At[k * PA + m] = first operand (m, k)
-    double* Bt = At + DB * G3::PA;                // Bt[k * PB + c] = second operand (c, k)
+__device__ __forceinline__ void item_potrf(TS* __restrict__ A, long lda, int n, double* __restrict__ dinv, int* info,
+                                           int col_off, int it, int32_t* flags, int32_t* err, int64_t spin_limit,
+                                           char* lds) {
+    const int tid = threadIdx.x, lane = tid & 63, w = wave_uniform(tid >> 6);
+    const int nb = potrf_blocks(n);
+    int r = 0, rem = it;
+    while (rem >= max(1, r)) rem -= max(1, r++);
+    const bool tail = rem == max(1, r) - 1;
+    const int q = tail ? r - 1 : rem;  // this item's off-diagonal block is (r, q); row 0 has none
+    const int p0 = r * DB, pw = min(DB, n - p0);
+    auto flag = [&](int i, int j) { return flags + (i * (i + 1) / 2 + j); };
+    auto publish = [&](int i, int j) {
+        release_agent();
+        __hip_atomic_store(flag(i, j), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    double* At = reinterpret_cast<double*>(lds);
+    double* Bt = At + DB * BP;
     TTAD_GLOBAL TS* Ag = gmem(A);
-    TTAD_GLOBAL TS* Arow = Ag + p0;  // row block rb
-    acc_t accd[G3::WM][G3::WN], acc[G3::WM][G3::WN];
-    // accd = -A(rb, rb), lower part
+    TTAD_GLOBAL TS* Arow = Ag + p0;
+    const int lr = 16 * w + (lane & 15), lc = lane >> 4;  // this lane's row of the block, first column of a fragment
+    const LowerBlocks lb(w);
+    // A(r, q) and the lower part of A(r, r), loaded ahead of the first wait; the sums of products are formed from
+    // zero and subtracted once
+    d4_t av[4], ad[3], acc[4], accd[3];
 #pragma unroll
-    for (int a = 0; a < G3::WM; a++)
+    for (int cb = 0; cb < 4; cb++) av[cb] = acc[cb] = d4_t{0, 0, 0, 0};
 #pragma unroll
-        for (int b = 0; b < G3::WN; b++)
+    for (int b = 0; b < 3; b++) ad[b] = accd[b] = d4_t{0, 0, 0, 0};
+    if (r > 0) {
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int rr = G3::row_of(a, r), cc = G3::col_of(b, r);
-                accd[a][b][r] = (rr < pw && cc < pw && rr >= cc) ? -(double)Arow[rr + (long)(p0 + cc) * lda] : 0.0;
+        for (int cb = 0; cb < 4; cb++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const double v = (double)Arow[min(lr, pw - 1) + (long)(q * DB + 16 * cb + lc + 4 * e) * lda];
+                av[cb][e] = lr < pw ? v : 0.0;
             }
-    for (int j = 0; j < rb; j++) {
-        const int c0 = j * DB;  // panel j < rb is a full 64 columns
-        if (tid == 0) wait_count(prog + j, j + 1, err, spin_limit);
-        __syncthreads();  // Xinv(j) and L(j, 0..j) final; At / Bt free
-        stage64<TS, G3::PA>(At, Arow + (long)c0 * lda, lda, pw, DB);
-        stage64<double, G3::PB>(Bt, gmem(dinv) + (long)j * DB * DB, DB, DB, DB);
+    }
+    if (tail) {
+#pragma unroll
+        for (int b = 0; b < 3; b++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int rr = 16 * lb.I(b) + (lane & 15), cc = 16 * lb.J(b) + lc + 4 * e;
+                const double v = (double)Arow[min(rr, pw - 1) + (long)(p0 + min(cc, pw - 1)) * lda];
+                ad[b][e] = (rr < pw && cc < pw) ? v : (rr == cc ? 1.0 : 0.0);  // (identity padding)
+            }
+    }
+    for (int j = 0; j < q; j++) {
+        if (tid == 0) {
+            wait_count(flag(r, j), 1, err, spin_limit);
+            wait_count(flag(q, j), 1, err, spin_limit);
+        }
+        __syncthreads();  // both blocks are final; At / Bt are free
+        stage_pair(At, Arow + (long)j * DB * lda, lda, pw, Bt, Ag + q * DB + (long)j * DB * lda, lda);
         __syncthreads();
-        G3::zero(acc);
-        G3::compute(acc, At, lane, wr, wc);
+        mma64<false>(acc, At, Bt, w);
+        if (tail) mma64_lower(accd, At, lb);
+    }
+    if (r > 0) {
         __syncthreads();
-        // L(rb, j) into the tile and, as stored, into both operand buffers
 #pragma unroll
-        for (int a = 0; a < G3::WM; a++)
+        for (int cb = 0; cb < 4; cb++)
 #pragma unroll
-            for (int b = 0; b < G3::WN; b++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const int rr = G3::row_of(a, r), cc = G3::col_of(b, r);
-                    const TS v = (TS)acc[a][b][r];
-                    if (rr < pw) Arow[rr + (long)(c0 + cc) * lda] = v;
-                    At[cc * G3::PA + rr] = (double)v;
-                    Bt[cc * G3::PB + rr] = (double)v;
-                }
+            for (int e = 0; e < 4; e++) At[(16 * cb + lc + 4 * e) * BP + lr] = av[cb][e] - acc[cb][e];
+        if (tid == 0) wait_count(flag(q, q), 1, err, spin_limit);
         __syncthreads();
-        if (tid == 0) __hip_atomic_store(prog + rb, j + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-        G3::compute(accd, At, lane, wr, wc);  // -A(rb,rb) + L(rb,j) L(rb,j)^T
-        // blocks of this row to the right of panel j: A(rb,q) -= L(rb,j) L(q,j)^T
-        for (int q = j + 1; q < rb; q++) {
-            if (tid == 0) wait_count(prog + q, j + 1, err, spin_limit);
-            __syncthreads();  // L(q, j) final; Bt free
-            stage64<TS, G3::PB>(Bt, Ag + q * DB + (long)c0 * lda, lda, DB, DB);
-            TTAD_GLOBAL TS* C = Arow + (long)q * DB * lda;
+        stage_inv(Bt, gmem(dinv) + (long)q * DB * DB);
+        __syncthreads();
 #pragma unroll
-            for (int a = 0; a < G3::WM; a++)
+        for (int cb = 0; cb < 4; cb++) acc[cb] = d4_t{0, 0, 0, 0};
+        mma64<true>(acc, At, Bt, w);
+        __syncthreads();
+        // L(r, q) into the tile and, as stored, into LDS for the diagonal block's update
 #pragma unroll
-                for (int b = 0; b < G3::WN; b++)
+        for (int cb = 0; cb < 4; cb++)
 #pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        const int rr = G3::row_of(a, r), cc = G3::col_of(b, r);
-                        acc[a][b][r] = rr < pw ? -(double)C[rr + (long)cc * lda] : 0.0;
-                    }
+            for (int e = 0; e < 4; e++) {
+                const int cc = 16 * cb + lc + 4 * e;
+                const TS v = (TS)acc[cb][e];
+                if (lr < pw) Arow[lr + (long)(q * DB + cc) * lda] = v;
+                At[cc * BP + lr] = (double)v;
+            }
+        if (tail) {
             __syncthreads();
-            G3::compute(acc, At, lane, wr, wc);
-#pragma unroll
-            for (int a = 0; a < G3::WM; a++)
-#pragma unroll
-                for (int b = 0; b < G3::WN; b++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        const int rr = G3::row_of(a, r), cc = G3::col_of(b, r);
-                        if (rr < pw) C[rr + (long)cc * lda] = (TS)(-acc[a][b][r]);
-                    }
+            mma64_lower(accd, At, lb);
+        }
+        stores_done();
+        if (!tail) {
+            __syncthreads();
+            if (tid == 0) publish(r, q);
         }
     }
-    // diagonal block (identity padding): factor and invert in LDS
-    double* D = At;
-    double* X = D + DB * DP;
-    __syncthreads();
+    if (tail) {
+        double *D = Bt, *X = At;
 #pragma unroll
-    for (int a = 0; a < G3::WM; a++)
+        for (int b = 0; b < 3; b++)
+            if (b < lb.cnt) {
 #pragma unroll
-        for (int b = 0; b < G3::WN; b++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int rr = G3::row_of(a, r), cc = G3::col_of(b, r);
-                D[rr + cc * DP] = (rr < pw && cc < pw) ? (rr >= cc ? -accd[a][b][r] : 0.0) : (rr == cc ? 1.0 : 0.0);
+                for (int e = 0; e < 4; e++) {
+                    const int rr = 16 * lb.I(b) + (lane & 15), cc = 16 * lb.J(b) + lc + 4 * e;
+                    D[rr + cc * DP] = ad[b][e] - accd[b][e];
+                }
             }
-    __syncthreads();
-    const int bad = lds_potrf_inv64(D, X, pw);
-    if (bad && tid == 0) atomicCAS(info, 0, col_off + p0 + bad);
-    {
+        __syncthreads();
+        const int bad = lds_potrf_inv64(D, X, pw, [&] {
+            if (r > 0 && lane == 0) publish(r, q);  // its write-back runs beside the first panel
+        });
         constexpr int PER = DB * DB / NTHREADS;
         const int i = tid % DB, j0 = tid / DB;
-        TTAD_GLOBAL double* Xg = gmem(dinv) + (long)rb * DB * DB;
+        TTAD_GLOBAL double* Xg = gmem(dinv) + (long)r * DB * DB;
 #pragma unroll
-        for (int q = 0; q < PER; q++) {
-            const int j = j0 + q * (NTHREADS / DB);
-            const double dv = D[i + j * DP], xv = X[i + j * DP];
-            if (i < pw && j < pw && i >= j) Arow[i + (long)(p0 + j) * lda] = (TS)dv;
-            Xg[i + j * DB] = xv;
+        for (int e = 0; e < PER; e++) {
+            const int j = j0 + e * (NTHREADS / DB);
+            Xg[i + j * DB] = X[i + j * DP];
+        }
+        stores_done();
+        __syncthreads();
+        if (tid == 0) {
+            publish(r, r);
+            if (bad) atomicCAS(info, 0, col_off + p0 + bad);
+        }
+#pragma unroll
+        for (int e = 0; e < PER; e++) {
+            const int j = j0 + e * (NTHREADS / DB);
+            if (i < pw && j < pw && i >= j) Arow[i + (long)(p0 + j) * lda] = (TS)D[i + j * DP];
         }
     }
-    __syncthreads();
     if (tid == 0) {
-        __hip_atomic_store(prog + rb, rb + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
         // the last item of the task to finish clears the flags for the next run on this tile
-        if (__hip_atomic_fetch_add(prog + POTRF_FIN, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == nrb - 1) {
-            for (int i = 0; i < nrb; i++) __hip_atomic_store(prog + i, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(prog + POTRF_FIN, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
+        int32_t* fin = flags + nb * (nb + 1) / 2;
+        if (__hip_atomic_fetch_add(fin, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == potrf_items(n) - 1)
+            for (int e = 0; e <= nb * (nb + 1) / 2; e++)
+                __hip_atomic_store(flags + e, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 
@@ -1404,13 +1381,11 @@ constexpr int LDS_GEMM_BF16_1 = GemmNTbf16<float, GEMM_BM, GEMM_BM, false, true>
 template <typename TS, int PREC> constexpr int gemm_item_lds() {
     return PREC == P_BF16X3 ? LDS_GEMM_BF16 : PREC == P_BF16 ? LDS_GEMM_BF16_1 : sizeof(TS) == 8 ? LDS_GEMM_F64 : LDS_GEMM_F32;
 }
-constexpr int LDS_POTRF = cmax(PotrfGemm<double>::G::LDS_BYTES, POTRF_LDS);
-constexpr int LDS_POTRF_ROWS = cmax(GemmNT<double, double, double, DB, DB, DB, false, true>::STAGE * 8, POTRF_LDS);
 constexpr int LDS_TRSM = cmax(GemmNT<double, double, double, TRSM_BM, DB, 32, true, true>::LDS_BYTES,
                               GemmNT<double, double, double, TRSM_BM, DB, DB, false, true>::STAGE * 8);
 constexpr int LDS_TRSM_F32 = cmax(GemmNT<float, float, float, TRSM_BM_F32, DB, trsm_bk<float>(), true, true>::LDS_BYTES,
                                   GemmNT<float, float, float, TRSM_BM_F32, DB, DB, false, true>::STAGE * 4);
 constexpr int LDS_ITEM_MAX =
-    cmax(cmax(cmax(LDS_GEMM_F64, LDS_GEMM_F32), cmax(LDS_GEMM_BF16, LDS_POTRF)), cmax(LDS_TRSM, LDS_POTRF_ROWS));
+    cmax(cmax(cmax(LDS_GEMM_F64, LDS_GEMM_F32), cmax(LDS_GEMM_BF16, LDS_POTRF)), LDS_TRSM);
 
 }  // namespace ttad

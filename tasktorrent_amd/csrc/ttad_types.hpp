@@ -27,7 +27,8 @@ struct DevMat {
     void* const* tiles;    // [nt*nt], entry i + j*nt
     double* const* dinv;   // [nt]: inverses of the 64x64 diagonal blocks of L_jj (FP64, 64x64 each, ld 64)
     int32_t* info;         // first non-positive pivot, 1-based global column; 0 = none
-    int32_t* pflags;       // [nt * 128]: progress flags of the row-block POTRF items of each diagonal tile (zero between runs)
+    int32_t* pflags;       // [nt * pf_stride]: flags of the POTRF items of each diagonal tile (zero between runs)
+    int32_t pf_stride;     // ints per tile: potrf_flags of the largest tile
     int32_t* locks;        // [nt * nt * 16]: accumulate-mode sub-tile locks of tile (i, j) (zero when free)
     // [nt*nt] or null: bf16 hi/lo planes of the off-diagonal FP32 tiles (i > j, bsz[j] % 32 == 0; other
     // entries null), written by the TRSM items that produce the tile and read by the bf16x3 GEMM items.

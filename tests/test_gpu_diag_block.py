@@ -36,3 +36,22 @@ def test_bad_pivot_column(ctx, oracle, col):
     ref = A.copy(order="F")
     info = ctx.potrf(to_dev(A), n, n)
     assert info == oracle.dpotrf(ref) == col + 1
+
+
+@pytest.mark.parametrize("n", [255, 256, 257, 320, 449, 513, 1030])
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+def test_potrf_block_items(ctx, oracle, n, dtype):
+    # tiles of several 64-row blocks with a ragged last one, leading dimension above n, twice on the same flags
+    import torch
+    A = oracle.spd_bbt(n, 40 + n)
+    ref = A.copy(order="F")
+    assert oracle.dpotrf(ref) == 0
+    ld = n + 3
+    for _ in range(2):
+        buf = torch.zeros((n, ld), dtype=torch.float64)
+        buf[:, :n] = torch.from_numpy(np.ascontiguousarray(A.T))
+        d = buf.to(torch.float32 if dtype == "f32" else torch.float64).cuda()
+        assert ctx.potrf(d, n, ld) == 0
+        out = from_dev(d)[:n]
+        assert rel(np.tril(out), np.tril(ref)) < (2e-6 if dtype == "f32" else 1e-13)
+        assert np.array_equal(np.triu(out, 1), np.triu(A.astype(np.float32) if dtype == "f32" else A, 1))
