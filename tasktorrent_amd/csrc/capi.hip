@@ -772,10 +772,18 @@ static int graph_prepare(ttad_graph* g) {
                 dm[s] = g->mats[s]->host_desc;
                 if (g->with_planes && g->mats[s]->tab_planes.p) dm[s].planes = g->mats[s]->tab_planes.as<void*>();
             }
-        const int ne = std::max(1, g->out_ptr[n]);
+        const size_t ne = std::max(1, g->out_ptr[n]);
+        std::vector<DevEdge> edges(ne);
+        for (int t = 0; t < n; t++) {
+            g->tasks[t].edge_off = g->out_ptr[t];
+            g->tasks[t].edge_cnt = g->out_ptr[t + 1] - g->out_ptr[t];
+            for (int e = g->out_ptr[t]; e < g->out_ptr[t + 1]; e++) {
+                const DevTask& x = g->tasks[g->out_idx[e]];
+                edges[e] = DevEdge{g->out_idx[e], x.n_items, x.bucket, g->q_base[x.bucket], g->bucket_items[x.bucket], {}};
+            }
+        }
         TTAD_HIP(g->d_tasks.alloc(n * sizeof(DevTask)));
-        TTAD_HIP(g->d_out_ptr.alloc((n + 1) * 4));
-        TTAD_HIP(g->d_out_idx.alloc(ne * 4));
+        TTAD_HIP(g->d_edges.alloc(ne * sizeof(DevEdge)));
         TTAD_HIP(g->d_deps0.alloc(n * 4));
         TTAD_HIP(g->d_deps.alloc(n * 4));
         TTAD_HIP(g->d_items_left.alloc(n * 4));
@@ -794,9 +802,7 @@ static int graph_prepare(ttad_graph* g) {
         TTAD_HIP(g->d_cu_slots.alloc((2 * CU_KEYS + NXCD * 64) * 4));  // slots, critical counts, idle primaries
         TTAD_HIP(g->d_mats.alloc(dm.size() * sizeof(DevMat)));
         TTAD_HIP(hipMemcpy(g->d_tasks.p, g->tasks.data(), n * sizeof(DevTask), hipMemcpyHostToDevice));
-        TTAD_HIP(hipMemcpy(g->d_out_ptr.p, g->out_ptr.data(), (n + 1) * 4, hipMemcpyHostToDevice));
-        if (!g->out_idx.empty())
-            TTAD_HIP(hipMemcpy(g->d_out_idx.p, g->out_idx.data(), g->out_idx.size() * 4, hipMemcpyHostToDevice));
+        TTAD_HIP(hipMemcpy(g->d_edges.p, edges.data(), ne * sizeof(DevEdge), hipMemcpyHostToDevice));
         TTAD_HIP(hipMemcpy(g->d_q_base.p, g->q_base.data(), (g->n_buckets + 1) * 4, hipMemcpyHostToDevice));
         TTAD_HIP(hipMemcpy(g->d_q_home.p, g->q_home.data(), g->n_buckets * 4, hipMemcpyHostToDevice));
         TTAD_HIP(hipMemcpy(g->d_mats.p, dm.data(), dm.size() * sizeof(DevMat), hipMemcpyHostToDevice));
@@ -844,8 +850,7 @@ static DevGraph graph_image(ttad_graph* g, bool trace, int64_t spin_limit) {
     d.total_items = g->total_items;
     d.n_init = g->n_init;
     d.tasks = g->d_tasks.as<DevTask>();
-    d.out_ptr = g->d_out_ptr.as<int32_t>();
-    d.out_idx = g->d_out_idx.as<int32_t>();
+    d.edges = g->d_edges.as<DevEdge>();
     d.deps0 = g->d_deps0.as<int32_t>();
     d.tail0 = g->d_tail0.as<int32_t>();
     d.init_items = g->d_init.as<int64_t>();

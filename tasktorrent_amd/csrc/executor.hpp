@@ -26,8 +26,7 @@ struct DevGraph {
     int32_t total_items;
     int32_t n_init;             // number of initially ready entries (prefilled queue slots)
     const DevTask* tasks;
-    const int32_t* out_ptr;     // CSR successors
-    const int32_t* out_idx;
+    const DevEdge* edges;       // out-edges, by task
     const int32_t* deps0;       // initial dependency counters (indegree - host seeds)
     const int32_t* tail0;       // initial queue tails per bucket
     const int64_t* init_items;  // [n_init] queue entries (task << 20) | item of the prefilled slots
@@ -72,6 +71,8 @@ constexpr int MAX_QUEUES = QUEUE_HOMED + QUEUE_BUCKETS * NXCD;
 __host__ __device__ constexpr int shared_queue(int b) { return b * QUEUE_SHARED_STRIDE; }
 __host__ __device__ constexpr int homed_queue(int x, int b) { return QUEUE_HOMED + x * QUEUE_BUCKETS + b; }
 constexpr int CLAIM_TRIES = 4;  // queues a claimer tries from one scan
+constexpr int IDLE_PRIMARIES = 8;  // idle primaries of an XCD (32 CUs) from which on its secondaries hold back
+constexpr int IDLE_BACKOFF = 10;  // log2 of the longest pause between the looks of an idle worker, x 64 cycles
 // Hardware id of the XCD (XCC) this wave runs on.
 __device__ __forceinline__ int xcc_id() {
     unsigned v;

@@ -43,25 +43,23 @@ __global__ __launch_bounds__(NTHREADS, vset_occupancy(VM)) void k_items(const De
 //   The workgroup runs that work item, then thread 0 decrements the
 //   task's remaining-items counter; the last item of a task decrements its
 //   successors' dependency counters and pushes every item of a successor that
-//   reaches zero into its queue. A worker exits when every queue is fully claimed.
+//   reaches zero into its queue. A worker exits when every item is done.
 // Memory ordering: item outputs are released (agent scope) before the counter
 // RMWs; queue entries are published with release stores and read with acquire
 // loads, so a consumer on another XCD sees the producer's tiles.
 // The loop also ends when the abort flag is raised (watchdog: no work found for
 // spin_limit ticks; queue overflow; an item variant missing from this instantiation).
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void push_task(const DevGraph& g, int s) {
-    const DevTask t = g.tasks[s];
+__device__ __forceinline__ void push_task(const DevGraph& g, const DevEdge& t) {
     const int b = t.bucket;
     const int pos = __hip_atomic_fetch_add(g.q_tail + b, t.n_items, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const int cap = g.q_base[b + 1] - g.q_base[b];
-    if (pos + t.n_items > cap) {
+    if (pos + t.n_items > t.cap) {
         __hip_atomic_store(g.abort_flag, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return;
     }
     // the caller's release fence orders these entries after the outputs they announce
     for (int r = 0; r < t.n_items; r++)
-        __hip_atomic_store(g.q_items + g.q_base[b] + pos + r, ((int64_t)s << 20) | r, __ATOMIC_RELAXED,
+        __hip_atomic_store(g.q_items + t.base + pos + r, ((int64_t)t.succ << 20) | r, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
     // claim credits (a claimer that gets a slot whose entry is not written yet polls it)
     __hip_atomic_fetch_add(g.q_count + b, t.n_items, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -96,71 +94,62 @@ __global__ __launch_bounds__(NTHREADS, vset_occupancy(VM)) void k_persistent(Dev
             // this XCD. Each scan reads the two (their counters lie in 256-byte blocks that only the workers
             // of one XCD hammer) in one memory round trip; the other XCDs' queues only when both are empty.
             int64_t got = -1;
+            int idle_scans = 0;
             const int64_t t_start = (int64_t)wall_clock64();
             for (;;) {
                 int cand[CLAIM_TRIES];  // queues to try, best first
                 int nc = 0;
-                bool any_open = false;
-                // a secondary leaves queues that the idle primaries can drain; nothing is taken while
-                // the other worker of this CU runs an item of the critical path
-                // the lane index, opaque to the compiler here: addresses derived from it are formed per scan
-                // instead of being hoisted out of the worker loop, where they would hold registers through
-                // every item
-                int lane = tid;
-                asm volatile("" : "+v"(lane));
-                // (idle primaries of this XCD for its own queues, of all XCDs for shared queues and stealing)
-                int idle[NXCD];
-#pragma unroll
-                for (int x = 0; x < NXCD; x++) idle[x] = primary ? 0 : ld_relaxed(g.idle_primary + x * 64);
-                const bool blocked = ld_relaxed(g.cu_crit + my_key) != 0;
-                const int cs = ld_relaxed(g.q_count + shared_queue(lane)), co = ld_relaxed(g.q_count + own_q + lane);
                 int reserve_all = 0, reserve_own = 0;
+                // A secondary does not even scan while a quarter of its XCD's primaries look for work. (From the
+                // first idle primary on, bf16x3 factorization n = 32768: 66.8 ms, since an idle primary may be held back
+                // by a critical item of its CU; from 8 on 57.1, from 16 on 57.2; n = 16384: 10.1, 10.9, 11.2 ms.)
+                if (primary || ld_relaxed(idle_primary) < IDLE_PRIMARIES) {
+                    // a secondary leaves queues that the idle primaries can drain; nothing is taken while
+                    // the other worker of this CU runs an item of the critical path
+                    // the lane index, opaque to the compiler here: addresses derived from it are formed per scan
+                    // instead of being hoisted out of the worker loop, where they would hold registers through
+                    // every item
+                    int lane = tid;
+                    asm volatile("" : "+v"(lane));
+                    // (idle primaries of this XCD for its own queues, of all XCDs for shared queues and stealing)
+                    int idle[NXCD];
 #pragma unroll
-                for (int x = 0; x < NXCD; x++) {
-                    reserve_all += idle[x];
-                    if (x == my_xcd) reserve_own = idle[x];
-                }
-                const unsigned long long ms = __ballot(!blocked && cs > reserve_all);
-                const unsigned long long mo = __ballot(!blocked && co > reserve_own);
-                // within a bucket the shared queue (POTRF, TRSM, FP64 updates) comes first
-                for (unsigned long long m = ms | mo; m != 0 && nc < CLAIM_TRIES; m &= m - 1) {
-                    const int b = __ffsll((long long)m) - 1;
-                    if ((ms >> b) & 1) cand[nc++] = shared_queue(b);
-                    if (nc < CLAIM_TRIES && ((mo >> b) & 1)) cand[nc++] = own_q + b;
-                }
-                if (nc == 0 && !blocked) {  // nothing on this XCD: steal from the best bucket of another one
-                    int cx[NXCD];
-#pragma unroll
-                    for (int x = 0; x < NXCD; x++) cx[x] = ld_relaxed(g.q_count + homed_queue(x, lane));
-                    unsigned long long mx[NXCD], any = 0;
+                    for (int x = 0; x < NXCD; x++) idle[x] = primary ? 0 : ld_relaxed(g.idle_primary + x * 64);
+                    const bool blocked = ld_relaxed(g.cu_crit + my_key) != 0;
+                    const int cs = ld_relaxed(g.q_count + shared_queue(lane)), co = ld_relaxed(g.q_count + own_q + lane);
 #pragma unroll
                     for (int x = 0; x < NXCD; x++) {
-                        mx[x] = x == my_xcd ? 0ull : __ballot(cx[x] > reserve_all);
-                        any |= mx[x];
+                        reserve_all += idle[x];
+                        if (x == my_xcd) reserve_own = idle[x];
                     }
-                    if (any) {
-                        const int b = __ffsll((long long)any) - 1;
+                    const unsigned long long ms = __ballot(!blocked && cs > reserve_all);
+                    const unsigned long long mo = __ballot(!blocked && co > reserve_own);
+                    // within a bucket the shared queue (POTRF, TRSM, FP64 updates) comes first
+                    for (unsigned long long m = ms | mo; m != 0 && nc < CLAIM_TRIES; m &= m - 1) {
+                        const int b = __ffsll((long long)m) - 1;
+                        if ((ms >> b) & 1) cand[nc++] = shared_queue(b);
+                        if (nc < CLAIM_TRIES && ((mo >> b) & 1)) cand[nc++] = own_q + b;
+                    }
+                    if (nc == 0 && !blocked) {  // nothing on this XCD: steal from the best bucket of another one
+                        int cx[NXCD];
 #pragma unroll
-                        for (int d = 1; d < NXCD; d++) {  // from the next XCD on, so that stealers spread
-                            const int x = (my_xcd + d) % NXCD;
-                            if (nc < CLAIM_TRIES && ((mx[x] >> b) & 1)) cand[nc++] = homed_queue(x, b);
+                        for (int x = 0; x < NXCD; x++) cx[x] = ld_relaxed(g.q_count + homed_queue(x, lane));
+                        unsigned long long mx[NXCD], any = 0;
+#pragma unroll
+                        for (int x = 0; x < NXCD; x++) {
+                            mx[x] = x == my_xcd ? 0ull : __ballot(cx[x] > reserve_all);
+                            any |= mx[x];
+                        }
+                        if (any) {
+                            const int b = __ffsll((long long)any) - 1;
+#pragma unroll
+                            for (int d = 1; d < NXCD; d++) {  // from the next XCD on, so that stealers spread
+                                const int x = (my_xcd + d) % NXCD;
+                                if (nc < CLAIM_TRIES && ((mx[x] >> b) & 1)) cand[nc++] = homed_queue(x, b);
+                            }
                         }
                     }
                 }
-                if (nc == 0) {  // nothing claimable: is anything left to claim at all?
-                    int qs[NXCD + 1], hs[NXCD + 1];  // this lane's bucket: the shared queue, the homed ones
-#pragma unroll
-                    for (int x = 0; x <= NXCD; x++) {
-                        const int q = x == NXCD ? shared_queue(lane) : homed_queue(x, lane);
-                        hs[x] = ld_relaxed(g.q_head + q);
-                        qs[x] = g.q_base[q + 1] - g.q_base[q];
-                    }
-                    bool open = false;
-#pragma unroll
-                    for (int x = 0; x <= NXCD; x++) open |= hs[x] < qs[x];
-                    any_open = __ballot(open) != 0;
-                }
-                const bool all_claimed = nc == 0 && !any_open;
                 if (nc > 0) {
                     int64_t e = -1;
                     if (tid == 0) {
@@ -204,7 +193,8 @@ __global__ __launch_bounds__(NTHREADS, vset_occupancy(VM)) void k_persistent(Dev
                     for (uint32_t q = rng >> 28; q > 0; q--) __builtin_amdgcn_s_sleep(1);
                     continue;
                 }
-                if (all_claimed || ld_relaxed(g.abort_flag) != 0) {  // every item is taken: this worker is done
+                // every item done (or the run stopped): this worker is done
+                if (ld_relaxed(g.done_items) == g.total_items || ld_relaxed(g.abort_flag) != 0) {
                     got = -2;
                     break;
                 }
@@ -213,7 +203,14 @@ __global__ __launch_bounds__(NTHREADS, vset_occupancy(VM)) void k_persistent(Dev
                     got = -2;
                     break;
                 }
-                __builtin_amdgcn_s_sleep(2);
+                // Idle workers look less often the longer they find nothing (a random 0 .. 2^k - 1 units of 64 cycles,
+                // k up to IDLE_BACKOFF): with hundreds of them idle the next item still meets a scanner within
+                // a fraction of a microsecond, and their loads no longer slow the claims and counters of the few
+                // workers on the critical path. Pauses of up to 2^2 / 2^8 / 2^10 units, bf16x3 factorization n = 16384:
+                // 12.1 / 10.4 / 10.2 ms; FP64 n = 2048 b = 256: 1.50 / 1.34 / 1.28 ms.
+                idle_scans = min(idle_scans + 1, IDLE_BACKOFF);
+                rng = rng * 1664525u + 1013904223u;
+                for (uint32_t q = rng >> (32 - idle_scans); q > 0; q--) __builtin_amdgcn_s_sleep(1);
             }
             if (tid == 0) {
                 s_item = got;
@@ -243,52 +240,64 @@ __global__ __launch_bounds__(NTHREADS, vset_occupancy(VM)) void k_persistent(Dev
         // below is issued only once all of this item's outputs sit in this XCD's L2.
         __builtin_amdgcn_s_waitcnt(0x0F70);
         __syncthreads();
-        if (tid == 0) {
-            // Release elision: an agent-scope release (buffer_wbl2) writes back every dirty line of this
-            // XCD's L2, so the item that leaves no other item of its task running on this XCD releases for
-            // all of them; the others skip it. This relies on the hardware, not on the memory model: an
-            // item's stores reached the L2 before its relaxed decrement was issued (the wait above), the
-            // decrements of one counter are serialized at the L2, and the last one's write-back is issued
-            // after its decrement returned, so it covers every earlier item's lines. Each item decrements
-            // the task's remaining count after that, so the count reaches zero only after every XCD that
-            // ran items of the task has released.
-            if (__hip_atomic_fetch_add(g.xcd_run + (long)task * NXCD + my_xcd, -1, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT) == 1)
-                release_agent();
-            if (!ran) __hip_atomic_store(g.abort_flag, 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const uint64_t t1 = g.trace ? wall_clock64() : 0;
-            // Counters are relaxed: the release above has written this item's outputs back before the decrement.
-            // The thread that takes a counter to zero acquires what the other decrements released; it has nothing
-            // of its own left to write back, so its next counter update and queue entries need no release.
-            const int left =
-                __hip_atomic_fetch_add(g.items_left + task, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - 1;
-            if (left == 0) {  // last item of the task: release its successors
+        if (tid < 64) {
+            int left = 0;
+            uint64_t t1 = 0;
+            // this lane's out-edge, on its way while the counters below are updated
+            DevEdge ed{};
+            if (tid < t.edge_cnt) ed = g.edges[t.edge_off + tid];
+            if (tid == 0) {
+                // Release elision: an agent-scope release (buffer_wbl2) writes back every dirty line of this
+                // XCD's L2, so the item that leaves no other item of its task running on this XCD releases for
+                // all of them; the others skip it. This relies on the hardware, not on the memory model: an
+                // item's stores reached the L2 before its relaxed decrement was issued (the wait above), the
+                // decrements of one counter are serialized at the L2, and the last one's write-back is issued
+                // after its decrement returned, so it covers every earlier item's lines. Each item decrements
+                // the task's remaining count after that, so the count reaches zero only after every XCD that
+                // ran items of the task has released.
+                if (__hip_atomic_fetch_add(g.xcd_run + (long)task * NXCD + my_xcd, -1, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT) == 1)
+                    release_agent();
+                if (!ran) __hip_atomic_store(g.abort_flag, 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (g.trace) t1 = wall_clock64();
+                // Counters are relaxed: the release above has written this item's outputs back before the decrement.
+                // The wave that takes a counter to zero acquires what the other decrements released; it has nothing
+                // of its own left to write back, so its next counter update and queue entries need no release.
+                left = __hip_atomic_fetch_add(g.items_left + task, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - 1;
+            }
+            left = __builtin_amdgcn_readfirstlane(left);
+            if (left == 0) {
+                // last item of the task: release its successors, one per lane (a task of an n-tile column has up to n
+                // of them; each costs two dependent memory round trips, its counter and its queue's tail).
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-                for (int q = g.out_ptr[task]; q < g.out_ptr[task + 1]; q++) {
-                    const int s = g.out_idx[q];
+                for (int q = tid; q < t.edge_cnt; q += 64) {
+                    if (q >= 64) ed = g.edges[t.edge_off + q];
                     const int d =
-                        __hip_atomic_fetch_add(g.deps + s, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - 1;
+                        __hip_atomic_fetch_add(g.deps + ed.succ, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - 1;
                     if (d == 0) {
                         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-                        push_task(g, s);
+                        push_task(g, ed);
                     }
                 }
-                __hip_atomic_fetch_add(g.done_items, t.n_items, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (tid == 0) __hip_atomic_fetch_add(g.done_items, t.n_items, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
-            if (g.trace) {  // {entry, workgroup, start, end, end of the successor release (last item only), 0}
-                const int slot = __hip_atomic_fetch_add(g.trace_cursor, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (slot < g.total_items) {
-                    uint64_t* rec = g.trace + TRACE_WORDS * (long)slot;
-                    rec[0] = (uint64_t)e;
-                    rec[1] = blockIdx.x;
-                    rec[2] = t0;
-                    rec[3] = t1;
-                    rec[4] = left == 0 ? wall_clock64() : 0;
-                    rec[5] = 0;
+            if (tid == 0) {
+                if (g.trace) {  // {entry, workgroup, start, end, end of the successor release (last item only), 0}
+                    const int slot =
+                        __hip_atomic_fetch_add(g.trace_cursor, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if (slot < g.total_items) {
+                        uint64_t* rec = g.trace + TRACE_WORDS * (long)slot;
+                        rec[0] = (uint64_t)e;
+                        rec[1] = blockIdx.x;
+                        rec[2] = t0;
+                        rec[3] = t1;
+                        rec[4] = left == 0 ? wall_clock64() : 0;
+                        rec[5] = 0;
+                    }
                 }
+                if (primary) __hip_atomic_fetch_add(idle_primary, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (t.crit) __hip_atomic_fetch_add(g.cu_crit + my_key, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
-            if (primary) __hip_atomic_fetch_add(idle_primary, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (t.crit) __hip_atomic_fetch_add(g.cu_crit + my_key, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
 }

@@ -51,6 +51,18 @@ struct DevTask {
     int32_t bucket;
     int32_t crit;  // on a longest path of the DAG: runs with no other item started on its CU
     int32_t accum; // GEMM/SYRK: add the product into C under the sub-tile lock (accumulate mode)
+    int32_t edge_off, edge_cnt;  // its out-edges in DevGraph::edges
+};
+
+// An out-edge of the graph with all that releasing its target takes: the task that completes reads it in one access
+// instead of the target's id, record and queue bounds in turn.
+struct alignas(16) DevEdge {
+    int32_t succ;     // target task
+    int32_t n_items;  // its work items
+    int32_t bucket;   // its queue
+    int32_t base;     // first slot of that queue in q_items
+    int32_t cap;      // slots of that queue
+    int32_t pad[3];
 };
 
 // Work items per task of tiles with elem_bytes-byte elements; host and device must agree.
