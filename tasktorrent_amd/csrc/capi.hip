@@ -72,6 +72,7 @@ static std::shared_ptr<StreamPlan> build_stream_plan(ttad_matrix* M, int prec, i
                                     : std::max(1, items_of(kind, M->bsz[i], M->bsz[j], (int)M->elem));
         t.bucket = 0;
         t.crit = 0;
+        t.sub = GEMM_BM;
         return t;
     };
     for (int k = 0; k < nt; k++) {
@@ -729,6 +730,24 @@ static int graph_prepare(ttad_graph* g) {
     if (g->mats_dirty) {
         int rate_khz = 100000;
         (void)hipDeviceGetAttribute(&rate_khz, hipDeviceAttributeWallClockRate, g->ctx->device);
+        // 128x128 items that the updates of step k of a matrix would have: a step that cannot give every other CU one has
+        // 64x64 items, and so has every update on a longest path (its latency counts, not its throughput). Up to half
+        // an item per CU / one / two, FP64 n = 4096 b = 256: 2.20 / 2.25 / 2.34 ms (none 2.75, no longest path 2.35). Accumulate-
+        // mode updates keep 128 (their locks are per 128x128 sub-tile).
+        std::map<std::pair<int, int>, long long> step_items;
+        auto update_items = [&](const DevTask& x, int sub) {
+            ttad_matrix* M = x.mat < (int)g->mats.size() ? g->mats[x.mat] : nullptr;
+            const bool in = M && x.i >= 0 && x.j >= 0 && x.i < M->nt && x.j < M->nt;
+            return in ? items_of(x.kind, M->bsz[x.i], M->bsz[x.j], (int)M->elem, sub) : 0;
+        };
+        for (auto& x : g->tasks)
+            if (x.kind == K_GEMM || x.kind == K_SYRK) step_items[{x.mat, x.k}] += update_items(x, GEMM_BM);
+        for (auto& x : g->tasks) {
+            x.sub = GEMM_BM;
+            if ((x.kind == K_GEMM || x.kind == K_SYRK) && !x.accum &&
+                (x.crit || 2 * step_items[{x.mat, x.k}] <= g->ctx->n_cu))
+                x.sub = GEMM_BS;
+        }
         for (int t = 0; t < n; t++) {
             DevTask& x = g->tasks[t];
             if (x.kind == K_NOP) {  // spin task: k microseconds, stored as device clock ticks
@@ -746,7 +765,7 @@ static int graph_prepare(ttad_graph* g) {
             if ((x.kind == K_GEMM || x.kind == K_SYRK) && ((x.prec == P_F64) != (M->storage == P_F64)))
                 return set_error(TTAD_ERR_INVALID, "graph: task %d precision does not match tile storage", t);
             x.n_items = x.kind == K_POTRF ? potrf_items(M->bsz[x.j])
-                                          : std::max(1, items_of(x.kind, M->bsz[x.i], M->bsz[x.j], (int)M->elem));
+                                          : std::max(1, items_of(x.kind, M->bsz[x.i], M->bsz[x.j], (int)M->elem, x.sub));
         }
         int needed = 0;
         for (auto& x : g->tasks)

@@ -125,6 +125,8 @@ __host__ __device__ inline int item_variant(int kind, int prec, int storage) {
 constexpr int vset_lds(int vm) {
     int b = 0;
     if (vm & V_F64S) b = cmax(b, cmax(cmax(LDS_GEMM_F64, LDS_POTRF), LDS_TRSM));
+    if (vm & V_F64S) b = cmax(b, gemm_item_lds<double, P_F64, GEMM_BS>());
+    if (vm & V_G32) b = cmax(b, gemm_item_lds<float, P_F32, GEMM_BS>());
     if (vm & V_F32S) b = cmax(b, cmax(LDS_POTRF, LDS_TRSM_F32));
     if (vm & V_G32) b = cmax(b, LDS_GEMM_F32);
     if (vm & V_GBF16) b = cmax(b, LDS_GEMM_BF16_1);
@@ -165,6 +167,19 @@ __device__ __attribute__((noinline)) void gemm_acc_call(const TS* A, long lda, c
                                                         int m, int n, int K, int r0, int c0, bool syrk, int32_t* lock,
                                                         int32_t* err, int64_t spin_limit, char* lds) {
     item_gemm_acc<TS, PREC>(A, lda, B, ldb, C, ldc, m, n, K, r0, c0, syrk, -1.0, lock, err, spin_limit, lds);
+}
+// 64x64 GEMM/SYRK items, out of line for the same reason. They are few and on or near the critical path, so their
+// waves run at raised priority like POTRF's and TRSM's.
+template <typename TS, int PREC, int VM>
+__device__ __attribute__((noinline)) void gemm_small_call(const TS* A, const TS* B, TS* C, int m, int n, int K, int r0,
+                                                          int c0, bool syrk, char* lds, const void* PA,
+                                                          const void* PB) {
+    __builtin_amdgcn_s_setprio(3);
+    const int mu = wave_uniform(m), nu = wave_uniform(n);
+    item_gemm<TS, PREC, GEMM_BS>(wave_uniform(A), mu, wave_uniform(B), nu, wave_uniform(C), mu, mu, nu, wave_uniform(K),
+                                 wave_uniform(r0), wave_uniform(c0), wave_uniform((int)syrk) != 0, -1.0, 1.0,
+                                 lds_uniform(lds), wave_uniform(PA), wave_uniform(PB));
+    __builtin_amdgcn_s_setprio(0);
 }
 template <typename TS, typename TC, int VM>
 __device__ __attribute__((noinline)) void trsm_call(const TS* L, long ldl, const double* dinv, TS* X, long ldx, int m,
@@ -261,8 +276,9 @@ __device__ __forceinline__ bool exec_item(const DevTask& t, int it, const DevMat
                 K = M.bsz[k];
             }
             int rb, cb;
-            decode_gemm_item(it, (m + GEMM_BM - 1) / GEMM_BM, syrk, rb, cb);
-            const int r0 = rb * GEMM_BM, c0 = cb * GEMM_BM;
+            const int sub = wave_uniform(t.sub);
+            decode_gemm_item(it, (m + sub - 1) / sub, syrk, rb, cb);
+            const int r0 = rb * sub, c0 = cb * sub;
             // accumulate mode: one lock word per 128x128 sub-tile (16 per tile, shared beyond 4x4 sub-tiles)
             int32_t* lock = nullptr;
             if constexpr ((VM & V_ACC) != 0) {
@@ -270,7 +286,7 @@ __device__ __forceinline__ bool exec_item(const DevTask& t, int it, const DevMat
             } else if (t.accum) {
                 return false;
             }
-#define TTAD_GEMM_ITEM(TS_, PREC_, CPRE_)                                                                         \
+#define TTAD_GEMM_ITEM(TS_, PREC_)                                                                                 \
     if constexpr ((VM & V_ACC) != 0) {                                                                             \
         if (lock) {                                                                                                \
             gemm_acc_call<TS_, PREC_, VM>((const TS_*)opA, m, (const TS_*)opB, n, (TS_*)opC, m, m, n, K, r0, c0,  \
@@ -278,19 +294,24 @@ __device__ __forceinline__ bool exec_item(const DevTask& t, int it, const DevMat
             return true;                                                                                           \
         }                                                                                                          \
     }                                                                                                              \
-    item_gemm<TS_, PREC_, CPRE_>((const TS_*)opA, m, (const TS_*)opB, n, (TS_*)opC, m, m, n, K, r0, c0, syrk,      \
-                                 -1.0, 1.0, lds, opPA, opPB);                                                      \
+    if (sub == GEMM_BS) {                                                                                          \
+        gemm_small_call<TS_, PREC_, VM>((const TS_*)opA, (const TS_*)opB, (TS_*)opC, m, n, K, r0, c0, syrk, lds,   \
+                                        opPA, opPB);                                                               \
+        return true;                                                                                               \
+    }                                                                                                              \
+    item_gemm<TS_, PREC_>((const TS_*)opA, m, (const TS_*)opB, n, (TS_*)opC, m, m, n, K, r0, c0, syrk, -1.0, 1.0,  \
+                          lds, opPA, opPB);                                                                        \
     return true;
             // Products read C after the last K-chunk: measured faster than reading it with the first chunk
             // for FP64 (factorization at n = 32768: 246.7 -> 229.4 ms) and for bf16x3 items (11 %).
             if constexpr ((VM & V_F64S) != 0)
-                if (t.prec == P_F64) { TTAD_GEMM_ITEM(double, P_F64, false) }
+                if (t.prec == P_F64) { TTAD_GEMM_ITEM(double, P_F64) }
             if constexpr ((VM & V_G32) != 0)
-                if (t.prec == P_F32) { TTAD_GEMM_ITEM(float, P_F32, false) }
+                if (t.prec == P_F32) { TTAD_GEMM_ITEM(float, P_F32) }
             if constexpr ((VM & V_GBF16) != 0)
-                if (t.prec == P_BF16) { TTAD_GEMM_ITEM(float, P_BF16, false) }
+                if (t.prec == P_BF16) { TTAD_GEMM_ITEM(float, P_BF16) }
             if constexpr ((VM & V_GBF16X3) != 0)
-                if (t.prec == P_BF16X3) { TTAD_GEMM_ITEM(float, P_BF16X3, false) }
+                if (t.prec == P_BF16X3) { TTAD_GEMM_ITEM(float, P_BF16X3) }
 #undef TTAD_GEMM_ITEM
             return false;
         }

@@ -243,9 +243,13 @@ __global__ __launch_bounds__(NTHREADS, vset_occupancy(VM)) void k_persistent(Dev
         if (tid < 64) {
             int left = 0;
             uint64_t t1 = 0;
-            // this lane's out-edge, on its way while the counters below are updated
+            // The task record is read again (its fields would hold registers through the item: the FP64 loop then spills)
+            // and this lane's out-edge, both on their way while the counters below are updated.
+            int task_again = task;
+            asm volatile("" : "+s"(task_again));
+            const DevTask tc = g.tasks[task_again];
             DevEdge ed{};
-            if (tid < t.edge_cnt) ed = g.edges[t.edge_off + tid];
+            if (tid < tc.edge_cnt) ed = g.edges[tc.edge_off + tid];
             if (tid == 0) {
                 // Release elision: an agent-scope release (buffer_wbl2) writes back every dirty line of this
                 // XCD's L2, so the item that leaves no other item of its task running on this XCD releases for
@@ -270,8 +274,8 @@ __global__ __launch_bounds__(NTHREADS, vset_occupancy(VM)) void k_persistent(Dev
                 // last item of the task: release its successors, one per lane (a task of an n-tile column has up to n
                 // of them; each costs two dependent memory round trips, its counter and its queue's tail).
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-                for (int q = tid; q < t.edge_cnt; q += 64) {
-                    if (q >= 64) ed = g.edges[t.edge_off + q];
+                for (int q = tid; q < tc.edge_cnt; q += 64) {
+                    if (q >= 64) ed = g.edges[tc.edge_off + q];
                     const int d =
                         __hip_atomic_fetch_add(g.deps + ed.succ, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - 1;
                     if (d == 0) {
@@ -279,7 +283,7 @@ __global__ __launch_bounds__(NTHREADS, vset_occupancy(VM)) void k_persistent(Dev
                         push_task(g, ed);
                     }
                 }
-                if (tid == 0) __hip_atomic_fetch_add(g.done_items, t.n_items, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (tid == 0) __hip_atomic_fetch_add(g.done_items, tc.n_items, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
             if (tid == 0) {
                 if (g.trace) {  // {entry, workgroup, start, end, end of the successor release (last item only), 0}
@@ -296,7 +300,7 @@ __global__ __launch_bounds__(NTHREADS, vset_occupancy(VM)) void k_persistent(Dev
                     }
                 }
                 if (primary) __hip_atomic_fetch_add(idle_primary, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (t.crit) __hip_atomic_fetch_add(g.cu_crit + my_key, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (tc.crit) __hip_atomic_fetch_add(g.cu_crit + my_key, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         }
     }
@@ -353,13 +357,14 @@ __global__ void k_graph_reset_b(DevGraph g) {
 // ---------------------------------------------------------------------------
 // Raw tile kernels behind the BLAS-shaped C-ABI entry points.
 // ---------------------------------------------------------------------------
-template <typename TS, int PREC>
-__global__ __launch_bounds__(NTHREADS, 2 * (gemm_item_lds<TS, PREC>() + 1024) <= 160 * 1024 ? 2 : 1) void k_raw_gemm(const TS* A, long lda, const TS* B, long ldb, TS* C, long ldc,
-                                                       int m, int n, int K, int syrk, double alpha, double beta) {
+template <typename TS, int PREC, int BM>
+__global__ __launch_bounds__(NTHREADS, 2) void k_raw_gemm(const TS* A, long lda, const TS* B, long ldb, TS* C, long ldc,
+                                                          int m, int n, int K, int syrk, double alpha, double beta) {
     extern __shared__ __align__(16) char lds[];
+    static_assert(2 * (gemm_item_lds<TS, PREC, BM>() + 1024) <= 160 * 1024, "two workgroups per CU");
     int rb, cb;
-    decode_gemm_item(blockIdx.x, (m + GEMM_BM - 1) / GEMM_BM, syrk != 0, rb, cb);
-    item_gemm<TS, PREC>(A, lda, B, ldb, C, ldc, m, n, K, rb * GEMM_BM, cb * GEMM_BM, syrk != 0, alpha, beta, lds);
+    decode_gemm_item(blockIdx.x, (m + BM - 1) / BM, syrk != 0, rb, cb);
+    item_gemm<TS, PREC, BM>(A, lda, B, ldb, C, ldc, m, n, K, rb * BM, cb * BM, syrk != 0, alpha, beta, lds);
 }
 
 // The items wait only on lower-numbered blocks of the launch, which are dispatched first.
@@ -492,10 +497,14 @@ hipError_t kernels_init() {
     TTAD_SETLDS2(k_persistent<VSETS[3]>, vset_lds(VSETS[3]));
     TTAD_SETLDS2(k_persistent<VSETS[4]>, vset_lds(VSETS[4]));
     TTAD_SETLDS2(k_persistent<VSETS[5]>, vset_lds(VSETS[5]));
-    TTAD_SETLDS2((k_raw_gemm<double, P_F64>), (gemm_item_lds<double, P_F64>()));
-    TTAD_SETLDS2((k_raw_gemm<float, P_F32>), (gemm_item_lds<float, P_F32>()));
-    TTAD_SETLDS2((k_raw_gemm<float, P_BF16>), (gemm_item_lds<float, P_BF16>()));
-    TTAD_SETLDS2((k_raw_gemm<float, P_BF16X3>), (gemm_item_lds<float, P_BF16X3>()));
+#define TTAD_SETLDS_GEMM(ts, prec)                                                                        \
+    TTAD_SETLDS2((k_raw_gemm<ts, prec, GEMM_BM>), (gemm_item_lds<ts, prec, GEMM_BM>()));                   \
+    TTAD_SETLDS2((k_raw_gemm<ts, prec, GEMM_BS>), (gemm_item_lds<ts, prec, GEMM_BS>()))
+    TTAD_SETLDS_GEMM(double, P_F64);
+    TTAD_SETLDS_GEMM(float, P_F32);
+    TTAD_SETLDS_GEMM(float, P_BF16);
+    TTAD_SETLDS_GEMM(float, P_BF16X3);
+#undef TTAD_SETLDS_GEMM
     TTAD_SETLDS2((k_raw_potrf<double>), LDS_POTRF);
     TTAD_SETLDS2((k_raw_potrf<float>), LDS_POTRF);
     TTAD_SETLDS2((k_raw_trsm<double, double>), LDS_TRSM);
@@ -572,23 +581,32 @@ void launch_persistent(int vset, const DevGraph& g, int n_workers, hipStream_t s
     }
 }
 
+template <typename TS, int PREC, int BM>
+static void raw_gemm(const void* A, long lda, const void* B, long ldb, void* C, long ldc, int m, int n, int K, int syrk,
+                     double alpha, double beta, hipStream_t s) {
+    const long tr = (m + BM - 1) / BM, tc = (n + BM - 1) / BM;
+    const long items = syrk ? tr * (tr + 1) / 2 : tr * tc;
+    hipLaunchKernelGGL((k_raw_gemm<TS, PREC, BM>), dim3((unsigned)items), dim3(NTHREADS), (gemm_item_lds<TS, PREC, BM>()), s,
+                       (const TS*)A, lda, (const TS*)B, ldb, (TS*)C, ldc, m, n, K, syrk, alpha, beta);
+}
+
+// 64x64 items where 128x128 ones would leave CUs without work. Measured, us with 128 / with 64, by the number of 128x128
+// items: 4 (m = n = k = 256) FP64 48 / 19, FP32 25 / 11, bf16x3 17 / 10; 64 (m = n = 1000, k = 300) FP64 74 / 31, bf16x3
+// 30 / 16; 144 (1536, 512) FP64 90 / 78, FP32 47 / 42, bf16x3 32 / 25; 256 (2048, 1024) FP64 175 / 191, FP32 92 / 97,
+// bf16x3 62 / 53; 484 (2816, 512) FP64 158 / 191, FP32 81 / 97, bf16x3 44 / 54.
+static bool raw_gemm_small(int prec, long items) { return items <= (prec == P_F64 || prec == P_F32 ? 192 : 256); }
+
 void launch_raw_gemm(int prec, const void* A, long lda, const void* B, long ldb, void* C, long ldc, int m, int n,
                      int K, int syrk, double alpha, double beta, hipStream_t s) {
-    const int tr = (m + GEMM_BM - 1) / GEMM_BM, tc = (n + GEMM_BM - 1) / GEMM_BM;
-    const int items = syrk ? tr * (tr + 1) / 2 : tr * tc;
+    const long tr = (m + GEMM_BM - 1) / GEMM_BM, tc = (n + GEMM_BM - 1) / GEMM_BM;
+    const long items = syrk ? tr * (tr + 1) / 2 : tr * tc;
     if (items <= 0) return;
-    if (prec == P_F64)
-        hipLaunchKernelGGL((k_raw_gemm<double, P_F64>), dim3(items), dim3(NTHREADS), (gemm_item_lds<double, P_F64>()), s,
-                           (const double*)A, lda, (const double*)B, ldb, (double*)C, ldc, m, n, K, syrk, alpha, beta);
-    else if (prec == P_F32)
-        hipLaunchKernelGGL((k_raw_gemm<float, P_F32>), dim3(items), dim3(NTHREADS), (gemm_item_lds<float, P_F32>()), s, (const float*)A,
-                           lda, (const float*)B, ldb, (float*)C, ldc, m, n, K, syrk, alpha, beta);
-    else if (prec == P_BF16)
-        hipLaunchKernelGGL((k_raw_gemm<float, P_BF16>), dim3(items), dim3(NTHREADS), (gemm_item_lds<float, P_BF16>()), s,
-                           (const float*)A, lda, (const float*)B, ldb, (float*)C, ldc, m, n, K, syrk, alpha, beta);
-    else
-        hipLaunchKernelGGL((k_raw_gemm<float, P_BF16X3>), dim3(items), dim3(NTHREADS), (gemm_item_lds<float, P_BF16X3>()), s,
-                           (const float*)A, lda, (const float*)B, ldb, (float*)C, ldc, m, n, K, syrk, alpha, beta);
+    const bool small = raw_gemm_small(prec, items);
+    auto* f = prec == P_F64    ? (small ? raw_gemm<double, P_F64, GEMM_BS> : raw_gemm<double, P_F64, GEMM_BM>)
+              : prec == P_F32  ? (small ? raw_gemm<float, P_F32, GEMM_BS> : raw_gemm<float, P_F32, GEMM_BM>)
+              : prec == P_BF16 ? (small ? raw_gemm<float, P_BF16, GEMM_BS> : raw_gemm<float, P_BF16, GEMM_BM>)
+                               : (small ? raw_gemm<float, P_BF16X3, GEMM_BS> : raw_gemm<float, P_BF16X3, GEMM_BM>);
+    f(A, lda, B, ldb, C, ldc, m, n, K, syrk, alpha, beta, s);
 }
 
 void launch_raw_potrf(int prec, void* A, long lda, int n, double* dinv, int* info, int32_t* flags, int32_t* err,

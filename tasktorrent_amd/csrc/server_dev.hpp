@@ -324,6 +324,7 @@ __device__ __forceinline__ void srv_exec(const DevServer& s, const SrvTask& t, i
             d.i = t.i;
             d.j = t.j;
             d.k = t.k;
+            d.sub = GEMM_BM;
             (void)exec_item<V_ALL>(d, it, s.mats, lds, s.err, s.spin_limit);  // request graphs only hold supported kinds
             break;
         }

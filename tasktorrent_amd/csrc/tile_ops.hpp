@@ -554,7 +554,9 @@ __device__ __forceinline__ void store_split4(unsigned short* __restrict__ planes
 // two buffers, so that two workgroups share a CU: one's barriers, loads and C traffic overlap
 // the other's MFMAs (FP64, m = n = 16384, K = 512: 43.5 TF/s with one 130 KB workgroup per CU,
 // 53 TF/s with two; 66 TF/s with the 16-byte loads, coalesced C and C read up front).
-template <typename TC> constexpr int gemm_bk() { return sizeof(TC) == 8 ? 16 : 32; }
+// 64x64 items take chunks twice as long: they are used where latency counts (few items in flight), and each chunk costs
+// a memory round trip.
+template <typename TC, int BM = GEMM_BM> constexpr int gemm_bk() { return (sizeof(TC) == 8 ? 16 : 32) * (GEMM_BM / BM); }
 // K-chunk of a TRSM item's update from the solved columns: each chunk waits for its loads (issued one chunk
 // ahead), so fewer chunks cost fewer round trips. 64 FP32 columns fit the LDS of the FP32 executors; the FP64
 // ones allow 32.
@@ -566,119 +568,85 @@ template <typename TS> constexpr int trsm_bk() { return sizeof(TS) == 4 ? 64 : 3
 // lower triangle (global row >= global col) is written (dsyrk 'L').
 // beta == 0 overwrites C without reading it (accumulate-mode temporaries).
 // ---------------------------------------------------------------------------
-// CPRE (the Cholesky update, alpha = -1, beta = 1): the accumulators start from -C, read
-// together with the first K-chunk instead of after the last one, and C = -acc is stored.
+// BM: rows and columns of the item, GEMM_BM or GEMM_BS.
 // PA / PB (bf16x3 only; null = none): the bf16 split planes of the operand tiles (A and B with lda and ldb
 // rows, plane_granule layout), used by items that lie wholly inside both with K % 32 == 0.
-template <typename TS, int PREC, bool CPRE = false>
+template <typename TS, int PREC, int BM = GEMM_BM>
 __device__ __forceinline__ void item_gemm(const TS* __restrict__ A, long lda, const TS* __restrict__ B, long ldb, TS* __restrict__ C,
                           long ldc, int m, int n, int K, int r0, int c0, bool syrk, double alpha, double beta,
                           char* lds, const void* PA = nullptr, const void* PB = nullptr) {
-    const int mv = min(GEMM_BM, m - r0), nv = min(GEMM_BM, n - c0);
+    const int mv = min(BM, m - r0), nv = min(BM, n - c0);
     if (mv <= 0 || nv <= 0) return;
     auto body = [&](auto* gsel) {
         using G = typename std::remove_pointer<decltype(gsel)>::type;
         typedef typename G::acc_t acc_t;
         acc_t acc[G::WM][G::WN];
         auto owned = [&](int rr, int cc) { return rr < mv && cc < nv && (!syrk || r0 + rr >= c0 + cc); };
-        if constexpr (CPRE) {
-#pragma unroll
-            for (int a = 0; a < G::WM; a++)
-#pragma unroll
-                for (int b = 0; b < G::WN; b++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        const int rr = G::row_of(a, r), cc = G::col_of(b, r);
-                        acc[a][b][r] = owned(rr, cc) ? -gmem(C)[(r0 + rr) + (long)(c0 + cc) * ldc] : TS(0);
-                    }
-        } else {
-            G::zero(acc);
-        }
+        G::zero(acc);
         bool planes = false;
         if constexpr (PREC == P_BF16X3)
-            planes = PA && PB && mv == GEMM_BM && nv == GEMM_BM && K % G::BK == 0;
+            planes = PA && PB && mv == BM && nv == BM && K % G::BK == 0;
         if constexpr (PREC == P_BF16X3) {
             if (planes)
                 G::run_planes(acc, static_cast<const u4_t*>(PA) + r0, (int)lda, static_cast<const u4_t*>(PB) + c0,
                               (int)ldb, K, lds);
         }
         if (!planes) G::run(acc, A + r0, lda, mv, B + c0, ldb, nv, K, lds);
-        if constexpr (CPRE) {
-#pragma unroll
-            for (int a = 0; a < G::WM; a++)
-#pragma unroll
-                for (int b = 0; b < G::WN; b++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        const int rr = G::row_of(a, r), cc = G::col_of(b, r);
-                        if (owned(rr, cc)) gmem(C)[(r0 + rr) + (long)(c0 + cc) * ldc] = (TS)(-acc[a][b][r]);
-                    }
-        } else {
-            // C is read after the last K-chunk. Every load of a group of fragment rows is issued before any
-            // store of the group: as far as the compiler knows a store may alias a later load, so a load and
-            // a store per element in turn would cost one memory round trip per element (64 per item). Groups:
-            // all of the item for FP32 tiles, one fragment row for FP64 (registers). Loads come from clamped addresses
-            // (C[0] for elements not owned), so none waits under a branch; interior items (all of the
-            // 128 x 128 owned) store without a condition.
-            const bool full = __builtin_amdgcn_readfirstlane(
-                                  (int)(mv == GEMM_BM && nv == GEMM_BM && (!syrk || r0 >= c0 + GEMM_BM))) != 0;
-            if constexpr (sizeof(TS) == 4) {
-                // Interior FP32 items go through LDS (free after the K loop): a lane's results lie along a row,
-                // C is column-major, so the accumulators are transposed in LDS and every thread then reads,
-                // updates and writes 16 contiguous bytes of C per access (16 loads and 16 stores per thread
-                // instead of 64 each). C is read first, so its latency overlaps the transposition.
-                if (full) {
-                    constexpr int P = GEMM_BM + 4;  // LDS column pitch: the 4 column groups of a wave hit distinct banks
-                    static_assert(GEMM_BM * P * 4 <= G::LDS_BYTES, "transposed item fits the item's LDS");
-                    typedef typename V16<TS>::u f4u;
-                    TS* T = reinterpret_cast<TS*>(lds);
-                    const int rg = threadIdx.x % 32, cl = threadIdx.x / 32;  // rows 4rg .. 4rg+3 of columns cl + 8j
-                    const long ldu = wave_uniform((int)ldc);
-                    TTAD_GLOBAL TS* base = gmem(C) + (r0 + 4 * rg) + (long)(c0 + cl) * ldu;
-                    constexpr int NJ = GEMM_BM / 8;
-                    f4_t cv[NJ];
-                    if (beta != 0.0) {
-#pragma unroll
-                        for (int j = 0; j < NJ; j++) cv[j] = *reinterpret_cast<TTAD_GLOBAL f4u*>(base + 8 * j * ldu);
-                    }
-#pragma unroll
-                    for (int a = 0; a < G::WM; a++)
-#pragma unroll
-                        for (int b = 0; b < G::WN; b++)
-#pragma unroll
-                            for (int r = 0; r < 4; r++) T[G::col_of(b, r) * P + G::row_of(a, r)] = acc[a][b][r];
-                    __syncthreads();
-#pragma unroll
-                    for (int j = 0; j < NJ; j++) {
-                        const f4_t v = *reinterpret_cast<const f4_t*>(T + (cl + 8 * j) * P + 4 * rg);
-                        f4_t o;
-#pragma unroll
-                        for (int r = 0; r < 4; r++) {
-                            const double x = alpha * (double)v[r];
-                            o[r] = (TS)(beta == 0.0 ? x : beta * (double)cv[j][r] + x);
-                        }
-                        *reinterpret_cast<TTAD_GLOBAL f4u*>(base + 8 * j * ldu) = o;
-                    }
-                    __syncthreads();  // the caller may use lds again
-                    return;
-                }
-            }
-            constexpr int AG = sizeof(TS) == 8 ? 1 : G::WM;
-#pragma unroll
-            for (int a0 = 0; a0 < G::WM; a0 += AG) {
-                TS cv[AG][G::WN][4];
+        // C is read after the last K-chunk. Every load of a group of fragment rows is issued before any
+        // store of the group: as far as the compiler knows a store may alias a later load, so a load and
+        // a store per element in turn would cost one memory round trip per element (64 per item). Groups:
+        // all of the item for FP32 tiles, one fragment row for FP64 (registers). Loads come from clamped addresses
+        // (C[0] for elements not owned), so none waits under a branch; interior items (all of the
+        // 128 x 128 owned) store without a condition.
+        const bool full = __builtin_amdgcn_readfirstlane(
+                              (int)(mv == BM && nv == BM && (!syrk || r0 >= c0 + BM))) != 0;
+        if constexpr (sizeof(TS) == 4) {
+            // Interior FP32 items go through LDS (free after the K loop): a lane's results lie along a row,
+            // C is column-major, so the accumulators are transposed in LDS and every thread then reads,
+            // updates and writes 16 contiguous bytes of C per access (16 loads and 16 stores per thread
+            // instead of 64 each). C is read first, so its latency overlaps the transposition.
+            if (full) {
+                constexpr int P = BM + 4;  // LDS column pitch: the 4 column groups of a wave hit distinct banks
+                static_assert(BM * P * 4 <= G::LDS_BYTES, "transposed item fits the item's LDS");
+                typedef typename V16<TS>::u f4u;
+                TS* T = reinterpret_cast<TS*>(lds);
+                constexpr int RL = BM / 4, CL = NTHREADS / RL;  // lanes along a column, columns per pass
+                const int rg = threadIdx.x % RL, cl = threadIdx.x / RL;  // rows 4rg .. 4rg+3 of columns cl + CL j
+                const long ldu = wave_uniform((int)ldc);
+                TTAD_GLOBAL TS* base = gmem(C) + (r0 + 4 * rg) + (long)(c0 + cl) * ldu;
+                constexpr int NJ = BM / CL;
+                f4_t cv[NJ];
                 if (beta != 0.0) {
 #pragma unroll
-                    for (int a = 0; a < AG; a++)
-#pragma unroll
-                        for (int b = 0; b < G::WN; b++)
-#pragma unroll
-                            for (int r = 0; r < 4; r++) {
-                                const int rr = G::row_of(a0 + a, r), cc = G::col_of(b, r);
-                                const long off = (r0 + rr) + (long)(c0 + cc) * ldc;
-                                cv[a][b][r] = gmem(C)[(full || owned(rr, cc)) ? off : 0];
-                            }
+                    for (int j = 0; j < NJ; j++) cv[j] = *reinterpret_cast<TTAD_GLOBAL f4u*>(base + CL * j * ldu);
                 }
+#pragma unroll
+                for (int a = 0; a < G::WM; a++)
+#pragma unroll
+                    for (int b = 0; b < G::WN; b++)
+#pragma unroll
+                        for (int r = 0; r < 4; r++) T[G::col_of(b, r) * P + G::row_of(a, r)] = acc[a][b][r];
+                __syncthreads();
+#pragma unroll
+                for (int j = 0; j < NJ; j++) {
+                    const f4_t v = *reinterpret_cast<const f4_t*>(T + (cl + CL * j) * P + 4 * rg);
+                    f4_t o;
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const double x = alpha * (double)v[r];
+                        o[r] = (TS)(beta == 0.0 ? x : beta * (double)cv[j][r] + x);
+                    }
+                    *reinterpret_cast<TTAD_GLOBAL f4u*>(base + CL * j * ldu) = o;
+                }
+                __syncthreads();  // the caller may use lds again
+                return;
+            }
+        }
+        constexpr int AG = sizeof(TS) == 8 && BM == GEMM_BM ? 1 : G::WM;
+#pragma unroll
+        for (int a0 = 0; a0 < G::WM; a0 += AG) {
+            TS cv[AG][G::WN][4];
+            if (beta != 0.0) {
 #pragma unroll
                 for (int a = 0; a < AG; a++)
 #pragma unroll
@@ -686,17 +654,27 @@ __device__ __forceinline__ void item_gemm(const TS* __restrict__ A, long lda, co
 #pragma unroll
                         for (int r = 0; r < 4; r++) {
                             const int rr = G::row_of(a0 + a, r), cc = G::col_of(b, r);
-                            const double v = alpha * (double)acc[a0 + a][b][r];
-                            const TS o = (TS)(beta == 0.0 ? v : beta * (double)cv[a][b][r] + v);
-                            if (full || owned(rr, cc)) gmem(C)[(r0 + rr) + (long)(c0 + cc) * ldc] = o;
+                            const long off = (r0 + rr) + (long)(c0 + cc) * ldc;
+                            cv[a][b][r] = gmem(C)[(full || owned(rr, cc)) ? off : 0];
                         }
             }
+#pragma unroll
+            for (int a = 0; a < AG; a++)
+#pragma unroll
+                for (int b = 0; b < G::WN; b++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const int rr = G::row_of(a0 + a, r), cc = G::col_of(b, r);
+                        const double v = alpha * (double)acc[a0 + a][b][r];
+                        const TS o = (TS)(beta == 0.0 ? v : beta * (double)cv[a][b][r] + v);
+                        if (full || owned(rr, cc)) gmem(C)[(r0 + rr) + (long)(c0 + cc) * ldc] = o;
+                    }
         }
     };
     if constexpr (PREC == P_BF16 || PREC == P_BF16X3) {
-        body((GemmNTbf16<TS, GEMM_BM, GEMM_BM, PREC == P_BF16X3, true>*)nullptr);
+        body((GemmNTbf16<TS, BM, BM, PREC == P_BF16X3, true>*)nullptr);
     } else {  // F64 tiles on FP64 MFMA, F32 tiles on FP32 MFMA
-        body((GemmNT<TS, TS, TS, GEMM_BM, GEMM_BM, gemm_bk<TS>(), true, true>*)nullptr);
+        body((GemmNT<TS, TS, TS, BM, BM, gemm_bk<TS, BM>(), true, true>*)nullptr);
     }
 }
 
@@ -1378,7 +1356,11 @@ constexpr int LDS_GEMM_F32 = GemmNT<float, float, float, GEMM_BM, GEMM_BM, gemm_
 constexpr int LDS_GEMM_BF16 = GemmNTbf16<float, GEMM_BM, GEMM_BM, true, true>::LDS_BYTES;
 constexpr int LDS_GEMM_BF16_1 = GemmNTbf16<float, GEMM_BM, GEMM_BM, false, true>::LDS_BYTES;
 // LDS of one GEMM item of the given storage / precision (the standalone kernels launch with it).
-template <typename TS, int PREC> constexpr int gemm_item_lds() {
+template <typename TS, int PREC, int BM = GEMM_BM> constexpr int gemm_item_lds() {
+    if (BM != GEMM_BM)
+        return PREC == P_BF16X3 ? GemmNTbf16<float, BM, BM, true, true>::LDS_BYTES
+               : PREC == P_BF16 ? GemmNTbf16<float, BM, BM, false, true>::LDS_BYTES
+                                : GemmNT<TS, TS, TS, BM, BM, gemm_bk<TS, BM>(), true, true>::LDS_BYTES;
     return PREC == P_BF16X3 ? LDS_GEMM_BF16 : PREC == P_BF16 ? LDS_GEMM_BF16_1 : sizeof(TS) == 8 ? LDS_GEMM_F64 : LDS_GEMM_F32;
 }
 constexpr int LDS_TRSM = cmax(GemmNT<double, double, double, TRSM_BM, DB, 32, true, true>::LDS_BYTES,

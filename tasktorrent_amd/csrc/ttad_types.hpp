@@ -11,6 +11,7 @@ enum Prec : int32_t { P_F64 = 0, P_F32 = 1, P_BF16 = 2, P_BF16X3 = 3 };
 
 constexpr int NTHREADS = 256;  // one workgroup = 4 wave64
 constexpr int GEMM_BM = 128;   // GEMM/SYRK work item = 128x128 output sub-tile
+constexpr int GEMM_BS = 64;    // or a 64x64 one, where the items of 128 leave CUs idle (DevTask::sub)
 constexpr int TRSM_BM = 32;      // TRSM work item of an FP64 tile: 32-row block (its latency is on the critical path)
 constexpr int TRSM_BM_F32 = 64;  // of an FP32 tile: 64-row block (half the items: fewer re-reads of the diagonal tile)
 __host__ __device__ constexpr int trsm_rows(int elem_bytes) { return elem_bytes == 8 ? TRSM_BM : TRSM_BM_F32; }
@@ -52,6 +53,7 @@ struct DevTask {
     int32_t crit;  // on a longest path of the DAG: runs with no other item started on its CU
     int32_t accum; // GEMM/SYRK: add the product into C under the sub-tile lock (accumulate mode)
     int32_t edge_off, edge_cnt;  // its out-edges in DevGraph::edges
+    int32_t sub;   // GEMM/SYRK: rows and columns of an item, GEMM_BM or GEMM_BS
 };
 
 // An out-edge of the graph with all that releasing its target takes: the task that completes reads it in one access
@@ -66,12 +68,13 @@ struct alignas(16) DevEdge {
 };
 
 // Work items per task of tiles with elem_bytes-byte elements; host and device must agree.
-__host__ __device__ inline int items_of(int kind, int bi, int bj, int elem_bytes) {
+// (sub: rows and columns of a GEMM/SYRK item).
+__host__ __device__ inline int items_of(int kind, int bi, int bj, int elem_bytes, int sub = GEMM_BM) {
     if (kind == K_POTRF) return 1;
     if (kind == K_TRSM) return (bi + trsm_rows(elem_bytes) - 1) / trsm_rows(elem_bytes);
-    const int tr = (bi + GEMM_BM - 1) / GEMM_BM;
+    const int tr = (bi + sub - 1) / sub;
     if (kind == K_SYRK) return tr * (tr + 1) / 2;
-    if (kind == K_GEMM) return tr * ((bj + GEMM_BM - 1) / GEMM_BM);
+    if (kind == K_GEMM) return tr * ((bj + sub - 1) / sub);
     return 1;
 }
 
