@@ -339,6 +339,7 @@ int ttad_matrix_create(ttad_context* ctx, int num_blocks, const int* block_sizes
         M->boff[i + 1] = M->boff[i] + block_sizes[i];
     }
     M->n = M->boff[num_blocks];
+    M->max_b = *std::max_element(M->bsz.begin(), M->bsz.end());
     const int nt = num_blocks;
     const size_t align = 256 / M->elem;
     M->tile_off.assign((size_t)nt * nt, 0);
@@ -370,7 +371,7 @@ int ttad_matrix_create(ttad_context* ctx, int num_blocks, const int* block_sizes
     TTAD_HIP(M->tab_tiles.alloc((size_t)nt * nt * sizeof(void*)));
     TTAD_HIP(M->tab_dinv.alloc(nt * sizeof(double*)));
     TTAD_HIP(M->info.alloc(sizeof(int)));
-    const int pf_stride = potrf_flags(*std::max_element(M->bsz.begin(), M->bsz.end()));
+    const int pf_stride = potrf_flags(M->max_b);
     M->pflags_bytes = (size_t)nt * pf_stride * sizeof(int32_t);
     TTAD_HIP(M->pflags.alloc(M->pflags_bytes));
     TTAD_HIP(M->locks.alloc((size_t)nt * nt * 16 * sizeof(int32_t)));
@@ -434,7 +435,7 @@ int ttad_matrix_set(ttad_matrix* M, const double* A, long long lda, int src_devi
     M->anorm_valid = false;
     hipStream_t s = pick(M->ctx, stream);
     if (src_device) {
-        launch_pack(M->storage, A, lda, M->desc.as<DevMat>(), M->nt, s);
+        launch_pack(M->storage, A, lda, M->desc.as<DevMat>(), M->nt, M->max_b, s);
         TTAD_HIP(hipGetLastError());
         return TTAD_OK;
     }
@@ -442,7 +443,7 @@ int ttad_matrix_set(ttad_matrix* M, const double* A, long long lda, int src_devi
     if (tmp.alloc((size_t)M->n * M->n * 8) != hipSuccess) return set_error(TTAD_ERR_OOM, "matrix_set: staging");
     TTAD_HIP(hipMemcpy2DAsync(tmp.p, (size_t)M->n * 8, A, (size_t)lda * 8, (size_t)M->n * 8, M->n,
                               hipMemcpyHostToDevice, s));
-    launch_pack(M->storage, tmp.as<double>(), M->n, M->desc.as<DevMat>(), M->nt, s);
+    launch_pack(M->storage, tmp.as<double>(), M->n, M->desc.as<DevMat>(), M->nt, M->max_b, s);
     TTAD_HIP(hipGetLastError());
     TTAD_HIP(hipStreamSynchronize(s));
     return TTAD_OK;
@@ -452,13 +453,13 @@ int ttad_matrix_get(ttad_matrix* M, double* A, long long lda, int dst_device, vo
     if (!M || !A || lda < std::max(1, M->n)) return set_error(TTAD_ERR_INVALID, "matrix_get: bad args");
     hipStream_t s = pick(M->ctx, stream);
     if (dst_device) {
-        launch_unpack(M->storage, A, lda, M->desc.as<DevMat>(), M->nt, 1, s);
+        launch_unpack(M->storage, A, lda, M->desc.as<DevMat>(), M->nt, M->max_b, 1, s);
         TTAD_HIP(hipGetLastError());
         return TTAD_OK;
     }
     DevBuf tmp;
     if (tmp.alloc((size_t)M->n * M->n * 8) != hipSuccess) return set_error(TTAD_ERR_OOM, "matrix_get: staging");
-    launch_unpack(M->storage, tmp.as<double>(), M->n, M->desc.as<DevMat>(), M->nt, 1, s);
+    launch_unpack(M->storage, tmp.as<double>(), M->n, M->desc.as<DevMat>(), M->nt, M->max_b, 1, s);
     TTAD_HIP(hipGetLastError());
     TTAD_HIP(hipMemcpy2DAsync(A, (size_t)lda * 8, tmp.p, (size_t)M->n * 8, (size_t)M->n * 8, M->n,
                               hipMemcpyDeviceToHost, s));

@@ -25,8 +25,9 @@ void launch_raw_potrf(int prec, void* A, long lda, int n, double* dinv, int* inf
 void launch_trtri_diag(int prec, const void* L, long ldl, int n, double* dinv, hipStream_t s);
 void launch_raw_trsm(int prec, const void* L, long ldl, const double* dinv, void* X, long ldx, int m, int n,
                      hipStream_t s);
-void launch_pack(int storage, const double* src, long lda, const DevMat* M, int nt, hipStream_t s);
-void launch_unpack(int storage, double* dst, long ldd, const DevMat* M, int nt, int zero_upper, hipStream_t s);
+// max_b: the largest tile size of M.
+void launch_pack(int storage, const double* src, long lda, const DevMat* M, int nt, int max_b, hipStream_t s);
+void launch_unpack(int storage, double* dst, long ldd, const DevMat* M, int nt, int max_b, int zero_upper, hipStream_t s);
 void launch_copy_tiles(int dst_storage, int src_storage, const DevMat* S, const DevMat* D, int nt, hipStream_t s);
 
 }  // namespace ttad

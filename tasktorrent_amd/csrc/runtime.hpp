@@ -88,7 +88,7 @@ struct ttad_context {
 struct ttad_matrix {
     ttad_context* ctx = nullptr;
     long long id = 0;
-    int nt = 0, n = 0, storage = TTAD_F64;
+    int nt = 0, n = 0, max_b = 0, storage = TTAD_F64;
     std::vector<int> bsz, boff;
     std::vector<size_t> tile_off;  // element offset of tile (i,j) (i >= j), index i + j*nt
     ttad::DevBuf tiles, dinv, tab_bsz, tab_boff, tab_tiles, tab_dinv, info, desc, pflags, locks;
