@@ -140,6 +140,15 @@ int ttad_init(int device, ttad_context** out) {
     }
     for (int q = 0; q < N_VSETS; q++) c->vset_workers_per_cu[q] = persistent_blocks_per_cu(q);
     c->workers_per_cu = c->vset_workers_per_cu[0];
+    if ((e = c->reports.alloc(ttad_context::REPORT_SLOTS * sizeof(GraphReport))) != hipSuccess) {
+        delete c;
+        return set_error(TTAD_ERR_OOM, "init: pinned report memory: %s", hipGetErrorString(e));
+    }
+    if ((e = c->readback.alloc(4096)) != hipSuccess) {
+        delete c;
+        return set_error(TTAD_ERR_OOM, "init: pinned readback memory: %s", hipGetErrorString(e));
+    }
+    for (int q = ttad_context::REPORT_SLOTS - 1; q >= 0; q--) c->free_reports.push_back(q);
     if (hipEventCreate(&c->ev_a) != hipSuccess || hipEventCreate(&c->ev_b) != hipSuccess) {
         delete c;
         return set_error(TTAD_ERR_DEVICE, "init: event creation failed");
@@ -224,8 +233,8 @@ static int potrf_common(ttad_context* ctx, int prec, int n, void* A, int lda, in
     launch_raw_potrf(prec, A, lda, n, ctx->scratch_dinv.as<double>(), info_err, ctx->scratch_pflags.as<int32_t>(),
                      info_err + 1, s);
     TTAD_HIP(hipGetLastError());
-    int he[2] = {0, 0};
-    TTAD_HIP(hipMemcpyAsync(he, info_err, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
+    const int* he = (const int*)ctx->readback.host;
+    TTAD_HIP(hipMemcpyAsync(ctx->readback.host, info_err, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
     TTAD_HIP(hipStreamSynchronize(s));
     if (he[1]) {
         (void)hipMemsetAsync(ctx->scratch_pflags.p, 0, ctx->scratch_pflags.bytes, s);
@@ -504,13 +513,13 @@ int ttad_potrf_tiled(ttad_context* ctx, ttad_matrix* M, int schedule, int prio_k
         return set_error(TTAD_ERR_INVALID, "potrf_tiled: precision %d does not match the tile storage", prec);
     if (info) *info = 0;
     hipStream_t s = pick(ctx, stream);
-    TTAD_HIP(hipMemsetAsync(M->info.p, 0, sizeof(int), s));
-    TTAD_HIP(hipMemsetAsync(M->pflags.p, 0, M->pflags_bytes, s));
     int rc = TTAD_OK;
     ctx->ev_valid = false;
     ctx->kernel_s = -1.0;
-    TTAD_HIP(hipEventRecord(ctx->ev_a, s));
     if (schedule == TTAD_SCHED_STREAM) {
+        TTAD_HIP(hipMemsetAsync(M->info.p, 0, sizeof(int), s));
+        TTAD_HIP(hipMemsetAsync(M->pflags.p, 0, M->pflags_bytes, s));
+        TTAD_HIP(hipEventRecord(ctx->ev_a, s));
         auto key = std::make_pair(M->id, prec);
         auto it = ctx->stream_plans.find(key);
         std::shared_ptr<StreamPlan> plan;
@@ -535,8 +544,14 @@ int ttad_potrf_tiled(ttad_context* ctx, ttad_matrix* M, int schedule, int prio_k
             return set_error(TTAD_ERR_DEVICE, "potrf_tiled: item variant missing from the executor (%d)", err);
         }
     } else if (schedule == TTAD_SCHED_PERSISTENT) {
-        rc = cholesky_persistent(ctx, M, prio_kind, prec, s, info);
+        // (its kernels clear the matrix's pivot report and flags themselves; its report holds the pivot)
+        int h = 0;
+        rc = cholesky_persistent(ctx, M, prio_kind, prec, s, &h);
         if (rc != TTAD_OK && rc != TTAD_ERR_NOT_SPD) return rc;
+        ctx->ev_valid = true;
+        if (info) *info = h;
+        if (h) return set_error(TTAD_ERR_NOT_SPD, "potrf_tiled: non-positive pivot at column %d", h);
+        return TTAD_OK;
     } else {
         return set_error(TTAD_ERR_INVALID, "potrf_tiled: unknown schedule %d", schedule);
     }
@@ -698,6 +713,17 @@ int ttad_graph_create(ttad_context* ctx, int n_tasks, const ttad_task_desc* task
     g->seeds.assign(n_tasks, 0);
     TTAD_HIP(hipEventCreate(&g->ev_start));
     TTAD_HIP(hipEventCreate(&g->ev_stop));
+    if (!ctx->free_reports.empty()) {
+        g->report_slot = ctx->free_reports.back();
+        ctx->free_reports.pop_back();
+        g->report = (GraphReport*)ctx->reports.host + g->report_slot;
+        g->report_dev = (GraphReport*)ctx->reports.dev + g->report_slot;
+    } else {
+        TTAD_HIP(g->own_report.alloc(sizeof(GraphReport)));
+        g->report = (GraphReport*)g->own_report.host;
+        g->report_dev = (GraphReport*)g->own_report.dev;
+    }
+    g->report->seq = 0;
     *out = g.release();
     return TTAD_OK;
 }
@@ -772,6 +798,7 @@ static int graph_prepare(ttad_graph* g) {
         for (auto& x : g->tasks)
             if (x.kind != K_NOP) needed |= item_variant(x.kind, x.prec, g->mats[x.mat]->storage) | (x.accum ? V_ACC : 0);
         g->vset = vset_index(needed);
+        g->has_accum = (needed & V_ACC) != 0;
         g->bucket_items.assign(g->n_buckets, 0);
         // queue entries hold (task << 20) | item in 64 bits and slots are 32-bit indices
         long long total = 0;
@@ -838,24 +865,20 @@ static int graph_prepare(ttad_graph* g) {
                 return set_error(TTAD_ERR_GRAPH, "graph: task %d has indegree %d but receives %d edges + %d seeds", t,
                                  g->indegree[t], incoming[t], g->seeds[t]);
         std::vector<int32_t> deps0(n), tail0(g->n_buckets, 0);
-        std::vector<int64_t> init;  // queue entries (task << 20) | item, as the device pushes them
-        std::vector<int32_t> init_slot;
+        std::vector<int64_t> items0(g->total_items, -1);  // queue entries (task << 20) | item, as the device pushes them
+        bool any_ready = false;
         for (int t = 0; t < n; t++) {
             deps0[t] = g->indegree[t] - g->seeds[t];
             if (deps0[t] == 0) {
                 const DevTask& x = g->tasks[t];
-                for (int r = 0; r < x.n_items; r++) {
-                    init_slot.push_back(g->q_base[x.bucket] + tail0[x.bucket]++);
-                    init.push_back(((int64_t)t << 20) | r);
-                }
+                any_ready = true;
+                for (int r = 0; r < x.n_items; r++)
+                    items0[g->q_base[x.bucket] + tail0[x.bucket]++] = ((int64_t)t << 20) | r;
             }
         }
-        if (init.empty()) return set_error(TTAD_ERR_GRAPH, "graph: no task is ready (seed one with ttad_graph_seed)");
-        g->n_init = (int)init.size();
-        TTAD_HIP(g->d_init.alloc(init.size() * 8));
-        TTAD_HIP(g->d_init_slot.alloc(init_slot.size() * 4));
-        TTAD_HIP(hipMemcpy(g->d_init.p, init.data(), init.size() * 8, hipMemcpyHostToDevice));
-        TTAD_HIP(hipMemcpy(g->d_init_slot.p, init_slot.data(), init_slot.size() * 4, hipMemcpyHostToDevice));
+        if (!any_ready) return set_error(TTAD_ERR_GRAPH, "graph: no task is ready (seed one with ttad_graph_seed)");
+        TTAD_HIP(g->d_q_items0.alloc(items0.size() * 8));
+        TTAD_HIP(hipMemcpy(g->d_q_items0.p, items0.data(), items0.size() * 8, hipMemcpyHostToDevice));
         TTAD_HIP(hipMemcpy(g->d_deps0.p, deps0.data(), n * 4, hipMemcpyHostToDevice));
         TTAD_HIP(hipMemcpy(g->d_tail0.p, tail0.data(), g->n_buckets * 4, hipMemcpyHostToDevice));
         g->seeds_dirty = false;
@@ -868,13 +891,13 @@ static DevGraph graph_image(ttad_graph* g, bool trace, int64_t spin_limit) {
     d.n_tasks = g->n_tasks;
     d.n_buckets = g->n_buckets;
     d.total_items = g->total_items;
-    d.n_init = g->n_init;
+    d.n_mats = (int)g->mats.size();
+    d.has_accum = g->has_accum;
     d.tasks = g->d_tasks.as<DevTask>();
     d.edges = g->d_edges.as<DevEdge>();
     d.deps0 = g->d_deps0.as<int32_t>();
     d.tail0 = g->d_tail0.as<int32_t>();
-    d.init_items = g->d_init.as<int64_t>();
-    d.init_slots = g->d_init_slot.as<int32_t>();
+    d.q_items0 = g->d_q_items0.as<int64_t>();
     d.deps = g->d_deps.as<int32_t>();
     d.items_left = g->d_items_left.as<int32_t>();
     d.gops = g->d_gops.as<GemmOperands>();
@@ -918,17 +941,12 @@ int ttad_graph_launch(ttad_graph* g, int n_workers, int trace, void* stream) {
     g->workers = n_workers > 0 ? n_workers : dflt;
     g->stream = pick(ctx, stream);
     launch_graph_reset(d, g->total_items, g->stream);
-    for (auto* M : g->mats)
-        if (M) {
-            TTAD_HIP(hipMemsetAsync(M->info.p, 0, sizeof(int), g->stream));
-            // POTRF flags: cleared by every completed task, and here after a stopped run
-            TTAD_HIP(hipMemsetAsync(M->pflags.p, 0, M->pflags_bytes, g->stream));
-            TTAD_HIP(hipMemsetAsync(M->locks.p, 0, (size_t)M->nt * M->nt * 16 * sizeof(int32_t), g->stream));
-        }
     TTAD_HIP(hipEventRecord(g->ev_start, g->stream));
     launch_persistent(g->vset, d, g->workers, g->stream);
     TTAD_HIP(hipGetLastError());
     TTAD_HIP(hipEventRecord(g->ev_stop, g->stream));
+    launch_graph_report(d, g->report_dev, ++g->seq, g->stream);
+    TTAD_HIP(hipGetLastError());
     g->running = true;
     return TTAD_OK;
 }
@@ -936,23 +954,26 @@ int ttad_graph_launch(ttad_graph* g, int n_workers, int trace, void* stream) {
 int ttad_graph_wait(ttad_graph* g, double timeout_s, ttad_graph_stats* stats) {
     if (!g) return set_error(TTAD_ERR_INVALID, "graph is NULL");
     if (!g->running) return set_error(TTAD_ERR_INVALID, "graph_wait: not launched");
+    // The run's report arrives in pinned memory: a read of it costs no call into the runtime. It is watched closely for
+    // the first milliseconds (short runs) and every 50 us afterwards, when the stream is asked for errors too.
     auto t0 = std::chrono::steady_clock::now();
-    for (;;) {
-        hipError_t e = hipEventQuery(g->ev_stop);
-        if (e == hipSuccess) break;
-        if (e != hipErrorNotReady) {
+    auto waited = [&]() { return std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count(); };
+    while (__atomic_load_n(&g->report->seq, __ATOMIC_ACQUIRE) != g->seq) {
+        const double w = waited();
+        if (timeout_s > 0 && w > timeout_s)
+            return set_error(TTAD_ERR_TIMEOUT, "graph_wait: timed out after %.1f s (graph still running)", timeout_s);
+        if (w < 5e-3) continue;
+        const hipError_t e = hipStreamQuery(g->stream);
+        if (e != hipSuccess && e != hipErrorNotReady) {
             g->running = false;
             return set_error(TTAD_ERR_DEVICE, "graph_wait: %s", hipGetErrorString(e));
         }
-        if (timeout_s > 0 &&
-            std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count() > timeout_s)
-            return set_error(TTAD_ERR_TIMEOUT, "graph_wait: timed out after %.1f s (graph still running)", timeout_s);
         std::this_thread::sleep_for(std::chrono::microseconds(50));
     }
     g->running = false;
-    int done = 0, abort_code = 0;
-    TTAD_HIP(hipMemcpy(&done, g->d_done.p, 4, hipMemcpyDeviceToHost));
-    TTAD_HIP(hipMemcpy(&abort_code, g->d_abort.p, 4, hipMemcpyDeviceToHost));
+    const int done = g->report->done, abort_code = g->report->abort_code;
+    g->info = g->report->info;
+    TTAD_HIP(hipEventSynchronize(g->ev_stop));
     float ms = 0.f;
     TTAD_HIP(hipEventElapsedTime(&ms, g->ev_start, g->ev_stop));
     if (stats) {
@@ -968,12 +989,7 @@ int ttad_graph_wait(ttad_graph* g, double timeout_s, ttad_graph_stats* stats) {
                          g->total_items);
     if (done != g->total_items)
         return set_error(TTAD_ERR_DEVICE, "graph finished with %d of %d items", done, g->total_items);
-    for (auto* M : g->mats) {
-        if (!M) continue;
-        int h = 0;
-        TTAD_HIP(hipMemcpy(&h, M->info.p, 4, hipMemcpyDeviceToHost));
-        if (h) return set_error(TTAD_ERR_NOT_SPD, "graph: non-positive pivot at column %d", h);
-    }
+    if (g->info) return set_error(TTAD_ERR_NOT_SPD, "graph: non-positive pivot at column %d", g->info);
     return TTAD_OK;
 }
 
@@ -1066,7 +1082,8 @@ int ttad_graph_write_deps(ttad_graph* g, const char* path) {
 
 int ttad_graph_destroy(ttad_graph* g) {
     if (!g) return TTAD_OK;
-    if (g->running) (void)hipEventSynchronize(g->ev_stop);
+    if (g->running) (void)hipStreamSynchronize(g->stream);  // (its report kernel too)
+    if (g->report_slot >= 0) g->ctx->free_reports.push_back(g->report_slot);
     if (g->ev_start) (void)hipEventDestroy(g->ev_start);
     if (g->ev_stop) (void)hipEventDestroy(g->ev_stop);
     delete g;

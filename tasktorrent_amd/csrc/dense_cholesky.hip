@@ -182,7 +182,6 @@ static bool ensure_planes(ttad_matrix* M) {
 }
 
 int cholesky_persistent(ttad_context* ctx, ttad_matrix* M, int prio_kind, int prec, hipStream_t s, int* info) {
-    (void)info;
     const auto key = std::make_tuple(M->id, prio_kind, prec);
     ttad_graph* g = nullptr;
     auto it = ctx->chol_graphs.find(key);
@@ -206,7 +205,10 @@ int cholesky_persistent(ttad_context* ctx, ttad_matrix* M, int prio_kind, int pr
     if (rc != TTAD_OK) return rc;
     ttad_graph_stats st{};
     rc = ttad_graph_wait(g, 120.0, &st);
-    if (rc == TTAD_OK) ctx->kernel_s = st.elapsed_s;
+    if (rc == TTAD_OK || rc == TTAD_ERR_NOT_SPD) {
+        ctx->kernel_s = st.elapsed_s;
+        if (info) *info = g->info;
+    }
     return rc;
 }
 

@@ -24,13 +24,13 @@ struct DevGraph {
     int32_t n_tasks;
     int32_t n_buckets;
     int32_t total_items;
-    int32_t n_init;             // number of initially ready entries (prefilled queue slots)
     const DevTask* tasks;
     const DevEdge* edges;       // out-edges, by task
     const int32_t* deps0;       // initial dependency counters (indegree - host seeds)
     const int32_t* tail0;       // initial queue tails per bucket
-    const int64_t* init_items;  // [n_init] queue entries (task << 20) | item of the prefilled slots
-    const int32_t* init_slots;  // [n_init] their slots in q_items
+    const int64_t* q_items0;    // [total_items] initial queue entries: those of ready tasks, else -1
+    int32_t n_mats;
+    int32_t has_accum;          // some update runs in accumulate mode (the tile locks are cleared before a run)
     int32_t* deps;
     int32_t* items_left;
     int32_t* q_head;            // [n_buckets]
@@ -55,6 +55,13 @@ struct DevGraph {
 };
 
 constexpr int TRACE_WORDS = 6;  // u64 per trace record
+
+// What a finished run tells the host, in pinned memory; seq is written last.
+struct GraphReport {
+    int32_t done, abort_code;
+    int32_t info;  // of the first bound matrix with a non-positive pivot, else 0
+    int32_t seq;
+};
 
 // XCDs of the device (MI355X: 8 XCDs of 32 CUs, each with its own L2).
 constexpr int NXCD = 8;

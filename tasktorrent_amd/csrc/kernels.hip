@@ -306,10 +306,11 @@ __global__ __launch_bounds__(NTHREADS, vset_occupancy(VM)) void k_persistent(Dev
     }
 }
 
-// Restores the counters and queues of a graph so that it can run again.
-__global__ void k_graph_reset_a(DevGraph g, int n_slots) {
+// Restores the counters and queues of a graph, and clears the pivot reports, POTRF flags and locks of its matrices, so
+// that it can run (again).
+__global__ void k_graph_reset(DevGraph g, int n_slots) {
     const int stride = gridDim.x * blockDim.x;
-    for (int x = blockIdx.x * blockDim.x + threadIdx.x; x < n_slots; x += stride) g.q_items[x] = -1;
+    for (int x = blockIdx.x * blockDim.x + threadIdx.x; x < n_slots; x += stride) g.q_items[x] = g.q_items0[x];
     for (int x = blockIdx.x * blockDim.x + threadIdx.x; x < g.n_tasks; x += stride) {
         g.deps[x] = g.deps0[x];
         g.items_left[x] = g.tasks[x].n_items;
@@ -341,17 +342,31 @@ __global__ void k_graph_reset_a(DevGraph g, int n_slots) {
         g.cu_crit[x] = 0;
     }
     for (int x = blockIdx.x * blockDim.x + threadIdx.x; x < NXCD * 64; x += stride) g.idle_primary[x] = 0;
+    for (int q = 0; q < g.n_mats; q++) {
+        const DevMat& M = g.mats[q];
+        if (!M.info) continue;  // slot not bound
+        for (int x = blockIdx.x * blockDim.x + threadIdx.x; x < M.nt * M.pf_stride; x += stride) M.pflags[x] = 0;
+        if (g.has_accum)
+            for (long x = blockIdx.x * blockDim.x + threadIdx.x; x < (long)M.nt * M.nt * 16; x += stride) M.locks[x] = 0;
+        if (blockIdx.x == 0 && threadIdx.x == 0) *M.info = 0;
+    }
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         *g.done_items = 0;
         *g.abort_flag = 0;
         if (g.trace_cursor) *g.trace_cursor = 0;
     }
 }
-__global__ void k_graph_reset_b(DevGraph g) {
-    const int stride = gridDim.x * blockDim.x;
-    for (int x = blockIdx.x * blockDim.x + threadIdx.x; x < g.n_init; x += stride) {
-        g.q_items[g.init_slots[x]] = g.init_items[x];
-    }
+__global__ void k_graph_report(DevGraph g, GraphReport* out, int seq) {
+    if (threadIdx.x != 0) return;
+    int info = 0;
+    for (int q = 0; q < g.n_mats && info == 0; q++)
+        if (g.mats[q].info) info = *g.mats[q].info;
+    out->done = *g.done_items;
+    out->abort_code = *g.abort_flag;
+    out->info = info;
+    __atomic_thread_fence(__ATOMIC_RELEASE);  // system scope
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __hip_atomic_store(&out->seq, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // ---------------------------------------------------------------------------
@@ -614,8 +629,10 @@ __global__ void k_read_clock(uint64_t* out) {
 void launch_read_clock(uint64_t* out, hipStream_t s) { hipLaunchKernelGGL(k_read_clock, dim3(1), dim3(64), 0, s, out); }
 
 void launch_graph_reset(const DevGraph& g, int n_slots, hipStream_t s) {
-    hipLaunchKernelGGL(k_graph_reset_a, dim3(256), dim3(256), 0, s, g, n_slots);
-    hipLaunchKernelGGL(k_graph_reset_b, dim3(64), dim3(256), 0, s, g);
+    hipLaunchKernelGGL(k_graph_reset, dim3(256), dim3(256), 0, s, g, n_slots);
+}
+void launch_graph_report(const DevGraph& g, GraphReport* out, int seq, hipStream_t s) {
+    hipLaunchKernelGGL(k_graph_report, dim3(1), dim3(64), 0, s, g, out, seq);
 }
 
 void launch_persistent(int vset, const DevGraph& g, int n_workers, hipStream_t s) {

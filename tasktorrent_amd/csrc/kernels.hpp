@@ -6,6 +6,7 @@
 namespace ttad {
 
 struct DevGraph;
+struct GraphReport;
 
 hipError_t kernels_init();
 // Resident persistent workers per CU of an executor instantiation (index into the variant sets).
@@ -14,6 +15,8 @@ int persistent_blocks_per_cu(int vset);
 void launch_items(int vset, const DevMat* mats, const DevTask* tasks, const int32_t* prefix, int n_tasks,
                   int n_items, int32_t* err, hipStream_t s);
 void launch_graph_reset(const DevGraph& g, int n_slots, hipStream_t s);
+// Writes the report of a finished run to pinned host memory (its device address).
+void launch_graph_report(const DevGraph& g, GraphReport* out, int seq, hipStream_t s);
 // Writes the device wall clock (wall_clock64) to *out.
 void launch_read_clock(uint64_t* out, hipStream_t s);
 void launch_persistent(int vset, const DevGraph& g, int n_workers, hipStream_t s);

@@ -4,6 +4,7 @@
 
 #include <cstdarg>
 #include <cstdio>
+#include <cstring>
 #include <map>
 #include <memory>
 #include <string>
@@ -52,6 +53,27 @@ struct DevBuf {
     template <class T> T* as() const { return static_cast<T*>(p); }
 };
 
+// Small pinned, device-visible host memory owned by a handle.
+struct PinnedBuf {
+    void* host = nullptr;
+    void* dev = nullptr;
+    PinnedBuf() = default;
+    PinnedBuf(const PinnedBuf&) = delete;
+    PinnedBuf& operator=(const PinnedBuf&) = delete;
+    ~PinnedBuf() {
+        if (host) (void)hipHostFree(host);
+    }
+    hipError_t alloc(size_t b) {
+        hipError_t e = hipHostMalloc(&host, b, hipHostMallocMapped | hipHostMallocCoherent);
+        if (e != hipSuccess) {
+            host = nullptr;
+            return e;
+        }
+        memset(host, 0, b);
+        return hipHostGetDevicePointer(&dev, host, 0);
+    }
+};
+
 struct StreamPlan;  // cached host-sequenced schedule
 
 }  // namespace ttad
@@ -76,6 +98,11 @@ struct ttad_context {
     hipEvent_t ev_a = nullptr, ev_b = nullptr;  // bracket the last ttad_potrf_tiled on its stream
     bool ev_valid = false;
     double kernel_s = -1.0;  // event time of the last persistent factorization kernel (< 0: stream schedule)
+    // reports of finished graph runs: slots of pinned memory, one per graph (graphs beyond them allocate their own)
+    static constexpr int REPORT_SLOTS = 256;
+    ttad::PinnedBuf reports;
+    std::vector<int> free_reports;
+    ttad::PinnedBuf readback;  // 4 KB for small results that a call waits for (a copy to pageable memory is staged)
     // solve-phase workspace (grown on demand)
     ttad::DevBuf sw_Y, sw_D, sw_P, sw_R, sw_flags, sw_ticket, sw_err, sw_norms, sw_part;
     // options (ttad_set_option)
@@ -120,9 +147,15 @@ struct ttad_graph {
     bool with_planes = false;  // hand the matrices' bf16 planes to the items (a full Cholesky PTG only)
     std::vector<int32_t> spin_us;  // per task: spin time of a TTAD_SPIN task (microseconds)
     bool seeds_dirty = true, mats_dirty = true, running = false;
-    ttad::DevBuf d_tasks, d_edges, d_deps0, d_tail0, d_init, d_init_slot, d_deps, d_items_left, d_gops, d_q_head, d_q_tail, d_q_count, d_xcd_run,
+    ttad::DevBuf d_tasks, d_edges, d_deps0, d_tail0, d_q_items0, d_deps, d_items_left, d_gops, d_q_head, d_q_tail, d_q_count, d_xcd_run,
         d_q_base, d_q_home, d_q_items, d_done, d_abort, d_mats, d_trace, d_trace_cursor, d_cu_slots;
-    int n_init = 0;
+    bool has_accum = false;
+    // this graph's report slot (-1: its own pinned buffer), and the number of runs launched
+    int report_slot = -1;
+    ttad::PinnedBuf own_report;
+    ttad::GraphReport *report = nullptr, *report_dev = nullptr;
+    int seq = 0;
+    int info = 0;  // of the last run: the first non-positive pivot of a bound matrix, else 0
     int workers = 0;
     int vset = 4;  // executor instantiation (index into the item-variant sets) covering the graph
     bool traced = false;

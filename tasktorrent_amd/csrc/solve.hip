@@ -319,11 +319,10 @@ static int residual(ttad_context* ctx, ttad_matrix* A, int nrhs, const double* B
         hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(128), 0, s, norms, 3 * 32 + 8);
         hipLaunchKernelGGL((k_residual<16>), dim3(t.P), dim3(NTHREADS), 0, s, Md, t, B, ldb, X, ldx, R, ldr, 1,
                            norms, 1);
-        unsigned long long h = 0;
-        TTAD_HIP(hipMemcpyAsync(&h, norms, 8, hipMemcpyDeviceToHost, s));
+        TTAD_HIP(hipMemcpyAsync(ctx->readback.host, norms, 8, hipMemcpyDeviceToHost, s));
         TTAD_HIP(hipStreamSynchronize(s));
         double v;
-        memcpy(&v, &h, 8);
+        memcpy(&v, ctx->readback.host, 8);
         A->anorm = v;
         A->anorm_valid = true;
     }
@@ -368,8 +367,8 @@ static int residual(ttad_context* ctx, ttad_matrix* A, int nrhs, const double* B
                                Xc, ldx, Rc, ldr, nc, norms);
         }
         TTAD_HIP(hipGetLastError());
-        unsigned long long h[3 * 32];
-        TTAD_HIP(hipMemcpyAsync(h, norms, sizeof(unsigned long long) * 3 * nc, hipMemcpyDeviceToHost, s));
+        const unsigned long long* h = (const unsigned long long*)ctx->readback.host;
+        TTAD_HIP(hipMemcpyAsync(ctx->readback.host, norms, sizeof(unsigned long long) * 3 * nc, hipMemcpyDeviceToHost, s));
         TTAD_HIP(hipStreamSynchronize(s));
         for (int j = 0; j < nc; j++) {
             double rn, xn, bn;
@@ -386,10 +385,9 @@ static int residual(ttad_context* ctx, ttad_matrix* A, int nrhs, const double* B
 }
 
 static int check_err_flag(ttad_context* ctx, hipStream_t s) {
-    int32_t e = 0;
-    TTAD_HIP(hipMemcpyAsync(&e, ctx->sw_err.p, 4, hipMemcpyDeviceToHost, s));
+    TTAD_HIP(hipMemcpyAsync(ctx->readback.host, ctx->sw_err.p, 4, hipMemcpyDeviceToHost, s));
     TTAD_HIP(hipStreamSynchronize(s));
-    if (e) {  // cleared for the next call: a set flag also makes every device wait give up at once
+    if (*(const int32_t*)ctx->readback.host) {  // cleared for the next call: a set flag also makes every device wait give up at once
         TTAD_HIP(hipMemsetAsync(ctx->sw_err.p, 0, 4, s));
         TTAD_HIP(hipStreamSynchronize(s));
         return set_error(TTAD_ERR_TIMEOUT, "solve: a sweep block waited past the device watchdog");
@@ -417,11 +415,10 @@ static int refine(ttad_context* ctx, ttad_matrix* A, ttad_matrix* L, int nrhs, c
         hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(128), 0, s, norms, 1);
         hipLaunchKernelGGL(k_absmax_cols, dim3(256), dim3(256), 0, s, B, ldb, n, nrhs, norms);
         TTAD_HIP(hipGetLastError());
-        unsigned long long h = 0;
-        TTAD_HIP(hipMemcpyAsync(&h, norms, 8, hipMemcpyDeviceToHost, s));
+        TTAD_HIP(hipMemcpyAsync(ctx->readback.host, norms, 8, hipMemcpyDeviceToHost, s));
         TTAD_HIP(hipStreamSynchronize(s));
         double bmax;
-        memcpy(&bmax, &h, 8);
+        memcpy(&bmax, ctx->readback.host, 8);
         eta = std::isnan(bmax) ? INFINITY : (bmax > 0 ? 1.0 : 0.0);
     }
     while (eta > tol && it < max_iter) {
