@@ -769,10 +769,21 @@ static int graph_prepare(ttad_graph* g) {
         };
         for (auto& x : g->tasks)
             if (x.kind == K_GEMM || x.kind == K_SYRK) step_items[{x.mat, x.k}] += update_items(x, GEMM_BM);
+        // FP64: with more than 128 update items per CU in all the updates' throughput bounds the run and TRSM keeps its
+        // higher strips (n = 16384, b = 512, 374 per CU: 29.3 ms, 31.0 with the LDS form on the longest path and in
+        // the small steps); below, the chain does (n = 8192, 49 per CU: 5.4 and 5.2 ms).
+        long long update_total = 0;
+        for (auto& kv : step_items) update_total += kv.second;
+        const bool throughput = update_total > 128LL * g->ctx->n_cu;
         for (auto& x : g->tasks) {
             x.sub = GEMM_BM;
             if ((x.kind == K_GEMM || x.kind == K_SYRK) && !x.accum &&
                 (x.crit || 2 * step_items[{x.mat, x.k}] <= g->ctx->n_cu))
+                x.sub = GEMM_BS;
+            if (x.kind == K_TRSM && x.mat < (int)g->mats.size() && g->mats[x.mat] && x.j >= 0 && x.j < g->mats[x.mat]->nt &&
+                g->mats[x.mat]->bsz[x.j] <= TRSM_LDS_COLS &&
+                (g->mats[x.mat]->storage != P_F64 ||
+                 (!throughput && (x.crit || 2 * step_items[{x.mat, x.j}] <= g->ctx->n_cu))))
                 x.sub = GEMM_BS;
         }
         for (int t = 0; t < n; t++) {
@@ -796,7 +807,8 @@ static int graph_prepare(ttad_graph* g) {
         }
         int needed = 0;
         for (auto& x : g->tasks)
-            if (x.kind != K_NOP) needed |= item_variant(x.kind, x.prec, g->mats[x.mat]->storage) | (x.accum ? V_ACC : 0);
+            if (x.kind != K_NOP) needed |= item_variant(x.kind, x.prec, g->mats[x.mat]->storage) | (x.accum ? V_ACC : 0) |
+                                            (x.kind == K_TRSM && x.sub == GEMM_BS ? V_TLDS : 0);
         g->vset = vset_index(needed);
         g->has_accum = (needed & V_ACC) != 0;
         g->bucket_items.assign(g->n_buckets, 0);

@@ -116,12 +116,16 @@ enum ItemVariant : int {
     V_G32 = 4,       // GEMM/SYRK FP32
     V_GBF16 = 8,     // GEMM/SYRK BF16
     V_GBF16X3 = 16,  // GEMM/SYRK BF16x3
-    V_ALL = 31,
+    V_TLDS = 64,     // TRSM with the solved columns in LDS
     V_ACC = 32       // accumulate-mode GEMM/SYRK (only in the last set, so the others keep their registers)
 };
 // The compiled sets, smallest first.
-constexpr int N_VSETS = 6;
-constexpr int VSETS[N_VSETS] = {V_F64S, V_F32S | V_G32, V_F32S | V_GBF16, V_F32S | V_GBF16X3, V_ALL, V_ALL | V_ACC};
+// (FP64 tiles have two: the TRSM form in LDS, present in the kernel though no task uses it, makes the large
+// FP64 factorizations 5 % slower, n = 16384: 29.3 against 31.0 ms; why is not known.)
+constexpr int V_ALL = V_F64S | V_F32S | V_G32 | V_GBF16 | V_GBF16X3 | V_TLDS;
+constexpr int N_VSETS = 7;
+constexpr int VSETS[N_VSETS] = {V_F64S, V_F64S | V_TLDS, V_F32S | V_G32 | V_TLDS, V_F32S | V_GBF16 | V_TLDS,
+                                V_F32S | V_GBF16X3 | V_TLDS, V_ALL, V_ALL | V_ACC};
 
 __host__ __device__ inline int item_variant(int kind, int prec, int storage) {
     if (kind == K_GEMM || kind == K_SYRK)
@@ -134,6 +138,8 @@ constexpr int vset_lds(int vm) {
     if (vm & V_F64S) b = cmax(b, cmax(cmax(LDS_GEMM_F64, LDS_POTRF), LDS_TRSM));
     if (vm & V_F64S) b = cmax(b, gemm_item_lds<double, P_F64, GEMM_BS>());
     if (vm & V_G32) b = cmax(b, gemm_item_lds<float, P_F32, GEMM_BS>());
+    if ((vm & V_TLDS) && (vm & V_F64S)) b = cmax(b, trsm_lds_bytes<double>());
+    if ((vm & V_TLDS) && (vm & V_F32S)) b = cmax(b, trsm_lds_bytes<float>());
     if (vm & V_F32S) b = cmax(b, cmax(LDS_POTRF, LDS_TRSM_F32));
     if (vm & V_G32) b = cmax(b, LDS_GEMM_F32);
     if (vm & V_GBF16) b = cmax(b, LDS_GEMM_BF16_1);
@@ -188,13 +194,22 @@ __device__ __attribute__((noinline)) void gemm_small_call(const TS* A, const TS*
                                  lds_uniform(lds), wave_uniform(PA), wave_uniform(PB));
     __builtin_amdgcn_s_setprio(0);
 }
-template <typename TS, typename TC, int VM>
-__device__ __attribute__((noinline)) void trsm_call(const TS* L, long ldl, const double* dinv, TS* X, long ldx, int m,
-                                                    int n, int r0, char* lds, void* planes) {
+template <typename TS, int VM>
+__device__ __attribute__((noinline)) void trsm_call(const TS* L, const double* dinv, TS* X, int m, int n, int it,
+                                                    bool in_lds, char* lds, void* planes) {
     __builtin_amdgcn_s_setprio(3);
-    item_trsm<TS, TC>(wave_uniform(L), wave_uniform((int)ldl), wave_uniform(dinv), wave_uniform(X),
-                      wave_uniform((int)ldx), wave_uniform(m), wave_uniform(n), wave_uniform(r0), lds_uniform(lds),
-                      wave_uniform(planes));
+    const int mu = wave_uniform(m), nu = wave_uniform(n), iu = wave_uniform(it);
+    char* l = lds_uniform(lds);
+    bool done = false;
+    if constexpr ((VM & V_TLDS) != 0)
+        if (wave_uniform((int)in_lds)) {
+            item_trsm_lds<TS>(wave_uniform(L), nu, wave_uniform(dinv), wave_uniform(X), mu, mu, nu,
+                              iu * trsm_rows(sizeof(TS), true), l, wave_uniform(planes));
+            done = true;
+        }
+    if (!done)
+        item_trsm<TS, TS>(wave_uniform(L), nu, wave_uniform(dinv), wave_uniform(X), mu, mu, nu,
+                          iu * trsm_rows(sizeof(TS), false), l, wave_uniform(planes));
     __builtin_amdgcn_s_setprio(0);
 }
 
@@ -239,16 +254,18 @@ __device__ __forceinline__ bool exec_item(const DevTask& t, int it, const DevMat
         }
         case K_TRSM: {
             const int i = t.i, j = t.j, m = M.bsz[i], n = M.bsz[j];
+            const bool in_lds = t.sub == GEMM_BS;
+            if ((VM & V_TLDS) == 0 && in_lds) return false;
             if constexpr ((VM & V_F64S) != 0)
                 if (f64s) {
-                    trsm_call<double, double, VM>((const double*)tile(j, j), n, M.dinv[j], (double*)tile(i, j), m, m, n,
-                                              it * trsm_rows(8), lds, nullptr);
+                    trsm_call<double, VM>((const double*)tile(j, j), M.dinv[j], (double*)tile(i, j), m, n, it, in_lds, lds,
+                                        nullptr);
                     return true;
                 }
             if constexpr ((VM & V_F32S) != 0)
                 if (!f64s) {
-                    trsm_call<float, float, VM>((const float*)tile(j, j), n, M.dinv[j], (float*)tile(i, j), m, m, n,
-                                            it * trsm_rows(4), lds, planes(i, j));
+                    trsm_call<float, VM>((const float*)tile(j, j), M.dinv[j], (float*)tile(i, j), m, n, it, in_lds, lds,
+                                        planes(i, j));
                     return true;
                 }
             return false;

@@ -390,11 +390,17 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_raw_potrf(TS* A, long lda, int 
     item_potrf<TS>(A, lda, n, dinv, info, 0, blockIdx.x, flags, err, (int64_t)500000000, lds);
 }
 
-template <typename TS, typename TC>
-__global__ __launch_bounds__(NTHREADS) void k_raw_trsm(const TS* L, long ldl, const double* dinv, TS* X, long ldx,
-                                                       int m, int n) {
+// IN_LDS: the form that keeps the solved columns in LDS.
+template <typename TS, bool IN_LDS> constexpr int raw_trsm_lds() {
+    return IN_LDS ? trsm_lds_bytes<TS>() : sizeof(TS) == 8 ? LDS_TRSM : LDS_TRSM_F32;
+}
+template <typename TS, bool IN_LDS>
+__global__ __launch_bounds__(NTHREADS, 2) void k_raw_trsm(const TS* L, long ldl, const double* dinv, TS* X, long ldx,
+                                                          int m, int n) {
     extern __shared__ __align__(16) char lds[];
-    item_trsm<TS, TC>(L, ldl, dinv, X, ldx, m, n, blockIdx.x * trsm_rows(sizeof(TS)), lds);
+    const int r0 = blockIdx.x * trsm_rows(sizeof(TS), IN_LDS);
+    if constexpr (IN_LDS) item_trsm_lds<TS>(L, ldl, dinv, X, ldx, m, n, r0, lds);
+    else item_trsm<TS, TS>(L, ldl, dinv, X, ldx, m, n, r0, lds);
 }
 
 // Inverses of the 64x64 diagonal blocks of a lower-triangular n x n L (one block per workgroup).
@@ -556,12 +562,14 @@ hipError_t kernels_init() {
     TTAD_SETLDS2(k_items<VSETS[2]>, vset_lds(VSETS[2]));
     TTAD_SETLDS2(k_items<VSETS[3]>, vset_lds(VSETS[3]));
     TTAD_SETLDS2(k_items<VSETS[4]>, vset_lds(VSETS[4]));
+    TTAD_SETLDS2(k_items<VSETS[5]>, vset_lds(VSETS[5]));
     TTAD_SETLDS2(k_persistent<VSETS[0]>, vset_lds(VSETS[0]));
     TTAD_SETLDS2(k_persistent<VSETS[1]>, vset_lds(VSETS[1]));
     TTAD_SETLDS2(k_persistent<VSETS[2]>, vset_lds(VSETS[2]));
     TTAD_SETLDS2(k_persistent<VSETS[3]>, vset_lds(VSETS[3]));
     TTAD_SETLDS2(k_persistent<VSETS[4]>, vset_lds(VSETS[4]));
     TTAD_SETLDS2(k_persistent<VSETS[5]>, vset_lds(VSETS[5]));
+    TTAD_SETLDS2(k_persistent<VSETS[6]>, vset_lds(VSETS[6]));
 #define TTAD_SETLDS_GEMM(ts, prec)                                                                        \
     TTAD_SETLDS2((k_raw_gemm<ts, prec, GEMM_BM>), (gemm_item_lds<ts, prec, GEMM_BM>()));                   \
     TTAD_SETLDS2((k_raw_gemm<ts, prec, GEMM_BS>), (gemm_item_lds<ts, prec, GEMM_BS>()))
@@ -572,8 +580,10 @@ hipError_t kernels_init() {
 #undef TTAD_SETLDS_GEMM
     TTAD_SETLDS2((k_raw_potrf<double>), LDS_POTRF);
     TTAD_SETLDS2((k_raw_potrf<float>), LDS_POTRF);
-    TTAD_SETLDS2((k_raw_trsm<double, double>), LDS_TRSM);
-    TTAD_SETLDS2((k_raw_trsm<float, float>), LDS_TRSM_F32);
+    TTAD_SETLDS2((k_raw_trsm<double, true>), (raw_trsm_lds<double, true>()));
+    TTAD_SETLDS2((k_raw_trsm<double, false>), (raw_trsm_lds<double, false>()));
+    TTAD_SETLDS2((k_raw_trsm<float, true>), (raw_trsm_lds<float, true>()));
+    TTAD_SETLDS2((k_raw_trsm<float, false>), (raw_trsm_lds<float, false>()));
 #undef TTAD_SETLDS2
     return e;
 }
@@ -585,7 +595,8 @@ static const void* persistent_fn(int vset) {
         case 2: return (const void*)k_persistent<VSETS[2]>;
         case 3: return (const void*)k_persistent<VSETS[3]>;
         case 4: return (const void*)k_persistent<VSETS[4]>;
-        default: return (const void*)k_persistent<VSETS[5]>;
+        case 5: return (const void*)k_persistent<VSETS[5]>;
+        default: return (const void*)k_persistent<VSETS[6]>;
     }
 }
 
@@ -596,7 +607,8 @@ static int vset_lds_of(int vset) {
         case 2: return vset_lds(VSETS[2]);
         case 3: return vset_lds(VSETS[3]);
         case 4: return vset_lds(VSETS[4]);
-        default: return vset_lds(VSETS[5]);
+        case 5: return vset_lds(VSETS[5]);
+        default: return vset_lds(VSETS[6]);
     }
 }
 
@@ -619,7 +631,8 @@ void launch_items(int vset, const DevMat* mats, const DevTask* tasks, const int3
         case 1: hipLaunchKernelGGL(k_items<VSETS[1]>, grid, block, lds, s, mats, tasks, prefix, n_tasks, err); break;
         case 2: hipLaunchKernelGGL(k_items<VSETS[2]>, grid, block, lds, s, mats, tasks, prefix, n_tasks, err); break;
         case 3: hipLaunchKernelGGL(k_items<VSETS[3]>, grid, block, lds, s, mats, tasks, prefix, n_tasks, err); break;
-        default: hipLaunchKernelGGL(k_items<VSETS[4]>, grid, block, lds, s, mats, tasks, prefix, n_tasks, err); break;
+        case 4: hipLaunchKernelGGL(k_items<VSETS[4]>, grid, block, lds, s, mats, tasks, prefix, n_tasks, err); break;
+        default: hipLaunchKernelGGL(k_items<VSETS[5]>, grid, block, lds, s, mats, tasks, prefix, n_tasks, err); break;
     }
 }
 
@@ -644,7 +657,8 @@ void launch_persistent(int vset, const DevGraph& g, int n_workers, hipStream_t s
         case 2: hipLaunchKernelGGL(k_persistent<VSETS[2]>, grid, block, lds, s, g); break;
         case 3: hipLaunchKernelGGL(k_persistent<VSETS[3]>, grid, block, lds, s, g); break;
         case 4: hipLaunchKernelGGL(k_persistent<VSETS[4]>, grid, block, lds, s, g); break;
-        default: hipLaunchKernelGGL(k_persistent<VSETS[5]>, grid, block, lds, s, g); break;
+        case 5: hipLaunchKernelGGL(k_persistent<VSETS[5]>, grid, block, lds, s, g); break;
+        default: hipLaunchKernelGGL(k_persistent<VSETS[6]>, grid, block, lds, s, g); break;
     }
 }
 
@@ -693,17 +707,20 @@ void launch_trtri_diag(int prec, const void* L, long ldl, int n, double* dinv, h
         hipLaunchKernelGGL((k_trtri_diag<float>), dim3(nb), dim3(NTHREADS), 0, s, (const float*)L, ldl, n, dinv);
 }
 
+template <typename TS, bool IN_LDS>
+static void raw_trsm(const void* L, long ldl, const double* dinv, void* X, long ldx, int m, int n, hipStream_t s) {
+    const int bm = trsm_rows(sizeof(TS), IN_LDS);
+    hipLaunchKernelGGL((k_raw_trsm<TS, IN_LDS>), dim3((m + bm - 1) / bm), dim3(NTHREADS),
+                       (raw_trsm_lds<TS, IN_LDS>()), s, (const TS*)L, ldl, dinv, (TS*)X, ldx, m, n);
+}
+
 void launch_raw_trsm(int prec, const void* L, long ldl, const double* dinv, void* X, long ldx, int m, int n,
                      hipStream_t s) {
-    const int bm = trsm_rows(prec == P_F64 ? 8 : 4);
-    const int items = (m + bm - 1) / bm;
-    if (items <= 0) return;
-    if (prec == P_F64)
-        hipLaunchKernelGGL((k_raw_trsm<double, double>), dim3(items), dim3(NTHREADS), LDS_TRSM, s,
-                           (const double*)L, ldl, dinv, (double*)X, ldx, m, n);
-    else
-        hipLaunchKernelGGL((k_raw_trsm<float, float>), dim3(items), dim3(NTHREADS), LDS_TRSM_F32, s, (const float*)L,
-                           ldl, dinv, (float*)X, ldx, m, n);
+    if (m <= 0) return;
+    const bool in_lds = n <= TRSM_LDS_COLS && ldl < TRSM_LDS_MAX_LD && ldx < TRSM_LDS_MAX_LD;
+    auto* f = prec == P_F64 ? (in_lds ? raw_trsm<double, true> : raw_trsm<double, false>)
+                            : (in_lds ? raw_trsm<float, true> : raw_trsm<float, false>);
+    f(L, ldl, dinv, X, ldx, m, n, s);
 }
 
 static dim3 conv_grid(int nt, int max_b) { return dim3(nt, nt, (std::max(1, max_b) + CONV_COLS - 1) / CONV_COLS); }

@@ -1258,7 +1258,7 @@ __device__ __forceinline__ void item_potrf(TS* __restrict__ A, long lda, int n, 
 }
 
 // ---------------------------------------------------------------------------
-// TRSM work item: rows [r0, r0+trsm_rows(sizeof(TS))) of X (m x n) := X L^{-T} (Right, Lower,
+// TRSM work item: trsm_rows(sizeof(TS), false) rows of X (m x n) := X L^{-T} (Right, Lower,
 // Trans, NonUnit), in place, by 64-column blocks: the block's right-hand side goes
 // into the accumulators, the already solved columns times L's off-diagonal blocks
 // are subtracted (one GEMM), and the result is multiplied by the inverse of L's
@@ -1272,7 +1272,7 @@ template <typename TS, typename TC>
 __device__ __forceinline__ void item_trsm(const TS* __restrict__ L, long ldl, const double* __restrict__ dinv, TS* __restrict__ X,
                           long ldx, int m, int n, int r0, char* lds, void* planes = nullptr) {
     constexpr bool VEC = std::is_same<TS, TC>::value;
-    constexpr int BMT = trsm_rows(sizeof(TS));
+    constexpr int BMT = trsm_rows(sizeof(TS), false);
     using G = GemmNT<TS, TS, TC, BMT, DB, trsm_bk<TS>(), VEC, true>;  // update from the solved columns
     using G3 = GemmNT<TC, TC, TC, BMT, DB, DB, false, true>;  // times Dinv^T, both operands in LDS
     const int mv = min(BMT, m - r0);
@@ -1350,6 +1350,130 @@ __device__ __forceinline__ void item_trsm(const TS* __restrict__ L, long ldl, co
     }
 }
 
+// ---------------------------------------------------------------------------
+// TRSM work item for n <= TRSM_LDS_COLS columns: trsm_rows(sizeof(TS), true) rows of X := X L^{-T}, in place. The solved
+// columns stay in LDS (Xs[k][m]), where the next columns' products read them; L's blocks go from the L2 straight into
+// MFMA operands (a lane's element L(c, k), 128-byte segments), three chunks of 64 columns ahead: they do not depend on
+// the solve, so the loads run through its serial steps. Per 64-column block: wave w forms columns 16w .. 16w+15 of
+//   -t = -rhs + Xs L(block, 0:c0)^T, exchanged through LDS, then x = t Dinv^T (Dinv lower triangular)
+// with two barriers; sums in the order of item_trsm, so both forms give the same bits. What bounds it: the MFMAs of one
+// strip (512 columns in FP64: 12 us) and the exchanges. 256 columns 31 -> 17 us, 512 columns 90 -> 42 us (FP64, idle CUs).
+// Which TRSM tasks take it: the strip is half as high as item_trsm's, so L is read twice as often; FP32 tasks gain at
+// every size (bf16x3 n = 16384: 10.8 -> 9.0 ms), FP64 ones while the chain bounds the run (graph_prepare).
+// ---------------------------------------------------------------------------
+constexpr int TRSM_RING = 3;  // chunks of L in flight
+constexpr long TRSM_LDS_MAX_LD = 1 << 24;  // 32-bit byte offsets of 16 columns
+template <typename TS>
+__device__ __forceinline__ void item_trsm_lds(const TS* __restrict__ L, long ldl, const double* __restrict__ dinv,
+                                              TS* __restrict__ X, long ldx, int m, int n, int r0, char* lds,
+                                              void* planes = nullptr) {
+    typedef Mfma<TS> MF;
+    typedef typename MF::acc_t acc_t;
+    constexpr int RM = trsm_rows(sizeof(TS), true), RB = RM / 16;  // rows of the item, 16-row blocks
+    const int mv = min(RM, m - r0);
+    if (mv <= 0) return;
+    TS* Xs = reinterpret_cast<TS*>(lds);     // Xs[k * RM + m]
+    TS* Ts = Xs + TRSM_LDS_COLS * RM;        // the exchanged block, Ts[k * RM + m]
+    const int lane = threadIdx.x & 63, w = wave_uniform((int)threadIdx.x >> 6), l15 = lane & 15, kl = lane >> 4;
+    const int nblk = (n + DB - 1) / DB;
+    TTAD_GLOBAL TS* Xg = gmem(X) + r0;
+    TS bq[TRSM_RING][16];
+    // Element `off` bytes behind a uniform pointer: a scalar base and a 32-bit lane offset, no 64-bit lane address per
+    // load (leading dimensions are below TRSM_LDS_MAX_LD).
+    auto at = [](auto* base, unsigned off) {
+        using T = typename std::remove_cv<typename std::remove_pointer<decltype(base)>::type>::type;
+        return *reinterpret_cast<const TTAD_GLOBAL T*>(reinterpret_cast<const TTAD_GLOBAL char*>(gmem(base)) + off);
+    };
+    const unsigned lds_k = (unsigned)kl * (unsigned)ldl;  // this lane's k offset in L
+    // chunk kc of block cb into ring slot q: lane's elements L(64 cb + 16 w + l15, 64 kc + 4 ks + kl)
+    auto fetch = [&](TS (&b)[16], int cb, int kc) {
+        const unsigned off = ((unsigned)min(cb * DB + 16 * w + l15, n - 1) + lds_k) * (unsigned)sizeof(TS);
+#pragma unroll
+        for (int ks = 0; ks < 16; ks++) b[ks] = at(L + (long)(kc * DB + 4 * ks) * ldl, off);
+    };
+    auto fetch_block = [&](int cb) {
+#pragma unroll
+        for (int q = 0; q < TRSM_RING; q++)
+            if (q < cb) fetch(bq[q], cb, q);
+    };
+    TS rhs[RB][4];  // the right-hand side block of the next column block (result layout)
+    auto fetch_rhs = [&](int cb) {
+        const int c0 = cb * DB, cw = min(DB, n - c0);
+#pragma unroll
+        for (int a = 0; a < RB; a++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                rhs[a][r] = at(X + r0 + (long)c0 * ldx, ((unsigned)min(16 * a + l15, mv - 1) +
+                                                         (unsigned)min(16 * w + MF::row(lane, r), cw - 1) * (unsigned)ldx) *
+                                                            (unsigned)sizeof(TS));
+    };
+    fetch_rhs(0);
+    for (int cb = 0; cb < nblk; cb++) {
+        const int c0 = cb * DB, cw = min(DB, n - c0);
+        double dv[16];  // Dinv(16 w + l15, 4 ks + kl); zero above the diagonal
+#pragma unroll
+        for (int ks = 0; ks < 16; ks++)
+            dv[ks] = at(dinv + (long)cb * DB * DB + 4 * ks * DB, (unsigned)(16 * w + l15 + kl * DB) * 8u);
+        acc_t acc[RB];
+#pragma unroll
+        for (int a = 0; a < RB; a++) acc[a] = acc_t{-rhs[a][0], -rhs[a][1], -rhs[a][2], -rhs[a][3]};
+        if (cb + 1 < nblk) fetch_rhs(cb + 1);
+        auto product = [&](const TS (&b)[16], const TS* A) {
+#pragma unroll
+            for (int ks = 0; ks < 16; ks++)
+#pragma unroll
+                for (int a = 0; a < RB; a++)
+                    acc[a] = MF::mma(b[ks], A[(4 * ks + kl) * RM + 16 * a + l15], acc[a]);
+        };
+        for (int kc = 0; kc < cb; kc += TRSM_RING)
+#pragma unroll
+            for (int q = 0; q < TRSM_RING; q++)
+                if (kc + q < cb) {
+                    product(bq[q], Xs + (kc + q) * DB * RM);
+                    if (kc + q + TRSM_RING < cb) fetch(bq[q], cb, kc + q + TRSM_RING);
+                }
+        if (cb + 1 < nblk) fetch_block(cb + 1);
+#pragma unroll
+        for (int a = 0; a < RB; a++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                Ts[(16 * w + MF::row(lane, r)) * RM + 16 * a + l15] = -acc[a][r];
+        __syncthreads();
+#pragma unroll
+        for (int a = 0; a < RB; a++) acc[a] = acc_t{0, 0, 0, 0};
+        TS db[16];
+#pragma unroll
+        for (int ks = 0; ks < 16; ks++) db[ks] = (TS)dv[ks];
+#pragma unroll
+        for (int ks = 0; ks < 16; ks++)
+            if (ks < 4 * (w + 1)) {
+#pragma unroll
+                for (int a = 0; a < RB; a++)
+                    acc[a] = MF::mma(db[ks], Ts[(4 * ks + kl) * RM + 16 * a + l15], acc[a]);
+            }
+#pragma unroll
+        for (int a = 0; a < RB; a++) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int cc = 16 * w + MF::row(lane, r);
+                Xs[(c0 + cc) * RM + 16 * a + l15] = acc[a][r];
+                if (16 * a + l15 < mv && cc < cw) Xg[16 * a + l15 + (long)(c0 + cc) * ldx] = acc[a][r];
+            }
+            if constexpr (std::is_same<TS, float>::value) {
+                // a lane holds 4 consecutive columns of one row (cw is a multiple of 32 where there are planes)
+                const int cc = 16 * w + MF::row(lane, 0);
+                if (planes && 16 * a + l15 < mv && cc < cw)
+                    store_split4(static_cast<unsigned short*>(planes), (int)ldx, r0 + 16 * a + l15, c0 + cc, acc[a]);
+            }
+        }
+        __syncthreads();
+    }
+}
+
+template <typename TS> constexpr int trsm_lds_bytes() {
+    return (TRSM_LDS_COLS + DB) * trsm_rows(sizeof(TS), true) * (int)sizeof(TS);
+}
+
 // LDS bytes each item kind needs (the executor reserves the maximum).
 constexpr int LDS_GEMM_F64 = GemmNT<double, double, double, GEMM_BM, GEMM_BM, gemm_bk<double>(), true, true>::LDS_BYTES;
 constexpr int LDS_GEMM_F32 = GemmNT<float, float, float, GEMM_BM, GEMM_BM, gemm_bk<float>(), true, true>::LDS_BYTES;
@@ -1368,6 +1492,7 @@ constexpr int LDS_TRSM = cmax(GemmNT<double, double, double, TRSM_BM, DB, 32, tr
 constexpr int LDS_TRSM_F32 = cmax(GemmNT<float, float, float, TRSM_BM_F32, DB, trsm_bk<float>(), true, true>::LDS_BYTES,
                                   GemmNT<float, float, float, TRSM_BM_F32, DB, DB, false, true>::STAGE * 4);
 constexpr int LDS_ITEM_MAX =
-    cmax(cmax(cmax(LDS_GEMM_F64, LDS_GEMM_F32), cmax(LDS_GEMM_BF16, LDS_POTRF)), LDS_TRSM);
+    cmax(cmax(cmax(LDS_GEMM_F64, LDS_GEMM_F32), cmax(LDS_GEMM_BF16, LDS_POTRF)),
+         cmax(LDS_TRSM, cmax(trsm_lds_bytes<double>(), trsm_lds_bytes<float>())));
 
 }  // namespace ttad

@@ -12,9 +12,14 @@ enum Prec : int32_t { P_F64 = 0, P_F32 = 1, P_BF16 = 2, P_BF16X3 = 3 };
 constexpr int NTHREADS = 256;  // one workgroup = 4 wave64
 constexpr int GEMM_BM = 128;   // GEMM/SYRK work item = 128x128 output sub-tile
 constexpr int GEMM_BS = 64;    // or a 64x64 one, where the items of 128 leave CUs idle (DevTask::sub)
-constexpr int TRSM_BM = 32;      // TRSM work item of an FP64 tile: 32-row block (its latency is on the critical path)
-constexpr int TRSM_BM_F32 = 64;  // of an FP32 tile: 64-row block (half the items: fewer re-reads of the diagonal tile)
-__host__ __device__ constexpr int trsm_rows(int elem_bytes) { return elem_bytes == 8 ? TRSM_BM : TRSM_BM_F32; }
+// Rows of a TRSM work item. Up to TRSM_LDS_COLS columns the solved part of X stays in LDS: 16 FP64 or 32 FP32 rows of
+// 512 columns (64 KB, so that two workgroups share a CU). Wider tiles re-read it: 32 and 64 rows.
+constexpr int TRSM_LDS_COLS = 512;
+constexpr int TRSM_BM = 32;
+constexpr int TRSM_BM_F32 = 64;
+__host__ __device__ constexpr int trsm_rows(int elem_bytes, bool in_lds) {
+    return (elem_bytes == 8 ? TRSM_BM : TRSM_BM_F32) / (in_lds ? 2 : 1);
+}
 constexpr int DB = 64;         // diagonal sub-block size whose inverse POTRF leaves for TRSM
 
 // One tiled symmetric matrix in HBM. Tile (i,j), i >= j, is a column-major
@@ -53,7 +58,7 @@ struct DevTask {
     int32_t crit;  // on a longest path of the DAG: runs with no other item started on its CU
     int32_t accum; // GEMM/SYRK: add the product into C under the sub-tile lock (accumulate mode)
     int32_t edge_off, edge_cnt;  // its out-edges in DevGraph::edges
-    int32_t sub;   // GEMM/SYRK: rows and columns of an item, GEMM_BM or GEMM_BS
+    int32_t sub;   // GEMM/SYRK: rows and columns of an item, GEMM_BM or GEMM_BS; TRSM: GEMM_BS = items that keep X in LDS
 };
 
 // An out-edge of the graph with all that releasing its target takes: the task that completes reads it in one access
@@ -68,10 +73,13 @@ struct alignas(16) DevEdge {
 };
 
 // Work items per task of tiles with elem_bytes-byte elements; host and device must agree.
-// (sub: rows and columns of a GEMM/SYRK item).
+// (sub: as DevTask::sub).
 __host__ __device__ inline int items_of(int kind, int bi, int bj, int elem_bytes, int sub = GEMM_BM) {
     if (kind == K_POTRF) return 1;
-    if (kind == K_TRSM) return (bi + trsm_rows(elem_bytes) - 1) / trsm_rows(elem_bytes);
+    if (kind == K_TRSM) {
+        const int rows = trsm_rows(elem_bytes, sub == GEMM_BS);
+        return (bi + rows - 1) / rows;
+    }
     const int tr = (bi + sub - 1) / sub;
     if (kind == K_SYRK) return tr * (tr + 1) / 2;
     if (kind == K_GEMM) return tr * ((bj + sub - 1) / sub);

@@ -55,3 +55,25 @@ def test_potrf_block_items(ctx, oracle, n, dtype):
         out = from_dev(d)[:n]
         assert rel(np.tril(out), np.tril(ref)) < (2e-6 if dtype == "f32" else 1e-13)
         assert np.array_equal(np.triu(out, 1), np.triu(A.astype(np.float32) if dtype == "f32" else A, 1))
+
+
+@pytest.mark.parametrize("m,n", [(1, 64), (15, 65), (16, 127), (17, 192), (33, 448), (31, 511), (65, 512), (40, 513)])
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+def test_trsm_strips(ctx, m, n, dtype):
+    # strips of X in LDS (up to 512 columns) and beside them the form for wider L, odd leading dimensions
+    import torch
+    rng = np.random.default_rng(m * n)
+    L = np.tril(rng.standard_normal((n, n)) * (0.7 / np.sqrt(n)), -1) + np.diag(rng.uniform(1.2, 1.6, n))
+    B = rng.standard_normal((m, n))
+    dt = torch.float64 if dtype == "f64" else torch.float32
+    dL = torch.zeros((n, n + 1), dtype=torch.float64)
+    dL[:, :n] = torch.from_numpy(np.ascontiguousarray(L.T))
+    dB = torch.full((n, m + 3), 5.0, dtype=torch.float64)
+    dB[:, :m] = torch.from_numpy(np.ascontiguousarray(B.T))
+    dL, dB = dL.to(dt).cuda(), dB.to(dt).cuda()
+    Lr, Br = from_dev(dL)[:n], from_dev(dB)[:m]
+    ctx.trsm(m, n, dL, n + 1, dB, m + 3)
+    out = from_dev(dB)
+    want = np.linalg.solve(Lr, Br.T).T
+    assert rel(out[:m], want) < (2e-6 if dtype == "f32" else 1e-13)
+    assert (out[m:] == 5.0).all()
