@@ -73,6 +73,7 @@ static std::shared_ptr<StreamPlan> build_stream_plan(ttad_matrix* M, int prec, i
         t.bucket = 0;
         t.crit = 0;
         t.sub = GEMM_BM;
+        t.kspan = 1;
         return t;
     };
     for (int k = 0; k < nt; k++) {
@@ -676,6 +677,7 @@ int ttad_graph_create(ttad_context* ctx, int n_tasks, const ttad_task_desc* task
         x.n_items = 1;
         x.bucket = 0;
         x.crit = 0;
+        x.kspan = 1;
         g->spin_us[t] = d.kind == TTAD_SPIN ? d.k : 0;
     }
     for (int e = 0; e < n_edges; e++)
@@ -768,16 +770,17 @@ static int graph_prepare(ttad_graph* g) {
             return in ? items_of(x.kind, M->bsz[x.i], M->bsz[x.j], (int)M->elem, sub) : 0;
         };
         for (auto& x : g->tasks)
-            if (x.kind == K_GEMM || x.kind == K_SYRK) step_items[{x.mat, x.k}] += update_items(x, GEMM_BM);
+            if (x.kind == K_GEMM || x.kind == K_SYRK)
+                for (int q = 0; q < x.kspan; q++) step_items[{x.mat, x.k + q}] += update_items(x, GEMM_BM);
         // FP64: with more than 128 update items per CU in all the updates' throughput bounds the run and TRSM keeps its
-        // higher strips (n = 16384, b = 512, 374 per CU: 29.3 ms, 31.0 with the LDS form on the longest path and in
-        // the small steps); below, the chain does (n = 8192, 49 per CU: 5.4 and 5.2 ms).
+        // higher strips (n = 12288, b = 512, 145 per CU: 12.6 ms, 12.5 with the LDS form on the longest path and
+        // in the small steps; n = 16384, 26.1 either way); below, the chain does (n = 8192, 49 per CU: 5.4 and 5.2 ms).
         long long update_total = 0;
         for (auto& kv : step_items) update_total += kv.second;
         const bool throughput = update_total > 128LL * g->ctx->n_cu;
         for (auto& x : g->tasks) {
             x.sub = GEMM_BM;
-            if ((x.kind == K_GEMM || x.kind == K_SYRK) && !x.accum &&
+            if ((x.kind == K_GEMM || x.kind == K_SYRK) && !x.accum && x.kspan == 1 &&
                 (x.crit || 2 * step_items[{x.mat, x.k}] <= g->ctx->n_cu))
                 x.sub = GEMM_BS;
             if (x.kind == K_TRSM && x.mat < (int)g->mats.size() && g->mats[x.mat] && x.j >= 0 && x.j < g->mats[x.mat]->nt &&
@@ -846,7 +849,7 @@ static int graph_prepare(ttad_graph* g) {
         TTAD_HIP(g->d_deps0.alloc(n * 4));
         TTAD_HIP(g->d_deps.alloc(n * 4));
         TTAD_HIP(g->d_items_left.alloc(n * 4));
-        TTAD_HIP(g->d_gops.alloc((size_t)n * sizeof(GemmOperands)));
+        TTAD_HIP(g->d_gops.alloc((size_t)n * g->gop_stride * sizeof(GemmOperands)));
         TTAD_HIP(g->d_tail0.alloc(g->n_buckets * 4));
         TTAD_HIP(g->d_q_head.alloc(g->n_buckets * 4));
         TTAD_HIP(g->d_q_tail.alloc(g->n_buckets * 4));
@@ -913,6 +916,7 @@ static DevGraph graph_image(ttad_graph* g, bool trace, int64_t spin_limit) {
     d.deps = g->d_deps.as<int32_t>();
     d.items_left = g->d_items_left.as<int32_t>();
     d.gops = g->d_gops.as<GemmOperands>();
+    d.gop_stride = g->gop_stride;
     d.q_head = g->d_q_head.as<int32_t>();
     d.q_tail = g->d_q_tail.as<int32_t>();
     d.q_count = g->d_q_count.as<int32_t>();

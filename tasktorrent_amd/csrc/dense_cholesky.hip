@@ -148,6 +148,77 @@ static int build_cholesky_graph(ttad_context* ctx, int nb, int storage, int prec
     return TTAD_OK;
 }
 
+// Fuses consecutive updates GEMM(k, i, j), GEMM(k + 1, i, j), .. of a tile into one task of about `cols` columns (at most
+// KSPAN_MAX steps): C is then read and written once for all of them and the items'
+// claims, starts and releases are paid once. FP32 and bf16 items keep C in registers and subtract each step's product from
+// it, so the factor is bit for bit that of single steps; FP64 and bf16x3 ones have no registers left for that and sum the
+// steps' products in the accumulators in the order of k (the factor then depends on the partition and the size only).
+// Residual ||L L^T - A|| / ||A|| single / fused: FP64 n = 16384 b = 512 7.6e-16 / 6.0e-16; bf16x3 n = 24576 b = 512 6.02e-7 /
+// 6.00e-7, ill-conditioned 2.090e-6 / 2.088e-6 (2048 columns 2.096e-6: hence 1024 there); FP32 sums of 2048 columns would
+// have raised 2.8e-7 to 3.8e-7. A tile's last FUSE_GUARD steps stay single (a panel would wait for its group to fill:
+// 1 / 3 steps, FP64 n = 16384 b = 512: 26.9 / 27.8 ms), and so do steps of unequal or odd width (the K-chunks of all
+// steps run in one pipeline). Groups start at multiples of the span.
+constexpr int FUSE_GUARD = 1;
+static void fuse_updates(ttad_graph* g, const ttad_matrix* M, int cols) {
+    const int n = g->n_tasks;
+    std::vector<std::pair<std::array<int, 3>, int>> steps;  // (i, j, k) and the task, tile by tile in the order of k
+    for (int t = 0; t < n; t++) {
+        const DevTask& x = g->tasks[t];
+        if (x.kind == K_GEMM || x.kind == K_SYRK) steps.push_back({{x.i, x.j, x.k}, t});
+    }
+    std::sort(steps.begin(), steps.end());
+    std::vector<int> rep(n);
+    for (int t = 0; t < n; t++) rep[t] = t;
+    int head = -1;  // the task that the next step of its tile may join
+    for (auto& st : steps) {
+        const int i = st.first[0], j = st.first[1], k = st.first[2], t = st.second, b = M->bsz[k];
+        const int span = b > 0 ? std::min(KSPAN_MAX, cols / b) : 1;
+        const bool may = span > 1 && b % 64 == 0 && k < j - FUSE_GUARD;
+        DevTask* h = head >= 0 ? &g->tasks[head] : nullptr;
+        if (may && k % span != 0 && h && h->i == i && h->j == j && h->k + h->kspan == k && M->bsz[h->k] == b) {
+            rep[t] = head;
+            h->kspan++;
+            g->gop_stride = std::max(g->gop_stride, h->kspan);
+        } else {
+            head = may ? t : -1;
+        }
+    }
+    if (g->gop_stride == 1) return;
+    std::vector<int> id(n, -1);
+    int m = 0;
+    for (int t = 0; t < n; t++)
+        if (rep[t] == t) id[t] = m++;
+    std::vector<std::vector<int>> out(m);
+    std::vector<int32_t> indeg(m, 0), seeds(m, 0), spin(m, 0);
+    std::vector<DevTask> tasks(m);
+    for (int t = 0; t < n; t++) {
+        const int a = id[rep[t]];
+        if (rep[t] == t) {
+            tasks[a] = g->tasks[t];
+            spin[a] = g->spin_us[t];
+        }
+        seeds[a] += g->seeds[t];
+        indeg[a] += g->indegree[t];
+        for (int e = g->out_ptr[t]; e < g->out_ptr[t + 1]; e++) {
+            const int b = id[rep[g->out_idx[e]]];
+            if (a == b) indeg[a]--;  // the chain inside a group
+            else out[a].push_back(b);
+        }
+    }
+    g->n_tasks = m;
+    g->tasks = std::move(tasks);
+    g->indegree = std::move(indeg);
+    g->seeds = std::move(seeds);
+    g->spin_us = std::move(spin);
+    g->out_ptr.assign(1, 0);
+    g->out_idx.clear();
+    for (auto& o : out) {
+        g->out_idx.insert(g->out_idx.end(), o.begin(), o.end());
+        g->out_ptr.push_back((int32_t)g->out_idx.size());
+    }
+    g->mats_dirty = g->seeds_dirty = true;
+}
+
 // The bf16 hi/lo planes of M's off-diagonal tiles (FP32 storage): every tile (i, j), i > j, whose
 // column count bsz[j] is a multiple of 32 gets bsz[i] * bsz[j] * 4 bytes in one slab; the pointer table
 // is null elsewhere. Allocated once per matrix. Returns false (and allocates nothing) when the slab
@@ -189,6 +260,18 @@ int cholesky_persistent(ttad_context* ctx, ttad_matrix* M, int prio_kind, int pr
         const int rc = build_cholesky_graph(ctx, M->nt, M->storage, prec, prio_kind, &g);
         if (rc != TTAD_OK) return rc;
         ctx->chol_graphs[key] = g;
+        long long items = 0;  // 128 x 128 update items
+        for (auto& x : g->tasks)
+            if (x.kind == K_GEMM || x.kind == K_SYRK) items += items_of(x.kind, M->bsz[x.i], M->bsz[x.j], (int)M->elem);
+// Fused updates from 8 items per CU on: below, there are too few items to lose any to a longer one, and 64x64
+        // ones take over. 512 columns of sum where the panels' chain still counts, 2048 (bf16x3 1024, see fuse_updates)
+        // from 128 items per CU on, where C's traffic does. Kernel ms single / fused: FP64 n = 4096 b = 128 (17 per CU)
+        // 2.93 / 2.77, 1024 columns 3.19; n = 8192 b = 256 (79) 6.38 / 5.73, 2048 columns 6.52; n = 16384 b = 512 (343)
+        // 29.6 / 25.8, 1024 columns 26.6; b = 256 (650) 40.9 / 26.9; bf16x3 n = 32768 b = 512 (2720) 56.9 / 49.6; FP32
+        // n = 3000 b = 128 (8.6) 1.95 / 1.72, n = 16384 b = 512 14.8 / 14.2.
+        // Accumulate mode adds each product by itself and is left alone.
+        if (items > 8LL * ctx->n_cu && !(prio_kind & TTAD_ACCUMULATE))
+            fuse_updates(g, M, items <= 128LL * ctx->n_cu ? 512 : prec == TTAD_BF16X3 ? 1024 : 2048);
         // bf16x3 updates read their operands pre-split (written by the TRSM items of the same run,
         // which precede every update that reads them in the PTG); accumulate mode keeps the FP32 path
         if (prec == TTAD_BF16X3 && M->storage == TTAD_F32 && !(prio_kind & TTAD_ACCUMULATE) && planes_enabled() &&

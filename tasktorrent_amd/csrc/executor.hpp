@@ -7,18 +7,6 @@
 
 namespace ttad {
 
-// The operands of a GEMM/SYRK task, C(i,j) -= A(i,k) B(j,k)^T, resolved from the matrix's tile tables
-// before a run, so that an item finds them in one load with its task record instead of through the
-// matrix descriptor and its pointer tables (two more dependent memory round trips).
-struct alignas(16) GemmOperands {
-    const void* A;
-    const void* B;
-    void* C;
-    const void* PA;  // bf16 planes of A and B (null: none)
-    const void* PB;
-    int32_t m, n, K, pad;
-};
-
 // Device image of a task graph (built on the host from the Taskflow callbacks).
 struct DevGraph {
     int32_t n_tasks;
@@ -43,7 +31,9 @@ struct DevGraph {
     int32_t* done_items;
     int32_t* abort_flag;        // 1 = watchdog, 2 = queue overflow
     const DevMat* mats;
-    GemmOperands* gops;         // [n_tasks] resolved operands of the GEMM/SYRK tasks (filled before each run)
+    GemmOperands* gops;         // [n_tasks * gop_stride] resolved operands of the GEMM/SYRK tasks' steps (filled before
+                                // each run)
+    int32_t gop_stride;         // the largest kspan
     uint64_t* trace;            // optional: TRACE_WORDS x u64 per item {task<<20|item, wg, t_start, t_end,
                                 // t_end of the successor release (the task's last item; else 0), 0}
     int32_t* trace_cursor;
@@ -120,8 +110,8 @@ enum ItemVariant : int {
     V_ACC = 32       // accumulate-mode GEMM/SYRK (only in the last set, so the others keep their registers)
 };
 // The compiled sets, smallest first.
-// (FP64 tiles have two: the TRSM form in LDS, present in the kernel though no task uses it, makes the large
-// FP64 factorizations 5 % slower, n = 16384: 29.3 against 31.0 ms; why is not known.)
+// (FP64 tiles have two: the TRSM form in LDS, present though unused in a kernel with inline GEMM items, made the large
+// FP64 factorizations 5 % slower; with the items out of line they are alike, n = 16384: 26.1 ms.)
 constexpr int V_ALL = V_F64S | V_F32S | V_G32 | V_GBF16 | V_GBF16X3 | V_TLDS;
 constexpr int N_VSETS = 7;
 constexpr int VSETS[N_VSETS] = {V_F64S, V_F64S | V_TLDS, V_F32S | V_G32 | V_TLDS, V_F32S | V_GBF16 | V_TLDS,
@@ -194,6 +184,20 @@ __device__ __attribute__((noinline)) void gemm_small_call(const TS* A, const TS*
                                  lds_uniform(lds), wave_uniform(PA), wave_uniform(PB));
     __builtin_amdgcn_s_setprio(0);
 }
+// The executor's 128x128 GEMM/SYRK items, `span` steps of K columns each with operands go[0 .. span - 1]: out of line, with
+// registers of their own. Inline, the bf16x3 loop spilled with more than one step, and the FP64 loop's speed changed with
+// whatever else the kernel held (n = 8192, b = 512, no fused task: 5.3 ms inline, 5.1 so). FOLD as item_gemm (with it the
+// bf16x3 loop spills: n = 32768 45 -> 123 ms).
+template <typename TS, int PREC, int VM, bool FOLD>
+__device__ __attribute__((noinline)) void gemm_call(const GemmOperands* go, int span, int r0, int c0, bool syrk,
+                                                    char* lds) {
+    const GemmOperands* o = wave_uniform(go);
+    const int m = wave_uniform(o->m), n = wave_uniform(o->n);
+    item_gemm<TS, PREC, GEMM_BM, FOLD>((const TS*)wave_uniform(o->A), m, (const TS*)wave_uniform(o->B), n,
+                                       (TS*)wave_uniform(o->C), m, m, n, wave_uniform(o->K), wave_uniform(r0),
+                                       wave_uniform(c0), wave_uniform((int)syrk) != 0, -1.0, 1.0, lds_uniform(lds),
+                                       wave_uniform(o->PA), wave_uniform(o->PB), o + 1, wave_uniform(span) - 1);
+}
 template <typename TS, int VM>
 __device__ __attribute__((noinline)) void trsm_call(const TS* L, const double* dinv, TS* X, int m, int n, int it,
                                                     bool in_lds, char* lds, void* planes) {
@@ -218,7 +222,7 @@ __device__ __attribute__((noinline)) void trsm_call(const TS* L, const double* d
 // each other (item_potrf): the caller must
 // have every lower-numbered item of the task running or done; their waits give up
 // after spin_limit ticks or once *err is nonzero (and set *err = 1 when they time out).
-template <int VM>
+template <int VM, bool GOPS = false>
 __device__ __forceinline__ bool exec_item(const DevTask& t, int it, const DevMat* mats, char* lds, int32_t* err,
                                           int64_t spin_limit, const GemmOperands* go = nullptr) {
     if (t.kind == K_NOP) {  // spin task (scheduler-overhead benchmark): k device clock ticks, no tile access
@@ -280,6 +284,7 @@ __device__ __forceinline__ bool exec_item(const DevTask& t, int it, const DevMat
             // resolved before the run (persistent executor); the FP64 instantiation keeps the table lookups,
             // measured faster there (the FP64 items are long, the lookup latency is a small part of them)
             constexpr bool use_go = (VM & (V_G32 | V_GBF16 | V_GBF16X3)) != 0;
+            const int span = wave_uniform(t.kspan);
             if (use_go && go) {
                 opA = wave_uniform(go->A);
                 opB = wave_uniform(go->B);
@@ -318,7 +323,15 @@ __device__ __forceinline__ bool exec_item(const DevTask& t, int it, const DevMat
             return true;                                                                                           \
         }                                                                                                          \
     }                                                                                                              \
-    if (sub == GEMM_BS) {                                                                                          \
+    if (GOPS && sub == GEMM_BM) {                                                                                  \
+        constexpr bool fold = sizeof(TS_) == 4 && PREC_ != P_BF16X3;                                               \
+        if (fold && span > 1)                                                                                      \
+            gemm_call<TS_, PREC_, VM, fold>(go, span, r0, c0, syrk, lds);                                          \
+        else                                                                                                       \
+            gemm_call<TS_, PREC_, VM, false>(go, span, r0, c0, syrk, lds);                                         \
+        return true;                                                                                               \
+    }                                                                                                              \
+    if (GOPS || sub == GEMM_BS) {                                                                                  \
         gemm_small_call<TS_, PREC_, VM>((const TS_*)opA, (const TS_*)opB, (TS_*)opC, m, n, K, r0, c0, syrk, lds,   \
                                         opPA, opPB);                                                               \
         return true;                                                                                               \

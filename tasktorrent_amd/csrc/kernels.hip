@@ -227,14 +227,14 @@ __global__ __launch_bounds__(NTHREADS, vset_occupancy(VM)) void k_persistent(Dev
         const int task = __builtin_amdgcn_readfirstlane((int)(e >> 20));
         const int item = __builtin_amdgcn_readfirstlane((int)(e & 0xFFFFF));
         const DevTask t = g.tasks[task];
-        const GemmOperands go = g.gops[task];  // read with the task record (GEMM/SYRK items use it)
+        const GemmOperands* go = g.gops + (long)task * g.gop_stride;  // (GEMM/SYRK items use them)
         if (tid == 0) {
             if (t.crit) __hip_atomic_fetch_add(g.cu_crit + my_key, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_fetch_add(g.xcd_run + (long)task * NXCD + my_xcd, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         uint64_t t0 = 0;
         if (g.trace && tid == 0) t0 = wall_clock64();
-        const bool ran = exec_item<VM>(t, item, g.mats, lds, g.abort_flag, g.spin_limit, &go);
+        const bool ran = exec_item<VM, true>(t, item, g.mats, lds, g.abort_flag, g.spin_limit, go);
         // Every wave waits until the L2 has acknowledged its own stores (gfx9: vmcnt counts stores too;
         // encoding vmcnt(0) expcnt(7) lgkmcnt(15)) before the barrier: after it, thread 0's decrement
         // below is issued only once all of this item's outputs sit in this XCD's L2.
@@ -318,17 +318,19 @@ __global__ void k_graph_reset(DevGraph g, int n_slots) {
         if (t.kind == K_GEMM || t.kind == K_SYRK) {
             const DevMat& M = g.mats[t.mat];
             const long nt = M.nt;
-            GemmOperands o;
-            o.A = M.tiles[t.i + t.k * nt];
-            o.B = M.tiles[t.j + t.k * nt];
-            o.C = M.tiles[t.i + t.j * nt];
-            o.PA = M.planes ? M.planes[t.i + t.k * nt] : nullptr;
-            o.PB = M.planes ? M.planes[t.j + t.k * nt] : nullptr;
-            o.m = M.bsz[t.i];
-            o.n = M.bsz[t.j];
-            o.K = M.bsz[t.k];
-            o.pad = 0;
-            g.gops[x] = o;
+            for (int q = 0; q < t.kspan; q++) {
+                GemmOperands o;
+                o.A = M.tiles[t.i + (t.k + q) * nt];
+                o.B = M.tiles[t.j + (t.k + q) * nt];
+                o.C = M.tiles[t.i + t.j * nt];
+                o.PA = M.planes ? M.planes[t.i + (t.k + q) * nt] : nullptr;
+                o.PB = M.planes ? M.planes[t.j + (t.k + q) * nt] : nullptr;
+                o.m = M.bsz[t.i];
+                o.n = M.bsz[t.j];
+                o.K = M.bsz[t.k + q];
+                o.pad = 0;
+                g.gops[(long)x * g.gop_stride + q] = o;
+            }
         }
     }
     for (long x = blockIdx.x * blockDim.x + threadIdx.x; x < (long)g.n_tasks * NXCD; x += stride) g.xcd_run[x] = 0;

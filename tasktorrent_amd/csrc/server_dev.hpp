@@ -325,6 +325,7 @@ __device__ __forceinline__ void srv_exec(const DevServer& s, const SrvTask& t, i
             d.j = t.j;
             d.k = t.k;
             d.sub = GEMM_BM;
+            d.kspan = 1;
             (void)exec_item<V_ALL>(d, it, s.mats, lds, s.err, s.spin_limit);  // request graphs only hold supported kinds
             break;
         }

@@ -98,6 +98,17 @@ template <> struct V16<float> {
     typedef float u __attribute__((ext_vector_type(4), aligned(4)));
 };
 
+// What a product does after the last K-chunk of each pair of operands.
+struct NoFold {
+    static constexpr bool on = false;
+    __device__ void operator()() const {}
+};
+template <typename F> struct FoldWith {
+    static constexpr bool on = true;
+    F f;
+    __device__ __forceinline__ void operator()() const { f(); }
+};
+
 // ---------------------------------------------------------------------------
 // acc (BM x BN) += A(BM x K) * B(BN x K)^T with A, B column-major (lda, ldb),
 // rows >= mv of A and rows >= nv of B read as zero. TA/TB are storage types,
@@ -200,6 +211,11 @@ struct GemmNT {
         store_chunk<RB, EB, NVB, LB, KS_B, PB>(S + BK * PA, rb);
     }
 
+    static __device__ __forceinline__ void run(acc_t (&acc)[WM][WN], const TA* __restrict__ A, long lda, int mv,
+                                               const TB* __restrict__ B, long ldb, int nv, int K, char* lds) {
+        run(acc, A, lda, mv, B, ldb, nv, K, lds, nullptr, 0, 0, 0, NoFold());
+    }
+
     static __device__ __forceinline__ void compute(acc_t (&acc)[WM][WN], const TC* __restrict__ S, int lane, int wr,
                                                    int wc) {
         const TC* As = S + wr * (WM * 16) + (lane & 15);
@@ -221,11 +237,28 @@ struct GemmNT {
     }
 
     // Starts and ends with a workgroup barrier: the caller may use `lds` before and after.
+    // more > 0: further pairs of operands steps[0 .. more - 1] of K columns each (same shapes; their rows ra0 and rb0 on)
+    // follow in the same pipeline; K is then a multiple of BK.
+    // fold: called after the last chunk of each pair.
+    template <typename Fold>
     static __device__ __forceinline__ void run(acc_t (&acc)[WM][WN], const TA* __restrict__ A, long lda, int mv,
-                                               const TB* __restrict__ B, long ldb, int nv, int K, char* lds) {
+                                               const TB* __restrict__ B, long ldb, int nv, int K, char* lds,
+                                               const GemmOperands* __restrict__ steps, int more, int ra0, int rb0,
+                                               Fold fold) {
         TC* S0 = reinterpret_cast<TC*>(lds);
         const int tid = threadIdx.x;
         const int lane = tid & 63, w = tid >> 6, wr = w / WC, wc = w % WC;
+        const int K0 = K;
+        int next = K0;  // the first column of the next pair, which is addressed as if it followed the first
+        K += more * K0;
+        auto advance = [&](int k0) {
+            if (more > 0 && k0 == next && k0 < K) {
+                A = static_cast<const TA*>(wave_uniform(steps->A)) + ra0 - (long)k0 * lda;
+                B = static_cast<const TB*>(wave_uniform(steps->B)) + rb0 - (long)k0 * ldb;
+                steps++;
+                next += K0;
+            }
+        };
         const int nchunks = (K + BK - 1) / BK;
         __syncthreads();
         if (nchunks == 0) return;
@@ -233,14 +266,24 @@ struct GemmNT {
         RB rb[EB];
         load(ra, rb, A, lda, mv, B, ldb, nv, 0, K);
         store(S0, ra, rb);
+        advance(BK);
         if (nchunks > 1) load(ra, rb, A, lda, mv, B, ldb, nv, BK, K);
         __syncthreads();
+        int done = K0;
         for (int c = 0; c < nchunks; c++) {
             compute(acc, S0 + (c & 1) * STAGE, lane, wr, wc);
+            if constexpr (Fold::on)
+                if ((c + 1) * BK == done) {
+                    fold();
+                    done += K0;
+                }
             if (c + 1 < nchunks) {
                 // the other buffer was last read in chunk c-1, before the previous barrier
                 store(S0 + ((c + 1) & 1) * STAGE, ra, rb);
-                if (c + 2 < nchunks) load(ra, rb, A, lda, mv, B, ldb, nv, (c + 2) * BK, K);
+                if (c + 2 < nchunks) {
+                    advance((c + 2) * BK);
+                    load(ra, rb, A, lda, mv, B, ldb, nv, (c + 2) * BK, K);
+                }
             }
             __syncthreads();
         }
@@ -285,6 +328,10 @@ struct GemmNTbf16 {
     static constexpr int GB = BN * (BK / 8) / NTHREADS;
     static_assert(GA * NTHREADS == BM * (BK / 8) && GB * NTHREADS == BN * (BK / 8), "tile/thread mismatch");
 
+    static __device__ __forceinline__ void run(acc_t (&acc)[WM][WN], const TA* __restrict__ A, long lda, int mv,
+                                               const TA* __restrict__ B, long ldb, int nv, int K, char* lds) {
+        run(acc, A, lda, mv, B, ldb, nv, K, lds, nullptr, 0, 0, 0, NoFold());
+    }
     static __device__ __forceinline__ void zero(acc_t (&acc)[WM][WN]) {
 #pragma unroll
         for (int a = 0; a < WM; a++)
@@ -425,8 +472,22 @@ struct GemmNTbf16 {
     }
 
     // Starts and ends with a workgroup barrier: the caller may use `lds` before and after.
+    // steps, more, ra0, rb0, fold as GemmNT::run.
+    template <typename Fold>
     static __device__ __forceinline__ void run(acc_t (&acc)[WM][WN], const TA* __restrict__ A, long lda, int mv,
-                               const TA* __restrict__ B, long ldb, int nv, int K, char* lds) {
+                               const TA* __restrict__ B, long ldb, int nv, int K, char* lds,
+                               const GemmOperands* __restrict__ steps, int more, int ra0, int rb0, Fold fold) {
+        const int K0 = K;
+        int next = K0;
+        K += more * K0;
+        auto advance = [&](int k0) {
+            if (more > 0 && k0 == next && k0 < K) {
+                A = static_cast<const TA*>(wave_uniform(steps->A)) + ra0 - (long)k0 * lda;
+                B = static_cast<const TA*>(wave_uniform(steps->B)) + rb0 - (long)k0 * ldb;
+                steps++;
+                next += K0;
+            }
+        };
         unsigned short* S0 = reinterpret_cast<unsigned short*>(lds);
         const int tid = threadIdx.x;
         const int lane = tid & 63, w = tid >> 6, wr = w >> 1, wc = w & 1;
@@ -451,16 +512,24 @@ struct GemmNTbf16 {
         load_raw<GB, NTHREADS / BN>(rb, B, ldb, b_row, b_ok, b_g * 8, K, full(0));
         stage(S0);
         if (nchunks > 1) {
+            advance(BK);
             load_raw<GA, NTHREADS / BM>(ra, A, lda, a_row, a_ok, BK + a_g * 8, K, full(BK));
             load_raw<GB, NTHREADS / BN>(rb, B, ldb, b_row, b_ok, BK + b_g * 8, K, full(BK));
         }
         __syncthreads();
+        int done = K0;
         for (int c = 0; c < nchunks; c++) {
             compute(acc, S0 + (c & 1) * STAGE, lane, wr, wc);
+            if constexpr (Fold::on)
+                if ((c + 1) * BK == done) {
+                    fold();
+                    done += K0;
+                }
             if (c + 1 < nchunks) {
                 stage(S0 + ((c + 1) & 1) * STAGE);
                 if (c + 2 < nchunks) {
                     const int k0 = (c + 2) * BK;
+                    advance(k0);
                     load_raw<GA, NTHREADS / BM>(ra, A, lda, a_row, a_ok, k0 + a_g * 8, K, full(k0));
                     load_raw<GB, NTHREADS / BN>(rb, B, ldb, b_row, b_ok, k0 + b_g * 8, K, full(k0));
                 }
@@ -474,34 +543,47 @@ struct GemmNTbf16 {
     // item's first row, arows / brows are the tiles' row counts). Each thread moves whole 16-byte
     // granules, so a chunk costs 4 loads per operand and no conversion; the LDS buffers receive
     // exactly what run() would store from the FP32 values the planes were split from.
+    // more > 0: the planes of steps[0 .. more - 1] follow (their rows ra0 and rb0 on).
+    template <typename Fold>
     static __device__ __forceinline__ void run_planes(acc_t (&acc)[WM][WN], const u4_t* __restrict__ PA, int arows,
-                                                      const u4_t* __restrict__ PB, int brows, int K, char* lds) {
+                                                      const u4_t* __restrict__ PB, int brows, int K, char* lds,
+                                                      const GemmOperands* __restrict__ steps, int more, int ra0,
+                                                      int rb0, Fold fold) {
         static_assert(SPLIT && BK == 32, "plane chunks are 32 columns of hi and lo");
         unsigned short* S0 = reinterpret_cast<unsigned short*>(lds);
         const int tid = threadIdx.x;
         const int lane = tid & 63, w = tid >> 6, wr = w >> 1, wc = w & 1;
         const int a_row = tid % BM, b_row = tid % BN;
         const int a_g = __builtin_amdgcn_readfirstlane(tid / BM), b_g = __builtin_amdgcn_readfirstlane(tid / BN);
-        const int nchunks = wave_uniform(K / BK);
+        const int nc0 = wave_uniform(K / BK), nchunks = wave_uniform(nc0 * (1 + more));
+        int next = nc0;
         arows = wave_uniform(arows);
         brows = wave_uniform(brows);
         __syncthreads();
         if (nchunks == 0) return;
         u4_t ra[GA][2], rb[GB][2];
-        // a uniform granule base per (chunk, plane, group) plus this lane's 32-bit row offset
+        // uniform bases of the next chunk's granules, moved on with each fetch, plus this lane's 32-bit row offset
         const TTAD_GLOBAL u4_t* ga = gmem(wave_uniform(PA));
         const TTAD_GLOBAL u4_t* gb = gmem(wave_uniform(PB));
         auto fetch = [&](int c) {
+            if (more > 0 && c == next) {
+                ga = gmem(static_cast<const u4_t*>(wave_uniform(steps->PA)) + ra0);
+                gb = gmem(static_cast<const u4_t*>(wave_uniform(steps->PB)) + rb0);
+                steps++;
+                next += nc0;
+            }
 #pragma unroll
             for (int s = 0; s < GA; s++)
 #pragma unroll
                 for (int p = 0; p < 2; p++)
-                    ra[s][p] = (ga + plane_granule(c, p, a_g + s * (NTHREADS / BM), 0, arows))[a_row];
+                    ra[s][p] = (ga + plane_granule(0, p, a_g + s * (NTHREADS / BM), 0, arows))[a_row];
 #pragma unroll
             for (int s = 0; s < GB; s++)
 #pragma unroll
                 for (int p = 0; p < 2; p++)
-                    rb[s][p] = (gb + plane_granule(c, p, b_g + s * (NTHREADS / BN), 0, brows))[b_row];
+                    rb[s][p] = (gb + plane_granule(0, p, b_g + s * (NTHREADS / BN), 0, brows))[b_row];
+            ga += plane_granule(1, 0, 0, 0, arows);
+            gb += plane_granule(1, 0, 0, 0, brows);
         };
         auto stage = [&](unsigned short* S) {
             unsigned short* Ah = S;
@@ -525,8 +607,14 @@ struct GemmNTbf16 {
         stage(S0);
         if (nchunks > 1) fetch(1);
         __syncthreads();
+        int done = nc0;
         for (int c = 0; c < nchunks; c++) {
             compute(acc, S0 + (c & 1) * STAGE, lane, wr, wc);
+            if constexpr (Fold::on)
+                if (c + 1 == done) {
+                    fold();
+                    done += nc0;
+                }
             if (c + 1 < nchunks) {
                 stage(S0 + ((c + 1) & 1) * STAGE);
                 if (c + 2 < nchunks) fetch(c + 2);
@@ -571,10 +659,15 @@ template <typename TS> constexpr int trsm_bk() { return sizeof(TS) == 4 ? 64 : 3
 // BM: rows and columns of the item, GEMM_BM or GEMM_BS.
 // PA / PB (bf16x3 only; null = none): the bf16 split planes of the operand tiles (A and B with lda and ldb
 // rows, plane_granule layout), used by items that lie wholly inside both with K % 32 == 0.
-template <typename TS, int PREC, int BM = GEMM_BM>
+// steps, more: the operands of further steps of K columns each; C is then read and written once for all of them. K is a
+// multiple of 64 then, and either all steps have planes or none. FOLD: C (beta = 1, alpha = -1) is read before the first
+// step and each step's product is subtracted from it in registers, as items of one step would; without, the steps'
+// products are summed first.
+template <typename TS, int PREC, int BM = GEMM_BM, bool FOLD = false>
 __device__ __forceinline__ void item_gemm(const TS* __restrict__ A, long lda, const TS* __restrict__ B, long ldb, TS* __restrict__ C,
                           long ldc, int m, int n, int K, int r0, int c0, bool syrk, double alpha, double beta,
-                          char* lds, const void* PA = nullptr, const void* PB = nullptr) {
+                          char* lds, const void* PA = nullptr, const void* PB = nullptr,
+                          const GemmOperands* __restrict__ steps = nullptr, int more = 0) {
     const int mv = min(BM, m - r0), nv = min(BM, n - c0);
     if (mv <= 0 || nv <= 0) return;
     auto body = [&](auto* gsel) {
@@ -582,24 +675,54 @@ __device__ __forceinline__ void item_gemm(const TS* __restrict__ A, long lda, co
         typedef typename G::acc_t acc_t;
         acc_t acc[G::WM][G::WN];
         auto owned = [&](int rr, int cc) { return rr < mv && cc < nv && (!syrk || r0 + rr >= c0 + cc); };
+        const bool full = __builtin_amdgcn_readfirstlane(
+                              (int)(mv == BM && nv == BM && (!syrk || r0 >= c0 + BM))) != 0;
         G::zero(acc);
-        bool planes = false;
-        if constexpr (PREC == P_BF16X3)
-            planes = PA && PB && mv == BM && nv == BM && K % G::BK == 0;
-        if constexpr (PREC == P_BF16X3) {
-            if (planes)
-                G::run_planes(acc, static_cast<const u4_t*>(PA) + r0, (int)lda, static_cast<const u4_t*>(PB) + c0,
-                              (int)ldb, K, lds);
+        auto product = [&](auto fold) {
+            if constexpr (PREC == P_BF16X3)
+                if (PA && PB && mv == BM && nv == BM && K % G::BK == 0) {
+                    G::run_planes(acc, static_cast<const u4_t*>(PA) + r0, (int)lda, static_cast<const u4_t*>(PB) + c0,
+                                  (int)ldb, K, lds, steps, more, r0, c0, fold);
+                    return;
+                }
+            G::run(acc, A + r0, lda, mv, B + c0, ldb, nv, K, lds, steps, more, r0, c0, fold);
+        };
+        if constexpr (FOLD) {
+            acc_t tot[G::WM][G::WN];
+#pragma unroll
+            for (int a = 0; a < G::WM; a++)
+#pragma unroll
+                for (int b = 0; b < G::WN; b++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const int rr = G::row_of(a, r), cc = G::col_of(b, r);
+                        tot[a][b][r] = gmem(C)[(full || owned(rr, cc)) ? (r0 + rr) + (long)(c0 + cc) * ldc : 0];
+                    }
+            auto sub = [&]() {
+#pragma unroll
+                for (int a = 0; a < G::WM; a++)
+#pragma unroll
+                    for (int b = 0; b < G::WN; b++) {
+                        tot[a][b] -= acc[a][b];
+                        acc[a][b] = acc_t{0, 0, 0, 0};
+                    }
+            };
+            product(FoldWith<decltype(sub)>{sub});
+#pragma unroll
+            for (int a = 0; a < G::WM; a++)
+#pragma unroll
+                for (int b = 0; b < G::WN; b++) acc[a][b] = tot[a][b];
+            alpha = 1.0;
+            beta = 0.0;
+        } else {
+            product(NoFold());
         }
-        if (!planes) G::run(acc, A + r0, lda, mv, B + c0, ldb, nv, K, lds);
         // C is read after the last K-chunk. Every load of a group of fragment rows is issued before any
         // store of the group: as far as the compiler knows a store may alias a later load, so a load and
         // a store per element in turn would cost one memory round trip per element (64 per item). Groups:
         // all of the item for FP32 tiles, one fragment row for FP64 (registers). Loads come from clamped addresses
         // (C[0] for elements not owned), so none waits under a branch; interior items (all of the
         // 128 x 128 owned) store without a condition.
-        const bool full = __builtin_amdgcn_readfirstlane(
-                              (int)(mv == BM && nv == BM && (!syrk || r0 >= c0 + BM))) != 0;
         if constexpr (sizeof(TS) == 4) {
             // Interior FP32 items go through LDS (free after the K loop): a lane's results lie along a row,
             // C is column-major, so the accumulators are transposed in LDS and every thread then reads,

@@ -47,6 +47,20 @@ __host__ __device__ inline long plane_granule(int c, int p, int g, int r, int m)
     return ((long)(c * 2 + p) * 4 + g) * m + r;
 }
 
+constexpr int KSPAN_MAX = 8;  // steps of one fused update at most
+
+// The operands of a GEMM/SYRK task, C(i,j) -= A(i,k) B(j,k)^T, resolved from the matrix's tile tables
+// before a run, so that an item finds them in one load with its task record instead of through the
+// matrix descriptor and its pointer tables (two more dependent memory round trips).
+struct alignas(16) GemmOperands {
+    const void* A;
+    const void* B;
+    void* C;
+    const void* PA;  // bf16 planes of A and B (null: none)
+    const void* PB;
+    int32_t m, n, K, pad;
+};
+
 // Device task record.
 struct DevTask {
     int32_t kind;
@@ -58,6 +72,7 @@ struct DevTask {
     int32_t crit;  // on a longest path of the DAG: runs with no other item started on its CU
     int32_t accum; // GEMM/SYRK: add the product into C under the sub-tile lock (accumulate mode)
     int32_t edge_off, edge_cnt;  // its out-edges in DevGraph::edges
+    int32_t kspan; // GEMM/SYRK: steps k .. k + kspan - 1 in one task (fused updates of one tile), at most KSPAN_MAX
     int32_t sub;   // GEMM/SYRK: rows and columns of an item, GEMM_BM or GEMM_BS; TRSM: GEMM_BS = items that keep X in LDS
 };
 
