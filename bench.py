@@ -384,8 +384,8 @@ def trailing_update_leg(ctx, mn: int, k: int, reps: int = 10):
 def panel_leg(ctx, m: int, b: int, reps: int = 10):
     """The panel steps alone, FP64, as the factorization runs them.
 
-    POTRF: one b x b tile factored by the row-block items the factorization uses (b/64 workgroups that wait on
-    each other's progress flags), launched alone through the host-sequenced schedule of a one-tile matrix and
+    POTRF: one b x b tile factored by the block items the factorization uses (one workgroup per 64 x 64 block of the
+    lower half, waiting on each other's progress flags), launched alone through the host-sequenced schedule of a one-tile matrix and
     timed with events around that launch. TRSM: ttad_dtrsm on the m x b column of tiles below (the first
     panel's TRSM tasks at m = n - b). GB/s use the per-task algorithmic bytes: POTRF reads and writes its tile
     (2 b^2 8 bytes), a TRSM task reads L_jj and reads and writes its tile (3 b^2 8 bytes)."""
