@@ -427,7 +427,7 @@ def panel_leg(ctx, m: int, b: int, reps: int = 10):
     trsm_gbps = 3.0 * b * b * 8 * n_trsm / t_trsm / 1e9
     del A, Ls, P, Bm
     torch.cuda.empty_cache()
-    return {"potrf_tile": b, "potrf_items": b // 64, "potrf_ms": round(tp * 1e3, 4),
+    return {"potrf_tile": b, "potrf_items": (b // 64) * (b // 64 + 1) // 2, "potrf_ms": round(tp * 1e3, 4),
             "potrf_tflops": round(flops(b) / tp / 1e12, 4), "potrf_gbps": round(potrf_gbps, 2),
             "potrf_hbm_frac": round(potrf_gbps / 8000.0, 5),
             "trsm_shape": f"m={m} n={b} ({n_trsm:g} tile tasks)", "trsm_ms": round(t_trsm * 1e3, 4),

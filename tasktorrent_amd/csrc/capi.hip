@@ -629,7 +629,7 @@ static void mark_critical(ttad_graph& g) {
 
 // Which GEMM/SYRK work queues are homed per XCD. By default the FP32 / BF16 / bf16x3 updates are
 // (measured at n = 32768: bf16x3 time to solution 128.9 ms homed, 144.2 ms shared) and the FP64 ones share
-// one queue per priority bucket (FP64 factorization 223.7 ms shared, 229.4 ms homed); spin tasks are
+// one queue per priority bucket (FP64 factorization at n = 32768 186.4 ms shared, 186.2 homed; n = 12288 12.25 and 12.4); spin tasks are
 // homed. TTAD_XCD_AFFINITY=0 shares every queue, TTAD_XCD_AFFINITY=1 homes FP64 updates too.
 static bool xcd_homed(int kind, int prec) {
     static const int mode = [] {
