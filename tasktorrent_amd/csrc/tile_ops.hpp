@@ -1485,7 +1485,6 @@ __device__ __forceinline__ void item_trsm(const TS* __restrict__ L, long ldl, co
 // every size (bf16x3 n = 16384: 10.8 -> 9.0 ms), FP64 ones while the chain bounds the run (graph_prepare).
 // ---------------------------------------------------------------------------
 constexpr int TRSM_RING = 3;  // chunks of L in flight
-constexpr long TRSM_LDS_MAX_LD = 1 << 24;  // 32-bit byte offsets of 16 columns
 template <typename TS>
 __device__ __forceinline__ void item_trsm_lds(const TS* __restrict__ L, long ldl, const double* __restrict__ dinv,
                                               TS* __restrict__ X, long ldx, int m, int n, int r0, char* lds,
@@ -1502,7 +1501,7 @@ __device__ __forceinline__ void item_trsm_lds(const TS* __restrict__ L, long ldl
     TTAD_GLOBAL TS* Xg = gmem(X) + r0;
     TS bq[TRSM_RING][16];
     // Element `off` bytes behind a uniform pointer: a scalar base and a 32-bit lane offset, no 64-bit lane address per
-    // load (leading dimensions are below TRSM_LDS_MAX_LD).
+    // load (trsm_lane_offset).
     auto at = [](auto* base, unsigned off) {
         using T = typename std::remove_cv<typename std::remove_pointer<decltype(base)>::type>::type;
         return *reinterpret_cast<const TTAD_GLOBAL T*>(reinterpret_cast<const TTAD_GLOBAL char*>(gmem(base)) + off);
@@ -1522,13 +1521,12 @@ __device__ __forceinline__ void item_trsm_lds(const TS* __restrict__ L, long ldl
     TS rhs[RB][4];  // the right-hand side block of the next column block (result layout)
     auto fetch_rhs = [&](int cb) {
         const int c0 = cb * DB, cw = min(DB, n - c0);
+        const TS* base = X + r0 + (long)(c0 + trsm_wave_col(w, cw)) * ldx;
 #pragma unroll
         for (int a = 0; a < RB; a++)
 #pragma unroll
             for (int r = 0; r < 4; r++)
-                rhs[a][r] = at(X + r0 + (long)c0 * ldx, ((unsigned)min(16 * a + l15, mv - 1) +
-                                                         (unsigned)min(16 * w + MF::row(lane, r), cw - 1) * (unsigned)ldx) *
-                                                            (unsigned)sizeof(TS));
+                rhs[a][r] = at(base, trsm_lane_offset(min(16 * a + l15, mv - 1), MF::row(lane, r), w, cw, ldx, sizeof(TS)));
     };
     fetch_rhs(0);
     for (int cb = 0; cb < nblk; cb++) {

@@ -22,6 +22,20 @@ __host__ __device__ constexpr int trsm_rows(int elem_bytes, bool in_lds) {
 }
 constexpr int DB = 64;         // diagonal sub-block size whose inverse POTRF leaves for TRSM
 
+// Addresses of the TRSM items that keep X in LDS: a wave-uniform 64-bit base and a lane's offset of 32 bits, which spans
+// 16 columns of X, or 4 of L, whatever the column block (leading dimensions are below TRSM_LDS_MAX_LD).
+constexpr long TRSM_LDS_MAX_LD = 1 << 24;
+// The column of a block of cw columns at which wave w's part of the right-hand side begins (the last one for waves
+// behind the block's end).
+__host__ __device__ inline int trsm_wave_col(int w, int cw) { return 16 * w < cw ? 16 * w : cw - 1; }
+// Bytes from there to row `row` of the wave's column c, 0 .. 15 (clamped to the block's last).
+__host__ __device__ inline unsigned trsm_lane_offset(int row, int c, int w, int cw, long ldx, int elem_bytes) {
+    const int left = cw - 1 - trsm_wave_col(w, cw);
+    return ((unsigned)row + (unsigned)(c < left ? c : left) * (unsigned)ldx) * (unsigned)elem_bytes;
+}
+static_assert((15 * (TRSM_LDS_MAX_LD - 1) + TRSM_BM_F32) * 8 < (1LL << 32), "a lane's offset in X");
+static_assert((3 * (TRSM_LDS_MAX_LD - 1) + TRSM_LDS_COLS) * 8 < (1LL << 32), "a lane's offset in L");
+
 // One tiled symmetric matrix in HBM. Tile (i,j), i >= j, is a column-major
 // bsz[i] x bsz[j] array with leading dimension bsz[i] (block_sizes_lda,
 // 2d_cholesky.cpp:86-89), reached through the pointer table.
