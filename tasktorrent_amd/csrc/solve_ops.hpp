@@ -342,6 +342,7 @@ __device__ __forceinline__ void item_sweep(const DevMat& M, const SweepTab& tab,
                 }
             }
         }
+    stores_done();
     __syncthreads();
     if (threadIdx.x == 0) {
         release_agent();

@@ -47,6 +47,11 @@ __device__ __forceinline__ void release_agent() {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
+// Every store of this wave has reached the L2 (vmcnt(0) expcnt(7) lgkmcnt(15); gfx9 counts stores in vmcnt). Where one
+// thread releases what a whole workgroup has stored, every wave waits like this in front of the barrier behind which the
+// thread does: the barrier itself waits for no store, and release_agent only for those of its own wave.
+__device__ __forceinline__ void stores_done() { __builtin_amdgcn_s_waitcnt(0x0F70); }
+
 // The workgroup's dynamic LDS as a pointer in a scalar register. In a function called out of line its base is read
 // from a table in memory, and the compiler reads it again at every use it cannot hoist (a memory round trip in front
 // of LDS accesses on the critical path); the offset is opaque here, so it is read once.
@@ -1240,8 +1245,6 @@ __device__ __forceinline__ void stage_inv(double* Bt, const TTAD_GLOBAL double* 
 #pragma unroll
     for (int e = 0; e < PER; e++) Bt[(k0 + e * KS) * BP + m] = u[e];
 }
-// Every store of this wave has reached the L2 (vmcnt(0) expcnt(7) lgkmcnt(15); gfx9 counts stores in vmcnt).
-__device__ __forceinline__ void stores_done() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
 template <typename TS>
 __device__ __forceinline__ void item_potrf(TS* __restrict__ A, long lda, int n, double* __restrict__ dinv, int* info,
