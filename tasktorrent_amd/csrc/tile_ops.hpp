@@ -852,6 +852,7 @@ __device__ __forceinline__ void item_gemm_acc(const TS* __restrict__ A, long lda
                         *p = (TS)((double)(*p) + alpha * (double)acc[a][b][r]);
                     }
                 }
+        stores_done();
         __syncthreads();
         if (threadIdx.x == 0) {
             release_agent();
