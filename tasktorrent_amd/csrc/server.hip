@@ -119,6 +119,7 @@ __global__ __launch_bounds__(NTHREADS) void k_server(DevServer s) {
         const int task = (int)(e >> 16), item = (int)(e & 0xFFFF);
         const SrvTask t = s.tasks[task];
         srv_exec(s, t, task, item, lds);
+        stores_done();
         __syncthreads();
         if (tid == 0) {
             release_agent();

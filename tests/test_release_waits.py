@@ -24,7 +24,7 @@ def _unwaited(name):
     return [m.start() for m in RELEASE.finditer(src) if not re.search(WAIT + r"\s*$", src[:m.start()])]
 
 
-@pytest.mark.parametrize("name,sites", [("solve_ops.hpp", 1), ("tile_ops.hpp", 1)])
+@pytest.mark.parametrize("name,sites", [("solve_ops.hpp", 1), ("tile_ops.hpp", 1), ("server.hip", 1)])
 def test_stores_are_waited_for_in_front_of_the_barrier(name, sites):
     assert len(RELEASE.findall(_source(name))) == sites
     assert _unwaited(name) == []
