@@ -1153,8 +1153,8 @@ __device__ __forceinline__ int wait_count(const int32_t* count, int want, int32_
 
 
 // ---------------------------------------------------------------------------
-// POTRF of an n x n diagonal tile as items of 64x64 blocks, nb = ceil(n / 64) block rows. Row r has r items (row 0
-// one): block items (r, q), q < r - 1, and last its tail item, which owns blocks (r, r-1) and (r, r). An item keeps its
+// POTRF of an n x n diagonal tile as items of 64x64 blocks, nb = ceil(n / 64) block rows (potrf_item): block items
+// (r, q), q < r - 1, and per row a tail item, which owns blocks (r, r-1) and (r, r). An item keeps its
 // blocks in registers and is left-looking:
 //   A(r,q) -= L(r,j) L(q,j)^T, j = 0 .. q-1, each product once both blocks are published
 //   L(r,q)  = A(r,q) X(q)^T once X(q) = L(q,q)^{-1} is published
@@ -1169,10 +1169,6 @@ __device__ __forceinline__ int wait_count(const int32_t* count, int want, int32_
 constexpr int BP = DB + 2;  // LDS pitch of a 64x64 operand block: Blk[k * BP + m] = element (m, k)
 constexpr int LDS_POTRF = 2 * DB * BP * 8;
 static_assert(DB * BP * 8 + DB * DP * 8 <= LDS_POTRF && (DB * DP + 1) * 8 <= DB * BP * 8, "D, X and its flag word fit");
-__host__ __device__ inline int potrf_blocks(int n) { return (n + DB - 1) / DB; }
-__host__ __device__ inline int potrf_items(int n) { return 1 + potrf_blocks(n) * (potrf_blocks(n) - 1) / 2; }
-// ints of flags per tile: one per block, and the count of finished items (the last one clears them for the next run)
-__host__ __device__ inline int potrf_flags(int n) { return potrf_blocks(n) * (potrf_blocks(n) + 1) / 2 + 1; }
 
 // acc[cb] += At (rows 16w .. 16w+15) Bt^T (columns 16cb .. 16cb+15) of 64x64 operands in LDS; TRI: Bt is lower
 // triangular (k <= column), its zero blocks are skipped. A lane's results: row 16w + l%16, columns 16cb + l/16 + 4r.
@@ -1252,13 +1248,11 @@ __device__ __forceinline__ void item_potrf(TS* __restrict__ A, long lda, int n, 
                                            int col_off, int it, int32_t* flags, int32_t* err, int64_t spin_limit,
                                            char* lds) {
     const int tid = threadIdx.x, lane = tid & 63, w = wave_uniform(tid >> 6);
-    const int nb = potrf_blocks(n);
-    int r = 0, rem = it;
-    while (rem >= max(1, r)) rem -= max(1, r++);
-    const bool tail = rem == max(1, r) - 1;
-    const int q = tail ? r - 1 : rem;  // this item's off-diagonal block is (r, q); row 0 has none
+    const PotrfItem own = potrf_item(it);
+    const int r = own.r, q = own.q;
+    const bool tail = own.tail;
     const int p0 = r * DB, pw = min(DB, n - p0);
-    auto flag = [&](int i, int j) { return flags + (i * (i + 1) / 2 + j); };
+    auto flag = [&](int i, int j) { return flags + potrf_flag(i, j); };
     auto publish = [&](int i, int j) {
         release_agent();
         __hip_atomic_store(flag(i, j), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1377,9 +1371,8 @@ __device__ __forceinline__ void item_potrf(TS* __restrict__ A, long lda, int n, 
     }
     if (tid == 0) {
         // the last item of the task to finish clears the flags for the next run on this tile
-        int32_t* fin = flags + nb * (nb + 1) / 2;
-        if (__hip_atomic_fetch_add(fin, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == potrf_items(n) - 1)
-            for (int e = 0; e <= nb * (nb + 1) / 2; e++)
+        if (__hip_atomic_fetch_add(flags + potrf_fin(n), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == potrf_items(n) - 1)
+            for (int e = 0; e < potrf_flags(n); e++)
                 __hip_atomic_store(flags + e, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }

@@ -36,6 +36,28 @@ __host__ __device__ inline unsigned trsm_lane_offset(int row, int c, int w, int 
 static_assert((15 * (TRSM_LDS_MAX_LD - 1) + TRSM_BM_F32) * 8 < (1LL << 32), "a lane's offset in X");
 static_assert((3 * (TRSM_LDS_MAX_LD - 1) + TRSM_LDS_COLS) * 8 < (1LL << 32), "a lane's offset in L");
 
+// The items of POTRF of an n x n tile (item_potrf), numbered row by row of 64x64 blocks: row r has r of them (row 0 one),
+// the blocks (r, q), q < r - 1, and last its tail item, which owns (r, r-1) and (r, r).
+__host__ __device__ inline int potrf_blocks(int n) { return (n + DB - 1) / DB; }
+__host__ __device__ inline int potrf_items(int n) { return 1 + potrf_blocks(n) * (potrf_blocks(n) - 1) / 2; }
+struct PotrfItem {
+    int r, q;   // its off-diagonal block (row 0 has none: q = -1)
+    bool tail;  // it owns the diagonal block (r, r) too
+};
+__host__ __device__ inline PotrfItem potrf_item(int it) {
+    int r = 0, rem = it;
+    while (rem >= (r > 1 ? r : 1)) {
+        rem -= r > 1 ? r : 1;
+        r++;
+    }
+    const bool tail = rem == (r > 1 ? r : 1) - 1;
+    return {r, tail ? r - 1 : rem, tail};
+}
+// Flags of a tile: one per block, and behind them the count of finished items (the last one clears them for the next run).
+__host__ __device__ inline int potrf_flag(int r, int q) { return r * (r + 1) / 2 + q; }
+__host__ __device__ inline int potrf_fin(int n) { return potrf_flag(potrf_blocks(n), 0); }
+__host__ __device__ inline int potrf_flags(int n) { return potrf_fin(n) + 1; }
+
 // One tiled symmetric matrix in HBM. Tile (i,j), i >= j, is a column-major
 // bsz[i] x bsz[j] array with leading dimension bsz[i] (block_sizes_lda,
 // 2d_cholesky.cpp:86-89), reached through the pointer table.
