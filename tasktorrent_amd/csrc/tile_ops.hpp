@@ -1370,7 +1370,9 @@ __device__ __forceinline__ void item_potrf(TS* __restrict__ A, long lda, int n, 
         }
     }
     if (tid == 0) {
-        // the last item of the task to finish clears the flags for the next run on this tile
+        // the last item of the task to finish clears the flags for the next run on this tile; every item's own flags have
+        // arrived by then, since it waits for these stores before it counts itself
+        stores_done();
         if (__hip_atomic_fetch_add(flags + potrf_fin(n), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == potrf_items(n) - 1)
             for (int e = 0; e < potrf_flags(n); e++)
                 __hip_atomic_store(flags + e, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -153,3 +153,21 @@ def _two_tiles(tables, n, seed, workers, stores_waited):
 @pytest.mark.parametrize("workers", [1, 3, 1000])
 def test_any_interleaving_gives_the_factor(tables, n, workers):
     assert _two_tiles(tables, n, n + workers, workers, True) < 1e-13
+
+
+def _source():
+    import re
+    from pathlib import Path
+    src = (Path(__file__).resolve().parent.parent / "tasktorrent_amd" / "csrc" / "tile_ops.hpp").read_text()
+    src = re.sub(r"//[^\n]*", "", src)
+    a = src.index("item_potrf(TS*")
+    return src[a:src.index("\ntemplate <", a)]
+
+
+def test_flag_stores_are_waited_for_before_the_item_counts_itself(tables):
+    import re
+    src = _source()
+    end = src[src.rindex("publish(r, r)"):src.index("potrf_fin(n)")]
+    assert re.search(r"if \(tid == 0\) \{\s*stores_done\(\);\s*if \(__hip_atomic_fetch_add\(flags \+ $", end)
+    # without this wait, an item's flag can land behind the clearing of the last one: the model finds it
+    assert any(_two_tiles(tables, 128, seed, 1000, False) is None for seed in range(200))
