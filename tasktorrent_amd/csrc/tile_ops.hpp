@@ -1357,12 +1357,11 @@ __device__ __forceinline__ void item_potrf(TS* __restrict__ A, long lda, int n, 
             const int j = j0 + e * (NTHREADS / DB);
             Xg[i + j * DB] = X[i + j * DP];
         }
+        // (the word keeps the first report: a block that fails because of this one's NaNs waits for the flag below)
+        if (bad && tid == 0) atomicCAS(info, 0, col_off + p0 + bad);
         stores_done();
         __syncthreads();
-        if (tid == 0) {
-            publish(r, r);
-            if (bad) atomicCAS(info, 0, col_off + p0 + bad);
-        }
+        if (tid == 0) publish(r, r);
 #pragma unroll
         for (int e = 0; e < PER; e++) {
             const int j = j0 + e * (NTHREADS / DB);

@@ -171,3 +171,36 @@ def test_flag_stores_are_waited_for_before_the_item_counts_itself(tables):
     assert re.search(r"if \(tid == 0\) \{\s*stores_done\(\);\s*if \(__hip_atomic_fetch_add\(flags \+ $", end)
     # without this wait, an item's flag can land behind the clearing of the last one: the model finds it
     assert any(_two_tiles(tables, 128, seed, 1000, False) is None for seed in range(200))
+
+
+def _first_bad_pivot(seed, report_first, nb=4):
+    """The chain of diagonal blocks, each of which fails once an earlier one has (its inverse holds NaN): block r is
+    entered when block r - 1 has been published, and reports a bad pivot into the one word that keeps the first."""
+    rnd = random.Random(seed)
+    published, info = set(), [0]
+
+    def block(r):
+        while r > 0 and r - 1 not in published:
+            yield
+        for step in (("report", "publish") if report_first else ("publish", "report")):
+            if step == "publish":
+                published.add(r)
+            elif info[0] == 0:
+                info[0] = r + 1
+            yield
+
+    live = {r: block(r) for r in range(nb)}
+    while live:
+        r = rnd.choice(sorted(live))
+        try:
+            next(live[r])
+        except StopIteration:
+            del live[r]
+    return info[0]
+
+
+def test_bad_pivot_is_reported_before_the_block_is_published():
+    src = _source()
+    assert src.index("atomicCAS(info") < src.index("publish(r, r);")
+    assert all(_first_bad_pivot(seed, True) == 1 for seed in range(100))
+    assert any(_first_bad_pivot(seed, False) != 1 for seed in range(100))
