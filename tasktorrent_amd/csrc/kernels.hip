@@ -43,7 +43,7 @@ __global__ __launch_bounds__(NTHREADS, vset_occupancy(VM)) void k_items(const De
 //   The workgroup runs that work item, then thread 0 decrements the
 //   task's remaining-items counter; the last item of a task decrements its
 //   successors' dependency counters and pushes every item of a successor that
-//   reaches zero into its queue. A worker exits when every item is done.
+//   reaches zero into its queue. A worker exits when every item is done, or claimed by others.
 // Memory ordering: item outputs are released (agent scope) before the counter
 // RMWs; queue entries are published with release stores and read with acquire
 // loads, so a consumer on another XCD sees the producer's tiles.
@@ -94,7 +94,7 @@ __global__ __launch_bounds__(NTHREADS, vset_occupancy(VM)) void k_persistent(Dev
             // this XCD. Each scan reads the two (their counters lie in 256-byte blocks that only the workers
             // of one XCD hammer) in one memory round trip; the other XCDs' queues only when both are empty.
             int64_t got = -1;
-            int idle_scans = 0;
+            int idle_scans = 0, done_before = -1;
             const int64_t t_start = (int64_t)wall_clock64();
             for (;;) {
                 int cand[CLAIM_TRIES];  // queues to try, best first
@@ -194,15 +194,33 @@ __global__ __launch_bounds__(NTHREADS, vset_occupancy(VM)) void k_persistent(Dev
                     continue;
                 }
                 // every item done (or the run stopped): this worker is done
-                if (ld_relaxed(g.done_items) == g.total_items || ld_relaxed(g.abort_flag) != 0) {
+                const int done = ld_relaxed(g.done_items);
+                if (done == g.total_items || ld_relaxed(g.abort_flag) != 0) {
                     got = -2;
                     break;
                 }
-                if ((int64_t)wall_clock64() - t_start > g.spin_limit) {
-                    if (tid == 0) __hip_atomic_store(g.abort_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    got = -2;
-                    break;
+                // So it is once every item is claimed: nothing will come, however long the last items still run, and its CU
+                // is free for other work. The queues' heads are only looked at where that is likely, no task having
+                // finished since the last look after a longest pause, and before the watchdog is raised.
+                const bool expired = (int64_t)wall_clock64() - t_start > g.spin_limit;
+                if (expired || (idle_scans == IDLE_BACKOFF && done == done_before)) {
+                    int lane = tid;  // (opaque, as above)
+                    asm volatile("" : "+v"(lane));
+                    bool open = false;  // this lane's bucket: the shared queue, the homed ones
+#pragma unroll 1
+                    for (int x = 0; x <= NXCD; x++) {
+                        const int q = x == NXCD ? shared_queue(lane) : homed_queue(x, lane);
+                        open |= ld_relaxed(g.q_head + q) < g.q_base[q + 1] - g.q_base[q];
+                    }
+                    const bool any_open = __ballot(open) != 0;
+                    if (expired && any_open && tid == 0)
+                        __hip_atomic_store(g.abort_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if (expired || !any_open) {
+                        got = -2;
+                        break;
+                    }
                 }
+                done_before = done;
                 // Idle workers look less often the longer they find nothing (a random 0 .. 2^k - 1 units of 64 cycles,
                 // k up to IDLE_BACKOFF): with hundreds of them idle the next item still meets a scanner within
                 // a fraction of a microsecond, and their loads no longer slow the claims and counters of the few
