@@ -737,7 +737,7 @@ static void raw_trsm(const void* L, long ldl, const double* dinv, void* X, long 
 void launch_raw_trsm(int prec, const void* L, long ldl, const double* dinv, void* X, long ldx, int m, int n,
                      hipStream_t s) {
     if (m <= 0) return;
-    const bool in_lds = n <= TRSM_LDS_COLS && ldl < TRSM_LDS_MAX_LD && ldx < TRSM_LDS_MAX_LD;
+    const bool in_lds = ldl < TRSM_LDS_MAX_LD && ldx < TRSM_LDS_MAX_LD && trsm_in_lds(prec == P_F64 ? 8 : 4, m, n);
     auto* f = prec == P_F64 ? (in_lds ? raw_trsm<double, true> : raw_trsm<double, false>)
                             : (in_lds ? raw_trsm<float, true> : raw_trsm<float, false>);
     f(L, ldl, dinv, X, ldx, m, n, s);

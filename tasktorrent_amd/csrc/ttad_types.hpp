@@ -22,6 +22,20 @@ __host__ __device__ constexpr int trsm_rows(int elem_bytes, bool in_lds) {
 }
 constexpr int DB = 64;         // diagonal sub-block size whose inverse POTRF leaves for TRSM
 
+// Whether a raw TRSM of m rows and n columns takes the strips that keep X in LDS. These are half as high, so L is read twice
+// as often: they pay while all strips run at once (two on each of 256 CUs), where the time is one strip's chain, and behind
+// that as long as the chain is long. Measured, us of the other form / of this one: FP64 n = 512, 512 strips (m = 8192)
+// 101 / 83, 768 130 / 119, 875 148 / 144, 1024 132 / 147, 4096 426 / 522; n = 256, 512 strips 36.7 / 36.6, 768 45.7 /
+// 48.6, 1024 51.5 / 60.1; n = 64, 1024 17.4 / 19.9, 16384 98 / 130. FP32 n = 512, 512 strips (m = 16384) 108 / 84, 625 148
+// / 123, 1250 230 / 187, 8192 1145 / 1064; n = 256, 512 40.5 / 37.1, 1024 55.6 / 62.0, 1250 88.9 / 74.4; n = 128, 512 22.9 /
+// 22.2, 1024 27.2 / 32.1, 8192 143 / 160.
+__host__ __device__ inline bool trsm_in_lds(int elem_bytes, int m, int n) {
+    const int rows = trsm_rows(elem_bytes, true);
+    const long strips = ((long)m + rows - 1) / rows;
+    if (n > TRSM_LDS_COLS) return false;
+    return strips <= 512 || (elem_bytes == 8 ? n > 256 && strips < 1024 : n >= 256);
+}
+
 // Addresses of the TRSM items that keep X in LDS: a wave-uniform 64-bit base and a lane's offset of 32 bits, which spans
 // 16 columns of X, or 4 of L, whatever the column block (leading dimensions are below TRSM_LDS_MAX_LD).
 constexpr long TRSM_LDS_MAX_LD = 1 << 24;
