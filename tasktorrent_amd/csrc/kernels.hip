@@ -440,37 +440,61 @@ __global__ __launch_bounds__(NTHREADS) void k_trtri_diag(const TS* L, long ldl, 
 }
 
 // ---------------------------------------------------------------------------
-// Tile layout conversion: full column-major n x n (FP64) <-> lower tiles. One workgroup per tile and group of
-// CONV_COLS columns (blockIdx.z), a wave per column, each lane CONV_U accesses of V consecutive rows in flight: V = 2
+// Tile layout conversion: full column-major n x n (FP64) <-> lower tiles. Workgroups (i, j, z) share tile (i, j): every
+// gridDim.z-th group of CONV_COLS columns, a wave per column, each lane CONV_U accesses of V consecutive rows in flight: V = 2
 // (16 bytes of FP64) where the dense array's alignment and the tile's rows allow it. Bound by HBM. (One workgroup per
 // tile, an element at a time with a division each: n = 2048, b = 256 93 us to pack and 104 to unpack, now 10 and 10;
 // n = 16384, b = 512 0.88 and 1.25 ms, now 0.51 and 0.65.)
+// SMALL (no tile above CONV_SMALL rows): one workgroup per tile, element by element. A wave per column leaves lanes idle
+// there, and what bounds it is the launch of the workgroups and what each does before its first access. FP64, us to pack and
+// unpack with a wave per column / so: n = 4096, b = 8 127 and 230 / 72 and 98; n = 8192, b = 32 175 and 301 / 101 and 160,
+// b = 64 127 and 201 / 115 and 174 (b = 128 126 and 170, so 150 and 224).
 // ---------------------------------------------------------------------------
-constexpr int CONV_COLS = 16, CONV_U = 4;
+constexpr int CONV_COLS = 16, CONV_U = 4, CONV_SMALL = 64;
 template <typename T, int V> struct ConvVec { typedef T t __attribute__((ext_vector_type(V))); };
 template <typename T> struct ConvVec<T, 1> { typedef T t; };
-// f(row, column) for the first rows of every V-row access of columns q0 .. of an r x c tile, CONV_U at a time: load all,
-// then store all.
+// load(row, column) and store(row, column, value) for the first rows of every V-row access of this workgroup's groups of
+// columns of an r x c tile, CONV_U at a time: load all, then store all.
 template <int V, typename L, typename S>
 __device__ __forceinline__ void conv_tile(int r, int c, const L& load, const S& store) {
-    const int lane = threadIdx.x & 63, q0 = blockIdx.z * CONV_COLS + (threadIdx.x >> 6), q1 = min(c, ((int)blockIdx.z + 1) * CONV_COLS);
-    for (int q = q0; q < q1; q += 4)
-        for (int p0 = V * lane; p0 < r; p0 += 64 * V * CONV_U) {
-            decltype(load(0, 0)) v[CONV_U];
+    const int lane = threadIdx.x & 63;
+    for (int g = blockIdx.z; g * CONV_COLS < c; g += gridDim.z) {
+        const int q0 = g * CONV_COLS + (threadIdx.x >> 6), q1 = min(c, (g + 1) * CONV_COLS);
+        for (int q = q0; q < q1; q += 4)
+            for (int p0 = V * lane; p0 < r; p0 += 64 * V * CONV_U) {
+                decltype(load(0, 0)) v[CONV_U];
 #pragma unroll
-            for (int u = 0; u < CONV_U; u++)
-                if (p0 + u * 64 * V < r) v[u] = load(p0 + u * 64 * V, q);
+                for (int u = 0; u < CONV_U; u++)
+                    if (p0 + u * 64 * V < r) v[u] = load(p0 + u * 64 * V, q);
 #pragma unroll
-            for (int u = 0; u < CONV_U; u++)
-                if (p0 + u * 64 * V < r) store(p0 + u * 64 * V, q, v[u]);
+                for (int u = 0; u < CONV_U; u++)
+                    if (p0 + u * 64 * V < r) store(p0 + u * 64 * V, q, v[u]);
+            }
+    }
+}
+// The same for a matrix of small tiles: the tile's elements one by one, over all threads.
+template <typename L, typename S>
+__device__ __forceinline__ void conv_small(int r, int c, const L& load, const S& store) {
+    for (int e0 = threadIdx.x; e0 < r * c; e0 += NTHREADS * CONV_U) {
+        decltype(load(0, 0)) v[CONV_U];
+#pragma unroll
+        for (int u = 0; u < CONV_U; u++) {
+            const int e = e0 + u * NTHREADS;
+            if (e < r * c) v[u] = load(e % r, e / r);
         }
+#pragma unroll
+        for (int u = 0; u < CONV_U; u++) {
+            const int e = e0 + u * NTHREADS;
+            if (e < r * c) store(e % r, e / r, v[u]);
+        }
+    }
 }
 // Two rows per access need 16-byte aligned pairs of the dense array and whole pairs in the tile's columns.
 __device__ __forceinline__ bool conv_pairs(const double* dense, long ld, int r) {
     return ((uintptr_t)dense % 16) == 0 && (ld % 2) == 0 && (r % 2) == 0;
 }
 
-template <typename TS>
+template <typename TS, bool SMALL>
 __global__ __launch_bounds__(NTHREADS) void k_pack(const double* __restrict__ src, long lda, const DevMat* M, int nt) {
     const int i = blockIdx.x, j = blockIdx.y;
     if (i < j) return;
@@ -482,16 +506,19 @@ __global__ __launch_bounds__(NTHREADS) void k_pack(const double* __restrict__ sr
         constexpr int V = decltype(vc)::value;
         typedef typename ConvVec<double, V>::t sv;
         typedef typename ConvVec<TS, V>::t dv;
-        conv_tile<V>(r, c, [&](int p, int q) { return *reinterpret_cast<const TTAD_GLOBAL sv*>(gmem(base) + p + (long)q * lda); },
-                     [&](int p, int q, sv v) {
-                         if constexpr (V == 1) t[p + (long)q * r] = (TS)v;
-                         else *reinterpret_cast<TTAD_GLOBAL dv*>(t + p + (long)q * r) = __builtin_convertvector(v, dv);
-                     });
+        auto load = [&](int p, int q) { return *reinterpret_cast<const TTAD_GLOBAL sv*>(gmem(base) + p + (long)q * lda); };
+        auto store = [&](int p, int q, sv v) {
+            if constexpr (V == 1) t[p + (long)q * r] = (TS)v;
+            else *reinterpret_cast<TTAD_GLOBAL dv*>(t + p + (long)q * r) = __builtin_convertvector(v, dv);
+        };
+        if constexpr (SMALL) conv_small(r, c, load, store);
+        else conv_tile<V>(r, c, load, store);
     };
-    if (conv_pairs(base, lda, r)) run(std::integral_constant<int, 2>{});
+    if constexpr (SMALL) run(std::integral_constant<int, 1>{});
+    else if (conv_pairs(base, lda, r)) run(std::integral_constant<int, 2>{});
     else run(std::integral_constant<int, 1>{});
 }
-template <typename TS>
+template <typename TS, bool SMALL>
 __global__ __launch_bounds__(NTHREADS) void k_unpack(double* __restrict__ dst, long ldd, const DevMat* M, int nt, int zero_upper) {
     const int i = blockIdx.x, j = blockIdx.y;
     if (i < j && !zero_upper) return;
@@ -503,29 +530,31 @@ __global__ __launch_bounds__(NTHREADS) void k_unpack(double* __restrict__ dst, l
         constexpr int V = decltype(vc)::value;
         typedef typename ConvVec<double, V>::t dv;
         typedef typename ConvVec<TS, V>::t sv;
-        conv_tile<V>(r, c,
-                     [&](int p, int q) {
-                         if (i < j) return dv(0);
-                         if constexpr (V == 1) return (double)t[p + (long)q * r];
-                         else return __builtin_convertvector(*reinterpret_cast<const TTAD_GLOBAL sv*>(t + p + (long)q * r), dv);
-                     },
-                     [&](int p, int q, dv v) {
-                         TTAD_GLOBAL double* d = gmem(base) + p + (long)q * ldd;
-                         if (i == j && p < q) {  // the strict upper triangle
-                             if constexpr (V == 1) {
-                                 if (zero_upper) *d = 0.0;
-                             } else {
-                                 if (p + 1 < q) v[1] = 0.0;
-                                 v[0] = 0.0;
-                                 if (zero_upper) *reinterpret_cast<TTAD_GLOBAL dv*>(d) = v;
-                                 else if (p + 1 >= q) d[1] = v[1];
-                             }
-                             return;
-                         }
-                         *reinterpret_cast<TTAD_GLOBAL dv*>(d) = v;
-                     });
+        auto load = [&](int p, int q) {
+            if (i < j) return dv(0);
+            if constexpr (V == 1) return (double)t[p + (long)q * r];
+            else return __builtin_convertvector(*reinterpret_cast<const TTAD_GLOBAL sv*>(t + p + (long)q * r), dv);
+        };
+        auto store = [&](int p, int q, dv v) {
+            TTAD_GLOBAL double* d = gmem(base) + p + (long)q * ldd;
+            if (i == j && p < q) {  // the strict upper triangle
+                if constexpr (V == 1) {
+                    if (zero_upper) *d = 0.0;
+                } else {
+                    if (p + 1 < q) v[1] = 0.0;
+                    v[0] = 0.0;
+                    if (zero_upper) *reinterpret_cast<TTAD_GLOBAL dv*>(d) = v;
+                    else if (p + 1 >= q) d[1] = v[1];
+                }
+                return;
+            }
+            *reinterpret_cast<TTAD_GLOBAL dv*>(d) = v;
+        };
+        if constexpr (SMALL) conv_small(r, c, load, store);
+        else conv_tile<V>(r, c, load, store);
     };
-    if (conv_pairs(base, ldd, r)) run(std::integral_constant<int, 2>{});
+    if constexpr (SMALL) run(std::integral_constant<int, 1>{});
+    else if (conv_pairs(base, ldd, r)) run(std::integral_constant<int, 2>{});
     else run(std::integral_constant<int, 1>{});
 }
 // Tile-wise copy with conversion between two matrices of the same partition, one workgroup of 256 per lower
@@ -743,18 +772,26 @@ void launch_raw_trsm(int prec, const void* L, long ldl, const double* dinv, void
     f(L, ldl, dinv, X, ldx, m, n, s);
 }
 
-static dim3 conv_grid(int nt, int max_b) { return dim3(nt, nt, (std::max(1, max_b) + CONV_COLS - 1) / CONV_COLS); }
+// Workgroups per tile: one per group of the largest tile's columns, but no more than 2^20 in all where tiles are many (a
+// partition of small tiles and a few large ones would launch mostly empty ones: 512 tiles of 16 and one of 2048, 7.4 ms to pack
+// and 9.2 to unpack, so 0.86 and 1.7).
+static dim3 conv_grid(int nt, int max_b) {
+    const long groups = max_b <= CONV_SMALL ? 1 : (max_b + CONV_COLS - 1) / CONV_COLS;
+    return dim3(nt, nt, (unsigned)std::max(1L, std::min(groups, (1L << 20) / ((long)nt * nt))));
+}
 
 void launch_pack(int storage, const double* src, long lda, const DevMat* M, int nt, int max_b, hipStream_t s) {
-    const dim3 grid = conv_grid(nt, max_b), block(NTHREADS);
-    if (storage == P_F64) hipLaunchKernelGGL((k_pack<double>), grid, block, 0, s, src, lda, M, nt);
-    else hipLaunchKernelGGL((k_pack<float>), grid, block, 0, s, src, lda, M, nt);
+    const bool small = max_b <= CONV_SMALL;
+    auto* f = storage == P_F64 ? (small ? k_pack<double, true> : k_pack<double, false>)
+                               : (small ? k_pack<float, true> : k_pack<float, false>);
+    hipLaunchKernelGGL(f, conv_grid(nt, max_b), dim3(NTHREADS), 0, s, src, lda, M, nt);
 }
 
 void launch_unpack(int storage, double* dst, long ldd, const DevMat* M, int nt, int max_b, int zero_upper, hipStream_t s) {
-    const dim3 grid = conv_grid(nt, max_b), block(NTHREADS);
-    if (storage == P_F64) hipLaunchKernelGGL((k_unpack<double>), grid, block, 0, s, dst, ldd, M, nt, zero_upper);
-    else hipLaunchKernelGGL((k_unpack<float>), grid, block, 0, s, dst, ldd, M, nt, zero_upper);
+    const bool small = max_b <= CONV_SMALL;
+    auto* f = storage == P_F64 ? (small ? k_unpack<double, true> : k_unpack<double, false>)
+                               : (small ? k_unpack<float, true> : k_unpack<float, false>);
+    hipLaunchKernelGGL(f, conv_grid(nt, max_b), dim3(NTHREADS), 0, s, dst, ldd, M, nt, zero_upper);
 }
 
 void launch_copy_tiles(int dst_storage, int src_storage, const DevMat* S, const DevMat* D, int nt, hipStream_t s) {
