@@ -714,24 +714,14 @@ void launch_persistent(int vset, const DevGraph& g, int n_workers, hipStream_t s
 template <typename TS, int PREC, int BM>
 static void raw_gemm(const void* A, long lda, const void* B, long ldb, void* C, long ldc, int m, int n, int K, int syrk,
                      double alpha, double beta, hipStream_t s) {
-    const long tr = (m + BM - 1) / BM, tc = (n + BM - 1) / BM;
-    const long items = syrk ? tr * (tr + 1) / 2 : tr * tc;
-    hipLaunchKernelGGL((k_raw_gemm<TS, PREC, BM>), dim3((unsigned)items), dim3(NTHREADS), (gemm_item_lds<TS, PREC, BM>()), s,
+    hipLaunchKernelGGL((k_raw_gemm<TS, PREC, BM>), dim3((unsigned)raw_gemm_items(m, n, syrk != 0, BM)), dim3(NTHREADS), (gemm_item_lds<TS, PREC, BM>()), s,
                        (const TS*)A, lda, (const TS*)B, ldb, (TS*)C, ldc, m, n, K, syrk, alpha, beta);
 }
 
-// 64x64 items where 128x128 ones would leave CUs without work. Measured, us with 128 / with 64, by the number of 128x128
-// items: 4 (m = n = k = 256) FP64 48 / 19, FP32 25 / 11, bf16x3 17 / 10; 64 (m = n = 1000, k = 300) FP64 74 / 31, bf16x3
-// 30 / 16; 144 (1536, 512) FP64 90 / 78, FP32 47 / 42, bf16x3 32 / 25; 256 (2048, 1024) FP64 175 / 191, FP32 92 / 97,
-// bf16x3 62 / 53; 484 (2816, 512) FP64 158 / 191, FP32 81 / 97, bf16x3 44 / 54.
-static bool raw_gemm_small(int prec, long items) { return items <= (prec == P_F64 || prec == P_F32 ? 192 : 256); }
-
 void launch_raw_gemm(int prec, const void* A, long lda, const void* B, long ldb, void* C, long ldc, int m, int n,
                      int K, int syrk, double alpha, double beta, hipStream_t s) {
-    const long tr = (m + GEMM_BM - 1) / GEMM_BM, tc = (n + GEMM_BM - 1) / GEMM_BM;
-    const long items = syrk ? tr * (tr + 1) / 2 : tr * tc;
-    if (items <= 0) return;
-    const bool small = raw_gemm_small(prec, items);
+    if (m <= 0 || n <= 0) return;
+    const bool small = raw_gemm_small(prec, m, n, K, syrk != 0);
     auto* f = prec == P_F64    ? (small ? raw_gemm<double, P_F64, GEMM_BS> : raw_gemm<double, P_F64, GEMM_BM>)
               : prec == P_F32  ? (small ? raw_gemm<float, P_F32, GEMM_BS> : raw_gemm<float, P_F32, GEMM_BM>)
               : prec == P_BF16 ? (small ? raw_gemm<float, P_BF16, GEMM_BS> : raw_gemm<float, P_BF16, GEMM_BM>)

@@ -22,6 +22,26 @@ __host__ __device__ constexpr int trsm_rows(int elem_bytes, bool in_lds) {
 }
 constexpr int DB = 64;         // diagonal sub-block size whose inverse POTRF leaves for TRSM
 
+// Items of a raw GEMM (SYRK) of bm x bm of them.
+__host__ __device__ inline long raw_gemm_items(int m, int n, bool syrk, int bm) {
+    const long tr = ((long)m + bm - 1) / bm, tc = ((long)n + bm - 1) / bm;
+    return syrk ? tr * (tr + 1) / 2 : tr * tc;
+}
+// Whether a raw GEMM takes 64x64 items: where 128x128 ones would leave CUs without work. Measured, us with 128 / with 64,
+// by the number of 128x128 items: 4 (m = n = k = 256) FP64 48 / 19, FP32 25 / 11, bf16x3 17 / 10; 64 (m = n = 1000, k = 300)
+// FP64 74 / 31, bf16x3 30 / 16; 144 (1536, 512) FP64 90 / 78, FP32 47 / 42, bf16x3 32 / 25; 256 (2048, 1024) FP64 175 / 191,
+// FP32 92 / 97, bf16x3 62 / 53; 484 (2816, 512) FP64 158 / 191, FP32 81 / 97, bf16x3 44 / 54. Short products move mostly C,
+// and from 512 64x64 items (two on each CU) on, those gain nothing on it: 144 items, k = 16 FP64 14.2 / 15.2, k = 48 18.7 / 18.7,
+// k = 64 21.0 / 17.8; FP32 k = 16 9.1 / 11.2, k = 32 8.3 / 12.1, k = 48 11.5 / 13.2, k = 64 10.5 / 9.9 (121 items, k = 16 FP64
+// 13.9 / 10.2). Long bf16 products are bound by their operands, which these items read twice as often: 256 items, k =
+// 1024 37.8 / 37.2, 2048 66.0 / 67.0, 8192 238 / 255; 196 (1792) 1024 36.7 / 38.3, 8192 237 / 260, but ragged (1700) 4096 189 / 164.
+__host__ __device__ inline bool raw_gemm_small(int prec, int m, int n, int K, bool syrk) {
+    const long items = raw_gemm_items(m, n, syrk, GEMM_BM);
+    if (prec == P_F64 || prec == P_F32) return items <= (K < 64 ? 128 : 192);
+    if (prec == P_BF16 && K > 1024 && raw_gemm_items(m, n, syrk, GEMM_BS) > 768) return false;
+    return items <= 256;
+}
+
 // Whether a raw TRSM of m rows and n columns takes the strips that keep X in LDS. These are half as high, so L is read twice
 // as often: they pay while all strips run at once (two on each of 256 CUs), where the time is one strip's chain, and behind
 // that as long as the chain is long. Measured, us of the other form / of this one: FP64 n = 512, 512 strips (m = 8192)
