@@ -967,19 +967,23 @@ int ttad_graph_launch(ttad_graph* g, int n_workers, int trace, void* stream) {
     return TTAD_OK;
 }
 
+// Whether the last run's report has arrived.
+static bool reported(const ttad_graph* g) { return __atomic_load_n(&g->report->seq, __ATOMIC_ACQUIRE) == g->seq; }
+
 int ttad_graph_wait(ttad_graph* g, double timeout_s, ttad_graph_stats* stats) {
     if (!g) return set_error(TTAD_ERR_INVALID, "graph is NULL");
     if (!g->running) return set_error(TTAD_ERR_INVALID, "graph_wait: not launched");
     // The run's report arrives in pinned memory: a read of it costs no call into the runtime. It is watched closely for
-    // the first milliseconds (short runs) and every 50 us afterwards, when the stream is asked for errors too.
+    // the first milliseconds (short runs) and every 50 us afterwards, when the run's event is asked for errors too (not
+    // the stream: it is the caller's, who may have destroyed it by now).
     auto t0 = std::chrono::steady_clock::now();
     auto waited = [&]() { return std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count(); };
-    while (__atomic_load_n(&g->report->seq, __ATOMIC_ACQUIRE) != g->seq) {
+    while (!reported(g)) {
         const double w = waited();
         if (timeout_s > 0 && w > timeout_s)
             return set_error(TTAD_ERR_TIMEOUT, "graph_wait: timed out after %.1f s (graph still running)", timeout_s);
         if (w < 5e-3) continue;
-        const hipError_t e = hipStreamQuery(g->stream);
+        const hipError_t e = hipEventQuery(g->ev_stop);
         if (e != hipSuccess && e != hipErrorNotReady) {
             g->running = false;
             return set_error(TTAD_ERR_DEVICE, "graph_wait: %s", hipGetErrorString(e));
@@ -1098,7 +1102,11 @@ int ttad_graph_write_deps(ttad_graph* g, const char* path) {
 
 int ttad_graph_destroy(ttad_graph* g) {
     if (!g) return TTAD_OK;
-    if (g->running) (void)hipStreamSynchronize(g->stream);  // (its report kernel too)
+    // (the run, and the kernel behind it that writes the report)
+    if (g->running && hipEventSynchronize(g->ev_stop) == hipSuccess) {
+        const auto t0 = std::chrono::steady_clock::now();
+        while (!reported(g) && std::chrono::steady_clock::now() - t0 < std::chrono::seconds(5)) std::this_thread::yield();
+    }
     if (g->report_slot >= 0) g->ctx->free_reports.push_back(g->report_slot);
     if (g->ev_start) (void)hipEventDestroy(g->ev_start);
     if (g->ev_stop) (void)hipEventDestroy(g->ev_stop);
