@@ -100,10 +100,12 @@ __global__ __launch_bounds__(NTHREADS, vset_occupancy(VM)) void k_persistent(Dev
                 int cand[CLAIM_TRIES];  // queues to try, best first
                 int nc = 0;
                 int reserve_all = 0, reserve_own = 0;
-                // A secondary does not even scan while a quarter of its XCD's primaries look for work. (From the
-                // first idle primary on, bf16x3 factorization n = 32768: 66.8 ms, since an idle primary may be held back
-                // by a critical item of its CU; from 8 on 57.1, from 16 on 57.2; n = 16384: 10.1, 10.9, 11.2 ms.)
-                if (primary || ld_relaxed(idle_primary) < IDLE_PRIMARIES) {
+                // From its third look on, a secondary does not even scan while a quarter of its XCD's primaries look for
+                // work. (From the first idle primary on, bf16x3 factorization n = 32768: 66.8 ms, since an idle primary may be
+                // held back by a critical item of its CU; from 8 on 57.1, from 16 on 57.2; n = 16384: 10.1, 10.9, 11.2 ms.
+                // Primaries between two short tasks count as idle too: 2e5 independent empty tasks 16.2 ms held back from the
+                // first look on, 11.4 so, 15.9 from the second; factorizations alike.)
+                if (primary || idle_scans < 2 || ld_relaxed(idle_primary) < IDLE_PRIMARIES) {
                     // a secondary leaves queues that the idle primaries can drain; nothing is taken while
                     // the other worker of this CU runs an item of the critical path
                     // the lane index, opaque to the compiler here: addresses derived from it are formed per scan
