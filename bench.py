@@ -381,11 +381,18 @@ def trailing_update_leg(ctx, mn: int, k: int, reps: int = 10):
             "rocblas_tflops": round(fl / t_blas / 1e12, 3)}
 
 
+def potrf_items(b: int) -> int:
+    """Work items of POTRF of a b x b tile: one per 64 x 64 block below the block diagonal (the last of a block row with the
+    diagonal block beside it), and the first diagonal block."""
+    nb = (b + 63) // 64
+    return 1 + nb * (nb - 1) // 2
+
+
 def panel_leg(ctx, m: int, b: int, reps: int = 10):
     """The panel steps alone, FP64, as the factorization runs them.
 
-    POTRF: one b x b tile factored by the block items the factorization uses (one workgroup per 64 x 64 block of the
-    lower half, waiting on each other's progress flags), launched alone through the host-sequenced schedule of a one-tile matrix and
+    POTRF: one b x b tile factored by the block items the factorization uses (potrf_items workgroups, waiting on each
+    other's progress flags), launched alone through the host-sequenced schedule of a one-tile matrix and
     timed with events around that launch. TRSM: ttad_dtrsm on the m x b column of tiles below (the first
     panel's TRSM tasks at m = n - b). GB/s use the per-task algorithmic bytes: POTRF reads and writes its tile
     (2 b^2 8 bytes), a TRSM task reads L_jj and reads and writes its tile (3 b^2 8 bytes)."""
@@ -427,7 +434,7 @@ def panel_leg(ctx, m: int, b: int, reps: int = 10):
     trsm_gbps = 3.0 * b * b * 8 * n_trsm / t_trsm / 1e9
     del A, Ls, P, Bm
     torch.cuda.empty_cache()
-    return {"potrf_tile": b, "potrf_items": (b // 64) * (b // 64 + 1) // 2, "potrf_ms": round(tp * 1e3, 4),
+    return {"potrf_tile": b, "potrf_items": potrf_items(b), "potrf_ms": round(tp * 1e3, 4),
             "potrf_tflops": round(flops(b) / tp / 1e12, 4), "potrf_gbps": round(potrf_gbps, 2),
             "potrf_hbm_frac": round(potrf_gbps / 8000.0, 5),
             "trsm_shape": f"m={m} n={b} ({n_trsm:g} tile tasks)", "trsm_ms": round(t_trsm * 1e3, 4),

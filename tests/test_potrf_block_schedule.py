@@ -204,3 +204,9 @@ def test_bad_pivot_is_reported_before_the_block_is_published():
     assert src.index("atomicCAS(info") < src.index("publish(r, r);")
     assert all(_first_bad_pivot(seed, True) == 1 for seed in range(100))
     assert any(_first_bad_pivot(seed, False) != 1 for seed in range(100))
+
+
+@pytest.mark.parametrize("n", SIZES + [4096])
+def test_benchmark_reports_the_item_count(tables, n):
+    import bench
+    assert bench.potrf_items(n) == tables[n][0]
