@@ -198,14 +198,15 @@ __device__ __attribute__((noinline)) void gemm_call(const GemmOperands* go, int 
                                        wave_uniform(c0), wave_uniform((int)syrk) != 0, -1.0, 1.0, lds_uniform(lds),
                                        wave_uniform(o->PA), wave_uniform(o->PB), o + 1, wave_uniform(span) - 1);
 }
-template <typename TS, int VM>
+// LDS_FORM: the item may be one that keeps X in LDS (in_lds).
+template <typename TS, int VM, bool LDS_FORM>
 __device__ __attribute__((noinline)) void trsm_call(const TS* L, const double* dinv, TS* X, int m, int n, int it,
                                                     bool in_lds, char* lds, void* planes) {
     __builtin_amdgcn_s_setprio(3);
     const int mu = wave_uniform(m), nu = wave_uniform(n), iu = wave_uniform(it);
     char* l = lds_uniform(lds);
     bool done = false;
-    if constexpr ((VM & V_TLDS) != 0)
+    if constexpr (LDS_FORM)
         if (wave_uniform((int)in_lds)) {
             item_trsm_lds<TS>(wave_uniform(L), nu, wave_uniform(dinv), wave_uniform(X), mu, mu, nu,
                               iu * trsm_rows(sizeof(TS), true), l, wave_uniform(planes));
@@ -222,6 +223,8 @@ __device__ __attribute__((noinline)) void trsm_call(const TS* L, const double* d
 // each other (item_potrf): the caller must
 // have every lower-numbered item of the task running or done; their waits give up
 // after spin_limit ticks or once *err is nonzero (and set *err = 1 when they time out).
+// GOPS: the persistent executor's items, whose GEMM operands are resolved (go) and whose form t.sub chooses. Without, items
+// are 128x128 and TRSM strips the higher ones (the host-sequenced schedule and the serving loop never ask for others).
 template <int VM, bool GOPS = false>
 __device__ __forceinline__ bool exec_item(const DevTask& t, int it, const DevMat* mats, char* lds, int32_t* err,
                                           int64_t spin_limit, const GemmOperands* go = nullptr) {
@@ -259,16 +262,17 @@ __device__ __forceinline__ bool exec_item(const DevTask& t, int it, const DevMat
         case K_TRSM: {
             const int i = t.i, j = t.j, m = M.bsz[i], n = M.bsz[j];
             const bool in_lds = t.sub == GEMM_BS;
-            if ((VM & V_TLDS) == 0 && in_lds) return false;
+            constexpr bool lds_form = GOPS && (VM & V_TLDS) != 0;
+            if (!lds_form && in_lds) return false;
             if constexpr ((VM & V_F64S) != 0)
                 if (f64s) {
-                    trsm_call<double, VM>((const double*)tile(j, j), M.dinv[j], (double*)tile(i, j), m, n, it, in_lds, lds,
+                    trsm_call<double, VM, lds_form>((const double*)tile(j, j), M.dinv[j], (double*)tile(i, j), m, n, it, in_lds, lds,
                                         nullptr);
                     return true;
                 }
             if constexpr ((VM & V_F32S) != 0)
                 if (!f64s) {
-                    trsm_call<float, VM>((const float*)tile(j, j), M.dinv[j], (float*)tile(i, j), m, n, it, in_lds, lds,
+                    trsm_call<float, VM, lds_form>((const float*)tile(j, j), M.dinv[j], (float*)tile(i, j), m, n, it, in_lds, lds,
                                         planes(i, j));
                     return true;
                 }
@@ -305,7 +309,7 @@ __device__ __forceinline__ bool exec_item(const DevTask& t, int it, const DevMat
                 K = M.bsz[k];
             }
             int rb, cb;
-            const int sub = wave_uniform(t.sub);
+            const int sub = GOPS ? wave_uniform(t.sub) : GEMM_BM;
             decode_gemm_item(it, (m + sub - 1) / sub, syrk, rb, cb);
             const int r0 = rb * sub, c0 = cb * sub;
             // accumulate mode: one lock word per 128x128 sub-tile (16 per tile, shared beyond 4x4 sub-tiles)
@@ -323,21 +327,19 @@ __device__ __forceinline__ bool exec_item(const DevTask& t, int it, const DevMat
             return true;                                                                                           \
         }                                                                                                          \
     }                                                                                                              \
-    if (GOPS && sub == GEMM_BM) {                                                                                  \
+    if constexpr (GOPS) {                                                                                          \
         constexpr bool fold = sizeof(TS_) == 4 && PREC_ != P_BF16X3;                                               \
-        if (fold && span > 1)                                                                                      \
+        if (sub == GEMM_BS)                                                                                        \
+            gemm_small_call<TS_, PREC_, VM>((const TS_*)opA, (const TS_*)opB, (TS_*)opC, m, n, K, r0, c0, syrk,    \
+                                            lds, opPA, opPB);                                                      \
+        else if (fold && span > 1)                                                                                 \
             gemm_call<TS_, PREC_, VM, fold>(go, span, r0, c0, syrk, lds);                                          \
         else                                                                                                       \
             gemm_call<TS_, PREC_, VM, false>(go, span, r0, c0, syrk, lds);                                         \
-        return true;                                                                                               \
+    } else {                                                                                                       \
+        item_gemm<TS_, PREC_>((const TS_*)opA, m, (const TS_*)opB, n, (TS_*)opC, m, m, n, K, r0, c0, syrk, -1.0,   \
+                              1.0, lds, opPA, opPB);                                                               \
     }                                                                                                              \
-    if (GOPS || sub == GEMM_BS) {                                                                                  \
-        gemm_small_call<TS_, PREC_, VM>((const TS_*)opA, (const TS_*)opB, (TS_*)opC, m, n, K, r0, c0, syrk, lds,   \
-                                        opPA, opPB);                                                               \
-        return true;                                                                                               \
-    }                                                                                                              \
-    item_gemm<TS_, PREC_>((const TS_*)opA, m, (const TS_*)opB, n, (TS_*)opC, m, m, n, K, r0, c0, syrk, -1.0, 1.0,  \
-                          lds, opPA, opPB);                                                                        \
     return true;
             // Products read C after the last K-chunk: measured faster than reading it with the first chunk
             // for FP64 (factorization at n = 32768: 246.7 -> 229.4 ms) and for bf16x3 items (11 %).
