@@ -587,6 +587,7 @@ int ttad_last_elapsed(ttad_context* ctx, double* seconds) {
 // (POTRF 8, TRSM 3, GEMM/SYRK 1: one workgroup factors a whole tile, a TRSM item solves 64 rows
 // block column by block column). Those items run with no other item started on their CU.
 // TTAD_CRITICAL=0 turns it off (for comparisons).
+// Also the level of each task, the tasks before it on the longest way from a source: tasks of one level can run at once.
 static void mark_critical(ttad_graph& g) {
     static const bool on = [] {
         const char* v = getenv("TTAD_CRITICAL");
@@ -594,7 +595,8 @@ static void mark_critical(ttad_graph& g) {
     }();
     const int n = g.n_tasks;
     for (auto& t : g.tasks) t.crit = 0;
-    if (!on || n == 0) return;
+    g.level.assign(n, 0);
+    if (n == 0) return;
     std::vector<int> w(n), indeg(n, 0), order;
     order.reserve(n);
     for (int t = 0; t < n; t++) {
@@ -610,6 +612,10 @@ static void mark_critical(ttad_graph& g) {
             if (--indeg[g.out_idx[e]] == 0) order.push_back(g.out_idx[e]);
     }
     if ((int)order.size() != n) return;  // not a DAG: no marking (the graph would not complete anyway)
+    for (int t : order)
+        for (int e = g.out_ptr[t]; e < g.out_ptr[t + 1]; e++)
+            g.level[g.out_idx[e]] = std::max(g.level[g.out_idx[e]], g.level[t] + 1);
+    if (!on) return;
     std::vector<long long> top(n, 0), bot(n, 0);
     for (int t : order) {
         top[t] += w[t];
@@ -759,34 +765,48 @@ static int graph_prepare(ttad_graph* g) {
     if (g->mats_dirty) {
         int rate_khz = 100000;
         (void)hipDeviceGetAttribute(&rate_khz, hipDeviceAttributeWallClockRate, g->ctx->device);
-        // 128x128 items that the updates of step k of a matrix would have: a step that cannot give every other CU one has
-        // 64x64 items, and so has every update on a longest path (its latency counts, not its throughput). Up to half
-        // an item per CU / one / two, FP64 n = 4096 b = 256: 2.20 / 2.25 / 2.34 ms (none 2.75, no longest path 2.35). Accumulate-
-        // mode updates keep 128 (their locks are per 128x128 sub-tile).
-        std::map<std::pair<int, int>, long long> step_items;
-        auto update_items = [&](const DevTask& x, int sub) {
+        // 128x128 items that the updates of a level would have (in a factorization: those of one step): a level that cannot
+        // give every other CU one has 64x64 items, and so has every update on a longest path (its latency counts, not its
+        // throughput) unless that path's own items give every CU one (graphs of many equal branches, all of them longest
+        // paths). Up to half an item per CU / one / two, FP64 n = 4096 b = 256: 2.20 / 2.25 / 2.34 ms (none 2.75, no longest
+        // path 2.35). Accumulate-mode updates keep 128 (their locks are per 128x128 sub-tile).
+        const int levels = n > 0 ? *std::max_element(g->level.begin(), g->level.end()) + 2 : 2;
+        std::vector<long long> level_items(levels, 0), crit_items(levels, 0), crit_strips(levels, 0);
+        auto tile_items = [&](const DevTask& x, int sub) {
             ttad_matrix* M = x.mat < (int)g->mats.size() ? g->mats[x.mat] : nullptr;
             const bool in = M && x.i >= 0 && x.j >= 0 && x.i < M->nt && x.j < M->nt;
             return in ? items_of(x.kind, M->bsz[x.i], M->bsz[x.j], (int)M->elem, sub) : 0;
         };
-        for (auto& x : g->tasks)
-            if (x.kind == K_GEMM || x.kind == K_SYRK)
-                for (int q = 0; q < x.kspan; q++) step_items[{x.mat, x.k + q}] += update_items(x, GEMM_BM);
+        long long update_total = 0;
+        for (int t = 0; t < n; t++) {
+            const DevTask& x = g->tasks[t];
+            if (x.kind == K_GEMM || x.kind == K_SYRK) {
+                const int items = tile_items(x, GEMM_BM);
+                // (fused steps k, k + 1, ..: POTRF, TRSM and the update of each follow those of the last)
+                for (int q = 0; q < x.kspan; q++) level_items[std::min(g->level[t] + 3 * q, levels - 1)] += items;
+                update_total += (long long)items * x.kspan;
+                if (x.crit) crit_items[g->level[t]] += items;
+            } else if (x.kind == K_TRSM && x.crit) {
+                crit_strips[g->level[t]] += tile_items(x, GEMM_BS);
+            }
+        }
         // FP64: with more than 128 update items per CU in all the updates' throughput bounds the run and TRSM keeps its
         // higher strips (n = 12288, b = 512, 145 per CU: 12.6 ms, 12.5 with the LDS form on the longest path and
         // in the small steps; n = 16384, 26.1 either way); below, the chain does (n = 8192, 49 per CU: 5.4 and 5.2 ms).
-        long long update_total = 0;
-        for (auto& kv : step_items) update_total += kv.second;
+        // A longest path's strips take the LDS form while they all run at once (trsm_in_lds), a step's by its updates.
         const bool throughput = update_total > 128LL * g->ctx->n_cu;
-        for (auto& x : g->tasks) {
+        for (int t = 0; t < n; t++) {
+            DevTask& x = g->tasks[t];
+            const int lv = g->level[t];
             x.sub = GEMM_BM;
             if ((x.kind == K_GEMM || x.kind == K_SYRK) && !x.accum && x.kspan == 1 &&
-                (x.crit || 2 * step_items[{x.mat, x.k}] <= g->ctx->n_cu))
+                ((x.crit && crit_items[lv] <= g->ctx->n_cu) || 2 * level_items[lv] <= g->ctx->n_cu))
                 x.sub = GEMM_BS;
             if (x.kind == K_TRSM && x.mat < (int)g->mats.size() && g->mats[x.mat] && x.j >= 0 && x.j < g->mats[x.mat]->nt &&
                 g->mats[x.mat]->bsz[x.j] <= TRSM_LDS_COLS &&
                 (g->mats[x.mat]->storage != P_F64 ||
-                 (!throughput && (x.crit || 2 * step_items[{x.mat, x.j}] <= g->ctx->n_cu))))
+                 (!throughput && ((x.crit && crit_strips[lv] <= 2 * g->ctx->n_cu) ||
+                                  (!x.crit && 2 * level_items[lv + 1] <= g->ctx->n_cu)))))
                 x.sub = GEMM_BS;
         }
         for (int t = 0; t < n; t++) {

@@ -189,13 +189,14 @@ static void fuse_updates(ttad_graph* g, const ttad_matrix* M, int cols) {
     for (int t = 0; t < n; t++)
         if (rep[t] == t) id[t] = m++;
     std::vector<std::vector<int>> out(m);
-    std::vector<int32_t> indeg(m, 0), seeds(m, 0), spin(m, 0);
+    std::vector<int32_t> indeg(m, 0), seeds(m, 0), spin(m, 0), level(m, 0);
     std::vector<DevTask> tasks(m);
     for (int t = 0; t < n; t++) {
         const int a = id[rep[t]];
         if (rep[t] == t) {
             tasks[a] = g->tasks[t];
             spin[a] = g->spin_us[t];
+            level[a] = g->level[t];
         }
         seeds[a] += g->seeds[t];
         indeg[a] += g->indegree[t];
@@ -210,6 +211,7 @@ static void fuse_updates(ttad_graph* g, const ttad_matrix* M, int cols) {
     g->indegree = std::move(indeg);
     g->seeds = std::move(seeds);
     g->spin_us = std::move(spin);
+    g->level = std::move(level);
     g->out_ptr.assign(1, 0);
     g->out_idx.clear();
     for (auto& o : out) {

@@ -142,6 +142,7 @@ struct ttad_graph {
     int n_tasks = 0, n_buckets = 0, total_items = 0;  // n_buckets counts work queues
     std::vector<ttad::DevTask> tasks;
     std::vector<int32_t> indegree, seeds, out_ptr, out_idx, q_base, bucket_items;
+    std::vector<int32_t> level;   // per task: the tasks before it on the longest way from a source
     std::vector<int32_t> q_home;  // per queue: -1 shared, else the XCD whose workers it feeds first
     std::vector<ttad_matrix*> mats;
     bool with_planes = false;  // hand the matrices' bf16 planes to the items (a full Cholesky PTG only)
