@@ -849,8 +849,10 @@ static int graph_prepare(ttad_graph* g) {
         g->q_base.assign(g->n_buckets + 1, 0);
         for (int b = 0; b < g->n_buckets; b++) g->q_base[b + 1] = g->q_base[b] + g->bucket_items[b];
         std::vector<DevMat> dm(g->mats.size());
+        std::vector<int32_t> bound;
         for (size_t s = 0; s < g->mats.size(); s++)
             if (g->mats[s]) {
+                bound.push_back((int32_t)s);
                 dm[s] = g->mats[s]->host_desc;
                 if (g->with_planes && g->mats[s]->tab_planes.p) dm[s].planes = g->mats[s]->tab_planes.as<void*>();
             }
@@ -883,11 +885,14 @@ static int graph_prepare(ttad_graph* g) {
         TTAD_HIP(g->d_trace_cursor.alloc(4));
         TTAD_HIP(g->d_cu_slots.alloc((2 * CU_KEYS + NXCD * 64) * 4));  // slots, critical counts, idle primaries
         TTAD_HIP(g->d_mats.alloc(dm.size() * sizeof(DevMat)));
+        TTAD_HIP(g->d_bound.alloc(bound.size() * 4));
+        g->n_bound = (int)bound.size();
         TTAD_HIP(hipMemcpy(g->d_tasks.p, g->tasks.data(), n * sizeof(DevTask), hipMemcpyHostToDevice));
         TTAD_HIP(hipMemcpy(g->d_edges.p, edges.data(), ne * sizeof(DevEdge), hipMemcpyHostToDevice));
         TTAD_HIP(hipMemcpy(g->d_q_base.p, g->q_base.data(), (g->n_buckets + 1) * 4, hipMemcpyHostToDevice));
         TTAD_HIP(hipMemcpy(g->d_q_home.p, g->q_home.data(), g->n_buckets * 4, hipMemcpyHostToDevice));
         TTAD_HIP(hipMemcpy(g->d_mats.p, dm.data(), dm.size() * sizeof(DevMat), hipMemcpyHostToDevice));
+        TTAD_HIP(hipMemcpy(g->d_bound.p, bound.data(), bound.size() * 4, hipMemcpyHostToDevice));
         g->mats_dirty = false;
         g->seeds_dirty = true;
     }
@@ -926,7 +931,8 @@ static DevGraph graph_image(ttad_graph* g, bool trace, int64_t spin_limit) {
     d.n_tasks = g->n_tasks;
     d.n_buckets = g->n_buckets;
     d.total_items = g->total_items;
-    d.n_mats = (int)g->mats.size();
+    d.n_bound = g->n_bound;
+    d.bound = g->d_bound.as<int32_t>();
     d.has_accum = g->has_accum;
     d.tasks = g->d_tasks.as<DevTask>();
     d.edges = g->d_edges.as<DevEdge>();

@@ -17,7 +17,8 @@ struct DevGraph {
     const int32_t* deps0;       // initial dependency counters (indegree - host seeds)
     const int32_t* tail0;       // initial queue tails per bucket
     const int64_t* q_items0;    // [total_items] initial queue entries: those of ready tasks, else -1
-    int32_t n_mats;
+    int32_t n_bound;
+    const int32_t* bound;       // [n_bound] the slots of mats that a matrix is bound to
     int32_t has_accum;          // some update runs in accumulate mode (the tile locks are cleared before a run)
     int32_t* deps;
     int32_t* items_left;

@@ -364,9 +364,8 @@ __global__ void k_graph_reset(DevGraph g, int n_slots) {
         g.cu_crit[x] = 0;
     }
     for (int x = blockIdx.x * blockDim.x + threadIdx.x; x < NXCD * 64; x += stride) g.idle_primary[x] = 0;
-    for (int q = 0; q < g.n_mats; q++) {
-        const DevMat& M = g.mats[q];
-        if (!M.info) continue;  // slot not bound
+    for (int q = 0; q < g.n_bound; q++) {
+        const DevMat& M = g.mats[g.bound[q]];
         for (int x = blockIdx.x * blockDim.x + threadIdx.x; x < M.nt * M.pf_stride; x += stride) M.pflags[x] = 0;
         if (g.has_accum)
             for (long x = blockIdx.x * blockDim.x + threadIdx.x; x < (long)M.nt * M.nt * 16; x += stride) M.locks[x] = 0;
@@ -381,8 +380,7 @@ __global__ void k_graph_reset(DevGraph g, int n_slots) {
 __global__ void k_graph_report(DevGraph g, GraphReport* out, int seq) {
     if (threadIdx.x != 0) return;
     int info = 0;
-    for (int q = 0; q < g.n_mats && info == 0; q++)
-        if (g.mats[q].info) info = *g.mats[q].info;
+    for (int q = 0; q < g.n_bound && info == 0; q++) info = *g.mats[g.bound[q]].info;
     out->done = *g.done_items;
     out->abort_code = *g.abort_flag;
     out->info = info;

@@ -149,8 +149,9 @@ struct ttad_graph {
     std::vector<int32_t> spin_us;  // per task: spin time of a TTAD_SPIN task (microseconds)
     bool seeds_dirty = true, mats_dirty = true, running = false;
     int gop_stride = 1;  // the largest kspan of the tasks
+    int n_bound = 0;     // slots that a matrix is bound to
     ttad::DevBuf d_tasks, d_edges, d_deps0, d_tail0, d_q_items0, d_deps, d_items_left, d_gops, d_q_head, d_q_tail, d_q_count, d_xcd_run,
-        d_q_base, d_q_home, d_q_items, d_done, d_abort, d_mats, d_trace, d_trace_cursor, d_cu_slots;
+        d_q_base, d_q_home, d_q_items, d_done, d_abort, d_mats, d_bound, d_trace, d_trace_cursor, d_cu_slots;
     bool has_accum = false;
     // this graph's report slot (-1: its own pinned buffer), and the number of runs launched
     int report_slot = -1;
