@@ -583,9 +583,9 @@ int ttad_last_elapsed(ttad_context* ctx, double* seconds) {
 // ---------------------------------------------------------------------------
 // Device task graphs
 // ---------------------------------------------------------------------------
-// Marks the tasks on a longest path of the DAG, weighting each kind by the latency of its items
-// (POTRF 8, TRSM 3, GEMM/SYRK 1: one workgroup factors a whole tile, a TRSM item solves 64 rows
-// block column by block column). Those items run with no other item started on their CU.
+// Marks the tasks on a longest path of the DAG, weighting each kind by its latency
+// (POTRF 8, TRSM 3, GEMM/SYRK 1: a tile's pivots and a strip's block columns are chains). Their
+// items run with no other item started on their CU.
 // TTAD_CRITICAL=0 turns it off (for comparisons).
 // Also the level of each task, the tasks before it on the longest way from a source: tasks of one level can run at once.
 static void mark_critical(ttad_graph& g) {
@@ -791,8 +791,9 @@ static int graph_prepare(ttad_graph* g) {
             }
         }
         // FP64: with more than 128 update items per CU in all the updates' throughput bounds the run and TRSM keeps its
-        // higher strips (n = 12288, b = 512, 145 per CU: 12.6 ms, 12.5 with the LDS form on the longest path and
-        // in the small steps; n = 16384, 26.1 either way); below, the chain does (n = 8192, 49 per CU: 5.4 and 5.2 ms).
+        // higher strips (b = 512, ms so / with the LDS form on the longest path and in the small steps: n = 12288, 145 per CU,
+        // 12.3 / 12.2; n = 16384 25.7 / 25.8; 24576 80.0 / 80.8; 32768 185.0 / 187.0); below, the chain does (n = 8192, 49 per
+        // CU: 5.4 and 5.2 ms).
         // A longest path's strips take the LDS form while they all run at once (trsm_in_lds), a step's by its updates.
         const bool throughput = update_total > 128LL * g->ctx->n_cu;
         for (int t = 0; t < n; t++) {

@@ -111,8 +111,8 @@ enum ItemVariant : int {
     V_ACC = 32       // accumulate-mode GEMM/SYRK (only in the last set, so the others keep their registers)
 };
 // The compiled sets, smallest first.
-// (FP64 tiles have two: the TRSM form in LDS, present though unused in a kernel with inline GEMM items, made the large
-// FP64 factorizations 5 % slower; with the items out of line they are alike, n = 16384: 26.1 ms.)
+// (FP64 tiles have two: large factorizations bound by the updates run the one without the TRSM form in LDS. n = 16384 alike,
+// 25.7 ms; n = 24576 80.0 ms, 80.5 with the other set, 80.9 with its TRSM form too; n = 32768 185.0, 186.0 and 187.0.)
 constexpr int V_ALL = V_F64S | V_F32S | V_G32 | V_GBF16 | V_GBF16X3 | V_TLDS;
 constexpr int N_VSETS = 7;
 constexpr int VSETS[N_VSETS] = {V_F64S, V_F64S | V_TLDS, V_F32S | V_G32 | V_TLDS, V_F32S | V_GBF16 | V_TLDS,

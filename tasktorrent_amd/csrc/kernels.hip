@@ -45,8 +45,8 @@ __global__ __launch_bounds__(NTHREADS, vset_occupancy(VM)) void k_items(const De
 //   successors' dependency counters and pushes every item of a successor that
 //   reaches zero into its queue. A worker exits when every item is done, or claimed by others.
 // Memory ordering: item outputs are released (agent scope) before the counter
-// RMWs; queue entries are published with release stores and read with acquire
-// loads, so a consumer on another XCD sees the producer's tiles.
+// RMWs; queue entries are written and polled relaxed, behind that release and in front of
+// an acquire fence, so a consumer on another XCD sees the producer's tiles.
 // The loop also ends when the abort flag is raised (watchdog: no work found for
 // spin_limit ticks; queue overflow; an item variant missing from this instantiation).
 // ---------------------------------------------------------------------------
